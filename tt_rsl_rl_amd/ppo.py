@@ -310,10 +310,13 @@ class PPO:
             if self._perm_host is None or self._perm_host.numel() != B:
                 self._perm_host = torch.empty(B, dtype=torch.int64, pin_memory=True)
                 self._perm_dev = torch.empty(B, dtype=torch.int64, device=self.device)
+                if self._copy_stream is None:
+                    self._copy_stream = torch.cuda.Stream(self.device)  # (default priority)
+                    self._rest_copied = torch.cuda.Event()
+                # the buffer is this stream's memory: work still queued here may belong to its previous use, so the
+                # copies into it from the other stream start after that
+                self._copy_stream.wait_stream(torch.cuda.current_stream(self.device))
             perm = self._perm_dev
-            if self._copy_stream is None:
-                self._copy_stream = torch.cuda.Stream(self.device)  # (default priority)
-                self._rest_copied = torch.cuda.Event()
             copy_stream, rest_copied, host = self._copy_stream, self._rest_copied, self._perm_host
 
             def copy_rest(sp):  # on the worker, once perm[sp.split:] is final: its copy, beside the update's kernels

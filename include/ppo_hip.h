@@ -247,6 +247,44 @@ int ppo_linear_bwd_dw_ex(const ppo_linear_bwd_dw_problem* problems, int32_t coun
                          void* workspace, size_t workspace_bytes, const float* extra_grads,
                          const ppo_grad_range* extra, int32_t num_extra, double* norm_partials, ppo_stream_t stream);
 
+/* Largest magnitudes.  PPO_AMAX_WORDS words per tensor: PPO_AMAX_SLOTS slots, one per 128-byte line (its first word; the
+ * others are unused), the maximum over the slots being the fp32 bits of max |x| over the tensor's finite values (an
+ * upper bound serves as well).  ppo_amax writes the slots of each item (x: [rows, cols], row
+ * stride ld) and clears `clear_words` words at `clear`, the slots that kernels after it on the stream add to; both in
+ * one launch.  No counterpart in the reference. */
+#define PPO_AMAX_SLOTS 64
+#define PPO_AMAX_WORDS (PPO_AMAX_SLOTS * 32)
+#define PPO_MAX_AMAX_ITEMS 16
+typedef struct ppo_amax_item {
+  const float* x; int64_t ld;
+  int64_t rows;
+  int32_t cols;
+  float least;    /* the slots' maximum is at least this (>= 0) */
+  uint32_t* slots;
+} ppo_amax_item;
+int ppo_amax(const ppo_amax_item* items, int32_t count, uint32_t* clear, int64_t clear_words, ppo_stream_t stream);
+
+/* The three GEMMs with the operands' largest magnitudes known (ranges: one per problem, in the problems' order; a / b:
+ * the slots of the first and the second operand -- x and w, dz and w, dz and x -- and out: NULL, or slots that the
+ * forward and the input-grad raise by the largest |output| they write, h where there is an activation).  Launches whose
+ * ranges are all given and whose operands have 16-byte rows run on the fp16 matrix cores with each operand element
+ * scaled and split into two fp16 parts (fp32 accuracy, csrc/gemm_f16.hpp); any other launch is the plain entry point's,
+ * followed by a pass over its outputs where `out` is given.  flags as above. */
+typedef struct ppo_gemm_range {
+  const uint32_t* a;
+  const uint32_t* b;
+  uint32_t* out;
+} ppo_gemm_range;
+int ppo_linear_fwd_ranged(const ppo_linear_fwd_problem* problems, const ppo_gemm_range* ranges, int32_t count,
+                          int64_t rows, int32_t activation, int32_t flags, ppo_stream_t stream);
+int ppo_linear_bwd_dx_ranged(const ppo_linear_bwd_dx_problem* problems, const ppo_gemm_range* ranges, int32_t count,
+                             int64_t rows, int32_t activation, int32_t source, int32_t flags, void* workspace,
+                             size_t workspace_bytes, ppo_stream_t stream);
+int ppo_linear_bwd_dw_ranged(const ppo_linear_bwd_dw_problem* problems, const ppo_gemm_range* ranges, int32_t count,
+                             int64_t rows, int32_t flags, void* workspace, size_t workspace_bytes,
+                             const float* extra_grads, const ppo_grad_range* extra, int32_t num_extra,
+                             double* norm_partials, ppo_stream_t stream);
+
 /* ------------------------------------------------------------------------------------------------------------------
  * A7  Empirical observation normaliser, rsl_rl/modules/normalization.py:46-78.
  * ppo_obs_normalize: y = (x - mean) / (std + eps) over [rows, width] (forward, :46-48).
@@ -378,6 +416,19 @@ size_t ppo_head_workspace_bytes(int64_t rows, int32_t num_actions);
 int ppo_gauss_ppo_head(const ppo_loss_args* args, const ppo_policy_head* head, void* workspace,
                        size_t workspace_bytes, float* d_std_param, ppo_device_state* state, int32_t adaptive,
                        double desired_kl, double* trace, int32_t trace_rows, ppo_stream_t stream);
+
+/* The same, also raising the slots (PPO_AMAX_WORDS each, NULL: not wanted) of what it writes by their largest
+ * magnitudes: dz_actor, dz_critic and the loss arguments' d_mean and d_value. */
+typedef struct ppo_head_ranges {
+  uint32_t* dz_actor;
+  uint32_t* dz_critic;
+  uint32_t* d_mean;
+  uint32_t* d_value;
+} ppo_head_ranges;
+int ppo_gauss_ppo_head_ranged(const ppo_loss_args* args, const ppo_policy_head* head, const ppo_head_ranges* ranges,
+                              void* workspace, size_t workspace_bytes, float* d_std_param, ppo_device_state* state,
+                              int32_t adaptive, double desired_kl, double* trace, int32_t trace_rows,
+                              ppo_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------------------------------
  * Rollout-side Gaussian head for act() (rsl_rl/algorithms/ppo.py:124-135; rsl_rl/modules/distribution.py:183-232):

@@ -55,6 +55,19 @@ class GatherSegment(C.Structure):
                 ("norm_mean", C.c_void_p), ("norm_std", C.c_void_p), ("norm_eps", C.c_float), ("kind", i32)]
 
 
+AMAX_WORDS = 64 * 32  # 64 slots, one per 128-byte line
+MAX_AMAX_ITEMS = 16
+
+
+class AmaxItem(C.Structure):
+    _fields_ = [("x", C.c_void_p), ("ld", i64), ("rows", i64), ("cols", i32), ("least", C.c_float),
+                ("slots", C.c_void_p)]
+
+
+class GemmRange(C.Structure):
+    _fields_ = [("a", C.c_void_p), ("b", C.c_void_p), ("out", C.c_void_p)]
+
+
 class LinearFwdProblem(C.Structure):
     _fields_ = [("x", C.c_void_p), ("ldx", i64), ("w", C.c_void_p), ("b", C.c_void_p), ("z", C.c_void_p),
                 ("ldz", i64), ("h", C.c_void_p), ("ldh", i64), ("in_features", i32), ("out_features", i32)]
@@ -114,6 +127,10 @@ class PolicyHead(C.Structure):
                 ("dz_actor", C.c_void_p), ("ld_dz_actor", i64), ("dz_critic", C.c_void_p), ("ld_dz_critic", i64),
                 ("mean", C.c_void_p), ("ld_mean", i64), ("value", C.c_void_p), ("ld_value", i64),
                 ("k_actor", i32), ("k_critic", i32)]
+
+
+class HeadRanges(C.Structure):
+    _fields_ = [("dz_actor", C.c_void_p), ("dz_critic", C.c_void_p), ("d_mean", C.c_void_p), ("d_value", C.c_void_p)]
 
 
 class DeviceState(C.Structure):
@@ -187,6 +204,14 @@ _SIGNATURES = [
                                        C.c_size_t, C.c_void_p]),
     ("ppo_linear_bwd_dw_ex", C.c_int, [C.POINTER(LinearBwdDwProblem), i32, i64, i32, C.c_void_p, C.c_size_t, f32p,
                                        C.POINTER(GradRange), i32, C.c_void_p, C.c_void_p]),
+    ("ppo_amax", C.c_int, [C.POINTER(AmaxItem), i32, C.c_void_p, i64, C.c_void_p]),
+    ("ppo_linear_fwd_ranged", C.c_int, [C.POINTER(LinearFwdProblem), C.POINTER(GemmRange), i32, i64, i32, i32,
+                                        C.c_void_p]),
+    ("ppo_linear_bwd_dx_ranged", C.c_int, [C.POINTER(LinearBwdDxProblem), C.POINTER(GemmRange), i32, i64, i32, i32,
+                                           i32, C.c_void_p, C.c_size_t, C.c_void_p]),
+    ("ppo_linear_bwd_dw_ranged", C.c_int, [C.POINTER(LinearBwdDwProblem), C.POINTER(GemmRange), i32, i64, i32,
+                                           C.c_void_p, C.c_size_t, f32p, C.POINTER(GradRange), i32, C.c_void_p,
+                                           C.c_void_p]),
     ("ppo_obs_normalize", C.c_int, [f32p, i64, f32p, i64, i64, i32, f32p, f32p, C.c_float, C.c_void_p]),
     ("ppo_normalizer_update_workspace_bytes", C.c_size_t, [i64, i32]),
     ("ppo_normalizer_update", C.c_int, [C.POINTER(ColumnBlock), i32, i64, f32p, f32p, f32p, C.c_void_p, C.c_void_p,
@@ -199,6 +224,9 @@ _SIGNATURES = [
     ("ppo_head_workspace_bytes", C.c_size_t, [i64, i32]),
     ("ppo_gauss_ppo_head", C.c_int, [C.POINTER(LossArgs), C.POINTER(PolicyHead), C.c_void_p, C.c_size_t, f32p,
                                      C.c_void_p, i32, C.c_double, C.c_void_p, i32, C.c_void_p]),
+    ("ppo_gauss_ppo_head_ranged", C.c_int, [C.POINTER(LossArgs), C.POINTER(PolicyHead), C.POINTER(HeadRanges),
+                                            C.c_void_p, C.c_size_t, f32p, C.c_void_p, i32, C.c_double, C.c_void_p,
+                                            i32, C.c_void_p]),
     ("ppo_gauss_sample", C.c_int, [f32p, i64, f32p, i32, C.c_double, C.c_double, f32p, i64, f32p, i64, f32p, f32p,
                                    i64, i64, i32, C.c_void_p]),
     ("ppo_host_randperm", C.c_int, [C.c_void_p, C.c_size_t, i64, C.c_void_p]),

@@ -27,7 +27,7 @@
 #include <cstdlib>
 #include <cstring>
 
-#include "gemm_core.hpp"
+#include "gemm_f16.hpp"
 
 namespace ppo {
 namespace {
@@ -183,6 +183,11 @@ __global__ __launch_bounds__(256) void transpose_kernel(const TransposeGroup g) 
   }
 }
 
+// Below this k the two-part split's own error (7e-8 of a product, root mean square) is more than what bf16x6's six
+// roundings per k-group add up to: relative errors against fp64 of 7.3e-8 / 3.8e-8 (fp16x3 / bf16x6) at k = 16, 7.2e-8 /
+// 7.0e-8 at 48, 8.0e-8 / 1.0e-7 at 96, 1.2e-7 / 2.4e-7 at 512.
+constexpr int kF16MinK = 64;
+
 // Weight-grad: 128 x 128 tiles; split-K over the rows, in chunks that are multiples of the deepest (64-row) slab.
 // The split count fills ONE wave of resident blocks and no more: the bf16x6 tile runs three blocks per CU (the fp32
 // one two), so 768 blocks on the 256 CUs of a whole MI355X (fewer on a partitioned one).  A launch of 1,050 blocks
@@ -191,6 +196,7 @@ __global__ __launch_bounds__(256) void transpose_kernel(const TransposeGroup g) 
 // largest capacity, kDwMaxConcurrent, and a launch on a smaller device uses fewer splits, i.e. less workspace.
 constexpr int kDwBM = 128, kDwBN = 128, kDwChunk = 64;
 constexpr int kDwBlocksPerCu = 3;     // the bf16x6 kernel (168 VGPRs, 48 KiB LDS)
+constexpr int kDwF16BlocksPerCu = 2;  // the fp16x3 kernel (two accumulators: 256 VGPRs, 64 KiB LDS)
 constexpr int kDwF32BlocksPerCu = 2;  // the fp32 kernel, for operands without 16-byte rows
 constexpr int kDwMaxConcurrent = kDwBlocksPerCu * 256;
 
@@ -361,6 +367,131 @@ int launch_nt_bx6(Group& g, int count, hipStream_t s, const char* name, bool bf1
   return go(gemm_nt_bx6_kernel<128, 3, EPI, 2, true>);
 }
 
+// fp16x3 (every problem's operand ranges given) or the bf16-operand mode on gemm_nt_f16_kernel, under the requirements
+// of the bf16x6 kernel except that fp16x3 takes any k from kF16MinK (its last slab is masked).
+template <int EPI, bool BKM, int AR>
+int launch_nt_f16(Group& g, int count, hipStream_t s, const char* name) {
+  auto fits = [](const float* c, int64_t rows, int64_t ld) {
+    return c == nullptr || (w16_ok(c, ld) && rows * ld * 4 < (int64_t(1) << 31));
+  };
+  for (int i = 0; i < count; ++i) {
+    const Problem& p = g.p[i];
+    if (AR == ARITH_F16X3 && (p.amax_a == nullptr || p.amax_b == nullptr || p.K < kF16MinK)) return PPO_EUNSUPPORTED;
+    if (!w16_ok(p.A, p.lda) || !w16_ok(p.B, p.ldb) || (AR == ARITH_BF16 && p.K % 16 != 0) || p.N % 4 != 0)
+      return PPO_EUNSUPPORTED;
+    if (!fits(p.C, p.M, p.ldc) || (epi_fwd_act(EPI) && !fits(p.C2, p.M, p.ldc2))) return PPO_EUNSUPPORTED;
+    if (epi_act_grad(EPI) && !w16_ok(p.aux, p.ldaux)) return PPO_EUNSUPPORTED;
+    if ((EPI == EPI_BIAS || epi_fwd_act(EPI)) && reinterpret_cast<uintptr_t>(p.vec) % 16 != 0)
+      return PPO_EUNSUPPORTED;
+  }
+  int bn = 128, blocks, max_n = 0;
+  for (int i = 0; i < count; ++i) max_n = std::max(max_n, g.p[i].N);
+  if (int rc = assign_blocks(g, count, 128, bn, name, blocks)) return rc;
+  if (blocks == 0) return PPO_OK;
+  // 128 x 64 tiles (256 threads, three blocks per CU) where 128 x 128 ones would be half empty (24,576 rows, two
+  // problems: outputs 48 wide 35.5 -> 25.0 us) or would leave compute units without a block
+  if (max_n <= 64 || blocks < device_info().cus) {
+    bn = 64;
+    if (int rc = assign_blocks(g, count, 128, bn, name, blocks)) return rc;
+  }
+  auto go = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, s, g);
+    return check_launch(name);
+  };
+  if (bn == 64) return go(gemm_nt_f16_kernel<64, 2, 3, EPI, BKM, AR>, 256);
+  // 128 x 128: eight waves of 32 x 64 (128 registers, four waves per SIMD) for the forward, whose epilogue's activation
+  // then overlaps other waves' products (512 -> 256 features: 56 us against 63 with four waves of 64 x 64, 240 -> 512:
+  // 66 against 73); the input-grad's longer staging and epilogue do not fit 128 registers (74 against 69 us)
+  if constexpr (BKM) return go(gemm_nt_f16_kernel<128, 2, 2, EPI, BKM, AR>, 256);
+  else return go(gemm_nt_f16_kernel<128, 4, 4, EPI, BKM, AR>, 512);
+}
+
+// The 128 x 128 (128 x 64 for problems at most 64 columns wide) split-K weight-grad tiles of gemm_f16.hpp; the caller
+// has checked the operands.
+template <int OCC, int AR>
+int launch_tn_f16(Group& g, int count, hipStream_t s, const char* name) {
+  int blocks;
+  if (int rc = assign_blocks(g, count, 128, 128, name, blocks)) return rc;
+  blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    Problem& p = g.p[i];
+    p.tn64 = p.N <= 64 ? 1 : 0;
+    p.tiles_n = static_cast<int>(ceil_div(p.N, p.tn64 ? 64 : 128));
+    p.block_begin = blocks;
+    blocks += p.tiles_m * p.tiles_n * p.splits;  // (at most the 128 x 128 count assign_blocks checked)
+  }
+  if (blocks == 0) return PPO_OK;
+  hipLaunchKernelGGL((gemm_tn_f16_kernel<2, OCC, AR>), dim3(blocks), dim3(256), 0, s, g);
+  return check_launch(name);
+}
+
+// Largest magnitudes of a few tensors: block b of kAmaxSlots per item writes slot b (or raises it), 64 rows apart;
+// the last grid row clears the caller's words.
+struct AmaxGroup {
+  ppo_amax_item it[PPO_MAX_AMAX_ITEMS];
+  int32_t count, raise;
+  uint32_t* clear;
+  int64_t clear_words;
+};
+__global__ __launch_bounds__(256) void amax_kernel(const AmaxGroup g) {
+  const int b = blockIdx.x;
+  if (static_cast<int>(blockIdx.y) == g.count) {
+    for (int64_t i = int64_t(b) * 256 + threadIdx.x; i < g.clear_words; i += int64_t(kAmaxSlots) * 256) g.clear[i] = 0;
+    return;
+  }
+  const ppo_amax_item& T = g.it[blockIdx.y];
+  float m = T.least;
+  auto take = [&](float x) {
+    x = fabsf(x);
+    if (x < __builtin_inff()) m = fmaxf(m, x);
+  };
+  const bool vec = reinterpret_cast<uintptr_t>(T.x) % 16 == 0 && T.ld % 4 == 0;
+  const int q4 = vec ? T.cols >> 2 : 0;  // 16-byte pieces of a row, then its last columns one by one
+  const int rest = T.cols - 4 * q4;
+  const int64_t pieces = T.rows * q4, step = int64_t(kAmaxSlots) * 256;
+  for (int64_t i = int64_t(b) * 256 + threadIdx.x; i < pieces; i += 4 * step) {
+    f32x4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t k = min(i + j * step, pieces - 1);
+      v[j] = *reinterpret_cast<const f32x4*>(T.x + (k / q4) * T.ld + 4 * (k % q4));
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) take(v[j][c]);
+  }
+  if (rest > 0)
+    for (int64_t i = int64_t(b) * 256 + threadIdx.x; i < T.rows * rest; i += step)
+      take(T.x[(i / rest) * T.ld + 4 * q4 + i % rest]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  __shared__ float red[4];
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  if (g.raise) atomicMax(T.slots + b * kAmaxStride, __builtin_bit_cast(uint32_t, m));
+  else T.slots[b * kAmaxStride] = __builtin_bit_cast(uint32_t, m);
+}
+
+// A contiguous tensor counts as one row.
+void add_amax(AmaxGroup& g, const float* x, int64_t ld, int64_t rows, int cols, uint32_t* slots) {
+  ppo_amax_item& t = g.it[g.count++];
+  t.x = x; t.slots = slots;
+  t.rows = rows; t.cols = cols; t.ld = ld;
+  if (ld == cols && rows * cols <= INT32_MAX) {
+    t.cols = static_cast<int32_t>(rows * cols);
+    t.ld = (t.cols + 3) / 4 * 4;
+    t.rows = 1;
+  }
+}
+
+int launch_amax(const AmaxGroup& g, hipStream_t s, const char* who) {
+  hipLaunchKernelGGL(amax_kernel, dim3(kAmaxSlots, g.count + (g.clear_words > 0 ? 1 : 0)), dim3(256), 0, s, g);
+  return check_launch(who);
+}
+
 // Tile of the persistent NT launches: 0 = none (gemm_nt_kernel only).  A PPO_HIP_TUNING build reads `var`
 // (0 = off, 1..) for sweeps.
 int pipe_tile(const char* var, int dflt) {
@@ -425,6 +556,26 @@ namespace {
 
 bool flags_ok(int32_t flags) { return (flags & ~PPO_GEMM_BF16_OPERANDS) == 0; }
 
+void set_range(Problem& p, const ppo_gemm_range* ranges, int i) {
+  if (ranges == nullptr) return;
+  p.amax_a = ranges[i].a;
+  p.amax_b = ranges[i].b;
+  p.amax_c = ranges[i].out;
+}
+
+// After a launch of kernels that do not track their outputs' largest magnitude: a pass over the outputs that want it.
+int raise_outputs(const Group& g, int count, bool c2, hipStream_t s, const char* who) {
+  AmaxGroup ag{};
+  ag.raise = 1;
+  for (int i = 0; i < count; ++i) {
+    const Problem& p = g.p[i];
+    if (p.amax_c == nullptr) continue;
+    const float* x = c2 && p.C2 != nullptr ? p.C2 : p.C;
+    add_amax(ag, x, x == p.C2 ? p.ldc2 : p.ldc, p.M, p.N, p.amax_c);
+  }
+  return ag.count > 0 ? launch_amax(ag, s, who) : PPO_OK;
+}
+
 }  // namespace
 }  // namespace ppo
 
@@ -435,6 +586,12 @@ extern "C" int ppo_linear_fwd(const ppo_linear_fwd_problem* problems, int32_t co
 
 extern "C" int ppo_linear_fwd_ex(const ppo_linear_fwd_problem* problems, int32_t count, int64_t rows,
                                  int32_t activation, int32_t flags, ppo_stream_t stream) {
+  return ppo_linear_fwd_ranged(problems, nullptr, count, rows, activation, flags, stream);
+}
+
+extern "C" int ppo_linear_fwd_ranged(const ppo_linear_fwd_problem* problems, const ppo_gemm_range* ranges,
+                                     int32_t count, int64_t rows, int32_t activation, int32_t flags,
+                                     ppo_stream_t stream) {
   PPO_REQUIRE(flags_ok(flags), "ppo_linear_fwd: flags=%d", flags);
   const bool bf16 = (flags & PPO_GEMM_BF16_OPERANDS) != 0;
   PPO_REQUIRE(problems != nullptr && count >= 1 && count <= PPO_MAX_LINEAR_PROBLEMS,
@@ -464,18 +621,36 @@ extern "C" int ppo_linear_fwd_ex(const ppo_linear_fwd_problem* problems, int32_t
     p.c_vec = (q.z == nullptr || w16_ok(q.z, q.ldz)) && (!elu || q.h == nullptr || w16_ok(q.h, q.ldh));
     if (!elu) p.C2 = nullptr;
     p.act = activation;
+    set_range(p, ranges, i);
     max_n = std::max(max_n, q.out_features);
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   // measured on MI355X for 24576-row mini-batches: outputs wider than 128 like 128x128 tiles with 16-deep slabs,
   // narrower ones 128x64
-  auto run = [&](auto epi_c, const char* name) {
+  bool tracked = false;  // the kernel raised the outputs' slots
+  auto plain = [&](auto epi_c, const char* name) {
     constexpr int EPI = decltype(epi_c)::value;
     const int brc = launch_nt_bx6<EPI>(g, count, s, name, bf16);
-    if (brc != PPO_EUNSUPPORTED) return brc;
+    if (brc != PPO_EUNSUPPORTED) {
+      tracked = elu && !bf16;
+      return brc;
+    }
     const int prc = launch_nt_pipe_tile<EPI>(pipe_tile("PPO_HIP_PIPE_FWD", max_n > 128 ? 1 : 2), g, count, s, name);
     if (prc != PPO_EUNSUPPORTED) return prc;
     return launch_nt_tile<EPI>(pick_tile(max_n > 128 ? T128x128k16s2o3 : T128x64k32s2o4), g, count, s, name);
+  };
+  auto run = [&](auto epi_c, const char* name) {
+    if (!bf16 && ranges != nullptr) {
+      constexpr int EPI = decltype(epi_c)::value;
+      const int rc = EPI == EPI_BIAS_ACT && activation == PPO_ACT_TANH
+                         ? launch_nt_f16<EPI == EPI_BIAS_ACT ? EPI_BIAS_TANH : EPI, false, ARITH_F16X3>(g, count, s, name)
+                     : EPI == EPI_BIAS_ACT && activation == PPO_ACT_RELU
+                         ? launch_nt_f16<EPI == EPI_BIAS_ACT ? EPI_BIAS_RELU : EPI, false, ARITH_F16X3>(g, count, s, name)
+                         : launch_nt_f16<EPI, false, ARITH_F16X3>(g, count, s, name);
+      if (rc != PPO_EUNSUPPORTED) return rc;
+    }
+    const int rc = plain(epi_c, name);
+    return rc == PPO_OK && !tracked ? raise_outputs(g, count, elu, s, name) : rc;
   };
   if (!elu) return run(IntC<EPI_BIAS>{}, "linear_fwd");
   if (activation == PPO_ACT_ELU) return run(IntC<EPI_BIAS_ELU>{}, "linear_fwd_elu");
@@ -530,7 +705,7 @@ bool act_from_output_ok(int act) {
 
 int dx_gemm(const ppo_linear_bwd_dx_problem* problems, int32_t count, int64_t rows, int32_t activation,
             int32_t elu_source, void* workspace, size_t workspace_bytes, ppo_stream_t stream, const char* who,
-            int32_t flags = 0) {
+            int32_t flags = 0, const ppo_gemm_range* ranges = nullptr) {
   PPO_REQUIRE(flags_ok(flags), "%s: flags=%d", who, flags);
   const bool bf16 = (flags & PPO_GEMM_BF16_OPERANDS) != 0;
   PPO_REQUIRE(problems != nullptr && count >= 1 && count <= PPO_MAX_LINEAR_PROBLEMS, "%s: count=%d outside [1, %d]",
@@ -573,9 +748,10 @@ int dx_gemm(const ppo_linear_bwd_dx_problem* problems, int32_t count, int64_t ro
     p.c_vec = w16_ok(q.dz_prev, q.lddz_prev) && (q.z_prev == nullptr || w16_ok(q.z_prev, q.ldz_prev));
     p.elu_from_output = elu_source == PPO_ELU_FROM_OUTPUT;
     p.act = activation;
+    set_range(p, ranges, i);
     max_n = std::max(max_n, q.in_features);
   }
-  auto run = [&](auto epi_c, const char* name) {
+  auto plain = [&](auto epi_c, const char* name) {
     constexpr int EPI = decltype(epi_c)::value;
     // the bf16x6 kernel reads the weights as stored (k-major, 16-byte rows): no transpose
     const int krc = launch_nt_bx6<EPI, true>(g, count, s, name, bf16);
@@ -592,6 +768,20 @@ int dx_gemm(const ppo_linear_bwd_dx_problem* problems, int32_t count, int64_t ro
     const int prc = launch_nt_pipe_tile<EPI>(pipe_tile("PPO_HIP_PIPE_DX", max_n > 128 ? 3 : 2), g, count, s, name);
     if (prc != PPO_EUNSUPPORTED) return prc;
     return launch_nt_tile<EPI>(pick_tile(max_n > 128 ? T64x64k32s2o4 : T128x64k32s2o4), g, count, s, name);
+  };
+  auto run = [&](auto epi_c, const char* name) {
+    if (!bf16 && ranges != nullptr) {
+      constexpr int EPI = decltype(epi_c)::value;
+      const bool out = elu_source == PPO_ELU_FROM_OUTPUT;
+      const int rc = EPI == EPI_ACT_GRAD && activation == PPO_ACT_TANH && out
+                         ? launch_nt_f16<EPI == EPI_ACT_GRAD ? EPI_TANH_GRAD : EPI, true, ARITH_F16X3>(g, count, s, name)
+                     : EPI == EPI_ACT_GRAD && activation == PPO_ACT_RELU
+                         ? launch_nt_f16<EPI == EPI_ACT_GRAD ? EPI_RELU_GRAD : EPI, true, ARITH_F16X3>(g, count, s, name)
+                         : launch_nt_f16<EPI, true, ARITH_F16X3>(g, count, s, name);
+      if (rc != PPO_EUNSUPPORTED) return rc;
+    }
+    const int rc = plain(epi_c, name);
+    return rc == PPO_OK ? raise_outputs(g, count, false, s, name) : rc;
   };
   if (!any_act) return run(IntC<EPI_STORE>{}, "linear_bwd_dx");
   if (activation == PPO_ACT_ELU) return run(IntC<EPI_ELU_GRAD>{}, "linear_bwd_dx_elu");
@@ -621,6 +811,32 @@ extern "C" int ppo_linear_bwd_dx_ex(const ppo_linear_bwd_dx_problem* problems, i
                  "ppo_linear_bwd_dx_ex", flags);
 }
 
+extern "C" int ppo_linear_bwd_dx_ranged(const ppo_linear_bwd_dx_problem* problems, const ppo_gemm_range* ranges,
+                                        int32_t count, int64_t rows, int32_t activation, int32_t source, int32_t flags,
+                                        void* workspace, size_t workspace_bytes, ppo_stream_t stream) {
+  return dx_gemm(problems, count, rows, activation, source, workspace, workspace_bytes, stream,
+                 "ppo_linear_bwd_dx_ranged", flags, ranges);
+}
+
+extern "C" int ppo_amax(const ppo_amax_item* items, int32_t count, uint32_t* clear, int64_t clear_words,
+                        ppo_stream_t stream) {
+  PPO_REQUIRE(count >= 0 && count <= PPO_MAX_AMAX_ITEMS && (count == 0 || items != nullptr),
+              "ppo_amax: count=%d outside [0, %d]", count, PPO_MAX_AMAX_ITEMS);
+  PPO_REQUIRE(clear_words >= 0 && (clear_words == 0 || clear != nullptr), "ppo_amax: clear_words=%lld",
+              (long long)clear_words);
+  AmaxGroup g{};
+  for (int i = 0; i < count; ++i) {
+    const ppo_amax_item& q = items[i];
+    PPO_REQUIRE(q.x && q.slots && q.rows > 0 && q.cols > 0 && q.ld >= q.cols && q.least >= 0.0f, "ppo_amax: item %d", i);
+    add_amax(g, q.x, q.ld, q.rows, q.cols, q.slots);
+    g.it[i].least = q.least;
+  }
+  g.clear = clear;
+  g.clear_words = clear_words;
+  if (g.count == 0 && clear_words == 0) return PPO_OK;
+  return launch_amax(g, static_cast<hipStream_t>(stream), "ppo_amax");
+}
+
 extern "C" size_t ppo_linear_bwd_dw_workspace_bytes(const ppo_linear_bwd_dw_problem* problems, int32_t count,
                                                     int64_t rows) {
   if (problems == nullptr || count < 1 || count > PPO_MAX_LINEAR_PROBLEMS || !rows_ok(rows)) return 0;
@@ -634,7 +850,7 @@ namespace {
 
 int dw_gemm(const ppo_linear_bwd_dw_problem* problems, int32_t count, int64_t rows, void* workspace,
             size_t workspace_bytes, const float* extra_grads, const ppo_grad_range* extra, int32_t num_extra,
-            double* norm, ppo_stream_t stream, int32_t flags = 0) {
+            double* norm, ppo_stream_t stream, int32_t flags = 0, const ppo_gemm_range* ranges = nullptr) {
   PPO_REQUIRE(flags_ok(flags), "ppo_linear_bwd_dw: flags=%d", flags);
   const bool bf16 = (flags & PPO_GEMM_BF16_OPERANDS) != 0;
   PPO_REQUIRE(problems != nullptr && count >= 1 && count <= PPO_MAX_LINEAR_PROBLEMS,
@@ -662,7 +878,12 @@ int dw_gemm(const ppo_linear_bwd_dw_problem* problems, int32_t count, int64_t ro
   bool bx6 = true;
   for (int i = 0; i < count; ++i)
     bx6 = bx6 && w16_ok(problems[i].dz, problems[i].lddz) && w16_ok(problems[i].x, problems[i].ldx);
-  int occ = bx6 ? kDwBlocksPerCu : kDwF32BlocksPerCu;
+  // with every range known, fp16x3 (its k, the rows, from kF16MinK; the kernel needs one whole slab of 32)
+  bool f16 = bx6 && !bf16 && ranges != nullptr && rows >= kF16MinK;
+  for (int i = 0; i < count && f16; ++i)
+    f16 = ranges[i].a != nullptr && ranges[i].b != nullptr &&
+          32 * std::max(problems[i].lddz, problems[i].ldx) * 4 < (int64_t(1) << 31);
+  int occ = f16 ? kDwF16BlocksPerCu : bx6 ? kDwBlocksPerCu : kDwF32BlocksPerCu;
 #ifdef PPO_HIP_TUNING
   const char* cfg = std::getenv("PPO_HIP_DW_CFG");  // tuning aid: other slab depths / stages / occupancies
   if (cfg && !std::strcmp(cfg, "bx6o2")) occ = 2;
@@ -691,6 +912,7 @@ int dw_gemm(const ppo_linear_bwd_dw_problem* problems, int32_t count, int64_t ro
     p.colsum = q.db != nullptr ? reinterpret_cast<double*>(ws + plan.colsum_off[i]) : nullptr;
     p.M = q.out_features; p.N = q.in_features; p.K = static_cast<int>(rows);
     p.splits = plan.splits[i]; p.k_chunk = plan.k_chunk[i];
+    set_range(p, ranges, i);
     ReduceItem& r = rg.it[i];
     r.partial = p.C; r.colsum = p.colsum; r.dw = q.dw; r.db = q.db;
     r.out = q.out_features; r.in = q.in_features; r.ld = static_cast<int>(ldp); r.splits = plan.splits[i];
@@ -723,7 +945,9 @@ int dw_gemm(const ppo_linear_bwd_dw_problem* problems, int32_t count, int64_t ro
     rc = launch_tn_bx6<2>(g, count, s, "linear_bwd_dw");
   } else
 #endif
-  if (bx6) {
+  if (f16) {
+    rc = launch_tn_f16<kDwF16BlocksPerCu, ARITH_F16X3>(g, count, s, "linear_bwd_dw");
+  } else if (bx6) {
     rc = launch_tn_bx6<kDwBlocksPerCu>(g, count, s, "linear_bwd_dw", bf16);
   } else {
     rc = launch_tn<kDwBM, kDwBN, 32, 2, kDwF32BlocksPerCu>(g, count, s, "linear_bwd_dw");
@@ -754,6 +978,15 @@ extern "C" int ppo_linear_bwd_dw_norm(const ppo_linear_bwd_dw_problem* problems,
   PPO_REQUIRE(norm_partials != nullptr, "ppo_linear_bwd_dw_norm: null norm_partials");
   return dw_gemm(problems, count, rows, workspace, workspace_bytes, extra_grads, extra, num_extra, norm_partials,
                  stream);
+}
+
+extern "C" int ppo_linear_bwd_dw_ranged(const ppo_linear_bwd_dw_problem* problems, const ppo_gemm_range* ranges,
+                                        int32_t count, int64_t rows, int32_t flags, void* workspace,
+                                        size_t workspace_bytes, const float* extra_grads, const ppo_grad_range* extra,
+                                        int32_t num_extra, double* norm_partials, ppo_stream_t stream) {
+  PPO_REQUIRE(norm_partials != nullptr || num_extra == 0, "ppo_linear_bwd_dw_ranged: extra ranges need norm_partials");
+  return dw_gemm(problems, count, rows, workspace, workspace_bytes, extra_grads, extra, num_extra, norm_partials,
+                 stream, flags, ranges);
 }
 
 extern "C" int ppo_linear_bwd_dw_ex(const ppo_linear_bwd_dw_problem* problems, int32_t count, int64_t rows,

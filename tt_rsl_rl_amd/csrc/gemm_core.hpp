@@ -27,6 +27,7 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "amax.hpp"
 #include "common.hpp"
 
 namespace ppo {
@@ -46,12 +47,20 @@ enum Epilogue : int {
   EPI_LSTM_BWD = 6,  // one LSTM backward step: hidden-state gradient -> gate gradients (lstm.hip)
   EPI_BIAS_ACT = 7,  // EPI_BIAS_ELU for the other activations (Problem::act)
   EPI_ACT_GRAD = 8,  // EPI_ELU_GRAD for the other activations
+  EPI_BIAS_TANH = 9,   // fp16x3: the epilogues of tanh and ReLU inline (the call per element costs more than the
+  EPI_TANH_GRAD = 10,  // product: 48,000 rows x 400 features, two problems, forward 159 us with the call)
+  EPI_BIAS_RELU = 11,
+  EPI_RELU_GRAD = 12,
 };
 // The forward epilogues that add the bias and apply an activation, and the input-grad epilogues that multiply by its
 // derivative: ELU's own (the kernels every workload here runs, unchanged by the others' existence) and the generic
 // ones, which evaluate Problem::act per element.
-constexpr bool epi_fwd_act(int e) { return e == EPI_BIAS_ELU || e == EPI_BIAS_ACT; }
-constexpr bool epi_act_grad(int e) { return e == EPI_ELU_GRAD || e == EPI_ACT_GRAD; }
+constexpr bool epi_fwd_act(int e) {
+  return e == EPI_BIAS_ELU || e == EPI_BIAS_ACT || e == EPI_BIAS_TANH || e == EPI_BIAS_RELU;
+}
+constexpr bool epi_act_grad(int e) {
+  return e == EPI_ELU_GRAD || e == EPI_ACT_GRAD || e == EPI_TANH_GRAD || e == EPI_RELU_GRAD;
+}
 constexpr bool epi_generic(int e) { return e == EPI_BIAS_ACT || e == EPI_ACT_GRAD; }
 
 
@@ -81,6 +90,9 @@ struct Problem {
   const float* vec;  // bias [N]
   const float* aux;  // ELU'-source z_prev [M, N]
   double* colsum;    // [splits, M] sums of A over each split's k range (fp64: bias grads cancel heavily)
+  const uint32_t* amax_a;  // fp16x3 kernels: the operands' largest magnitudes (PPO_AMAX_SLOTS words each)
+  const uint32_t* amax_b;
+  uint32_t* amax_c;        // where the NT kernels leave the output's (null: not wanted)
   int64_t lda, ldb, ldc, ldc2, ldaux;
   int64_t partial_stride;  // floats between split partials of C
   int32_t M, N, K;
@@ -223,11 +235,65 @@ __device__ __forceinline__ void act_grad4(int act, int from_output, const f32x4&
 }
 
 
+// ELU with the degree-4 polynomial q that minimises the largest relative error of x + x^2 q(x) on [-0.7, 0] (least
+// squares reweighted towards the largest residual: 1.1e-8 before rounding, 1.07 ulp after against the Taylor form's
+// 1.21, root mean square 2.6e-8 as there) instead of elu_fwd's degree-7 Taylor one: three multiply-adds less per output
+// element of an epilogue that runs while the matrix cores wait.
+__device__ __forceinline__ float elu_fast(float x) {
+  float q = 0.0010357097489759326f;
+  q = fmaf(q, x, 0.008073252625763416f);
+  q = fmaf(q, x, 0.04157695546746254f);
+  q = fmaf(q, x, 0.16665293276309967f);
+  q = fmaf(q, x, 0.4999993145465851f);
+  const float near0 = fmaf(x * x, q, x);
+  const float far = __builtin_amdgcn_exp2f(x * 1.4426950408889634f) - 1.0f;
+  return x > 0.0f ? x : (x > -0.7f ? near0 : far);
+}
+
+// tanh: on |x| < 0.55 x + x^3 q(x^2) with q of degree 4 fitted as above (4e-10 before rounding), beyond
+// 1 - 2 / (2^(2 |x| log2 e) + 1) on the hardware exp2 and reciprocal: within 2 ulp.
+__device__ __forceinline__ float tanh_fast(float x) {
+  const float x2 = x * x, ax = fabsf(x);
+  float q = -0.006274241488426924f;
+  q = fmaf(q, x2, 0.021071679890155792f);
+  q = fmaf(q, x2, -0.05385230854153633f);
+  q = fmaf(q, x2, 0.13332585990428925f);
+  q = fmaf(q, x2, -0.33333316445350647f);
+  const float near0 = fmaf(x * x2, q, x);
+  const float t = 1.0f - 2.0f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(ax * 2.8853900817779268f) + 1.0f);
+  return ax < 0.55f ? near0 : __builtin_copysignf(t, x);
+}
+
+template <int EPI>
+__device__ __forceinline__ void act_fwd4_fast(int act, const f32x4& o, f32x4& o2) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    o2[e] = EPI == EPI_BIAS_ELU    ? elu_fast(o[e])
+            : EPI == EPI_BIAS_TANH ? tanh_fast(o[e])
+            : EPI == EPI_BIAS_RELU ? (o[e] > 0.0f ? o[e] : 0.0f)
+                                   : act_fwd(act, o[e]);
+}
+
+template <int EPI>
+__device__ __forceinline__ void act_grad4_fast(int act, int from_output, const f32x4& x, const f32x4& src, f32x4& o) {
+  if constexpr (EPI == EPI_TANH_GRAD) {  // (from the output)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = x[e] * (1.0f - src[e] * src[e]);
+  } else if constexpr (EPI == EPI_RELU_GRAD) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = x[e] * (src[e] > 0.0f ? 1.0f : 0.0f);
+  } else {
+    act_grad4<epi_generic(EPI)>(act, from_output, x, src, o);
+  }
+}
+
 struct Group {
   Problem p[PPO_MAX_LINEAR_PROBLEMS];
   int32_t count;
   int32_t xcds;  // > 1: the device's XCDs; block ids are permuted so each XCD gets a contiguous range of tiles
 };
+
+static_assert(sizeof(Group) <= 4096, "kernel arguments");
 
 constexpr int kThreads = 256;
 
@@ -864,10 +930,15 @@ __device__ __forceinline__ void store_b128(__amdgpu_buffer_rsrc_t r, uint32_t of
 
 // The epilogue of one wave's (TM x TN) 32 x 32 accumulator tiles (layout as in gemm_nt_tile): each tile through the
 // wave's own LDS patch, finished in row order, TM * TN * 4 * OUTS buffer stores in every lane.
-template <int TM, int TN, int EPI, bool GEN>
-__device__ __forceinline__ void nt_pipe_epilogue_t(const Problem& P, const f32x16 (&acc)[TM][TN], int row0w,
-                                                   int col0w, float* patch, int lane) {
+// SCALED (the fp16x3 kernel): the accumulators hold 1 / (s0 s1) times the product, and the activations are the fast
+// forms.  AMAX: returns the largest magnitude among the values this lane wrote (the activation's output of a forward
+// layer).
+template <int TM, int TN, int EPI, bool GEN, bool SCALED = false, bool AMAX = SCALED>
+__device__ __forceinline__ float nt_pipe_epilogue_t(const Problem& P, const f32x16 (&acc)[TM][TN], int row0w,
+                                                    int col0w, float* patch, int lane, float s0 = 1.0f,
+                                                    float s1 = 1.0f) {
   constexpr int PS = 36;
+  [[maybe_unused]] float amax = 0.0f;
   const int h = lane >> 5;
   const int pr = lane >> 3, pc = 4 * (lane & 7);
   const int M = P.M, N = P.N;
@@ -909,26 +980,42 @@ __device__ __forceinline__ void nt_pipe_epilogue_t(const Problem& P, const f32x1
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
         const int r = pr + 8 * rr;
-        const f32x4 x = *reinterpret_cast<const f32x4*>(patch + r * PS + pc);
+        f32x4 x = *reinterpret_cast<const f32x4*>(patch + r * PS + pc);
+        if constexpr (SCALED) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = EPI == EPI_BIAS || epi_fwd_act(EPI) ? x[e] * s0 : x[e] * s0 * s1;
+        }
         const int m = row0w + i * 32 + r;
         const bool ok = m < M && n_in;
         const int64_t mm = ok ? m : 0;
-        f32x4 o, o2;
+        f32x4 o, o2 = {};
         if constexpr (EPI == EPI_BIAS || epi_fwd_act(EPI)) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = x[e] + bias[j][e];
-          if constexpr (epi_fwd_act(EPI)) act_fwd4<GEN>(P.act, o, o2);
+          for (int e = 0; e < 4; ++e) o[e] = SCALED ? fmaf(x[e], s1, bias[j][e]) : x[e] + bias[j][e];
+          if constexpr (epi_fwd_act(EPI)) {
+            if constexpr (SCALED) act_fwd4_fast<EPI>(P.act, o, o2);
+            else act_fwd4<GEN>(P.act, o, o2);
+          }
         } else if constexpr (epi_act_grad(EPI)) {
-          act_grad4<GEN>(P.act, P.elu_from_output, x, zsrc[i][j][rr], o);
+          if constexpr (SCALED) act_grad4_fast<EPI>(P.act, P.elu_from_output, x, zsrc[i][j][rr], o);
+          else act_grad4<GEN>(P.act, P.elu_from_output, x, zsrc[i][j][rr], o);
         } else {
           o = x;
         }
         store_b128(rc, ok ? static_cast<uint32_t>((mm * P.ldc + n) * 4) : kDropOffset, o);
         if constexpr (epi_fwd_act(EPI))
           store_b128(rc2, ok ? static_cast<uint32_t>((mm * P.ldc2 + n) * 4) : kDropOffset, o2);
+        if constexpr (AMAX) {
+          const f32x4 w = epi_fwd_act(EPI) ? o2 : o;
+          float q = amax;
+          raise2(q, w[0], w[1]);
+          raise2(q, w[2], w[3]);
+          amax = ok ? q : amax;
+        }
       }
     }
   }
+  return amax;
 }
 
 template <int TM, int TN, int EPI>
@@ -1955,7 +2042,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(OCC, O
   }
   if (kt < nk) step(kt, cs, RB_EVEN, 1 - RB_EVEN);
   float* const patch = reinterpret_cast<float*>(lds) + wave * 32 * PS;  // every wave is past the last barrier
-  nt_pipe_epilogue<TM, TN, EPI>(P, acc, row0 + wm * 64, col0 + wn * (BN / 2), patch, lane);
+  if constexpr (epi_fwd_act(EPI) && !BF16) {
+    const float m = nt_pipe_epilogue_t<TM, TN, EPI, epi_generic(EPI), false, true>(P, acc, row0 + wm * 64,
+                                                                                  col0 + wn * (BN / 2), patch, lane);
+    if (P.amax_c != nullptr) amax_publish(P.amax_c, m, lane, 4 * blockIdx.x + wave);
+  } else {
+    nt_pipe_epilogue<TM, TN, EPI>(P, acc, row0 + wm * 64, col0 + wn * (BN / 2), patch, lane);
+  }
 }
 
 // 16-byte direct loads need a 16-byte aligned base and a leading dimension that is a multiple of 4.

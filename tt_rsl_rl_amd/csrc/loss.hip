@@ -12,6 +12,7 @@
 // 50/50 on a tie; clamp() passes it on the closed interval [lo, hi].
 #include <cstdlib>
 
+#include "amax.hpp"
 #include "common.hpp"
 
 #pragma clang fp contract(off)
@@ -323,6 +324,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 struct HeadParams {
   LossParams lp;
   ppo_policy_head h;
+  ppo_head_ranges ranges;
 };
 
 __device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
@@ -462,6 +464,7 @@ __global__ __launch_bounds__(64 * WAVES) void ppo_head_kernel(const HeadParams P
   double acc_dstd[8];
 #pragma unroll
   for (int v = 0; v < 8; ++v) acc_dstd[v] = 0.0;
+  float max_dza = 0.0f, max_dzc = 0.0f, max_dm = 0.0f, max_dv = 0.0f;
 
   for (; tile < tiles; tile += stride) {
     const int64_t row = tile * kHeadRows + m;
@@ -509,12 +512,15 @@ __global__ __launch_bounds__(64 * WAVES) void ppo_head_kernel(const HeadParams P
             o[e] = in.hc[g][e] > 0.0f ? x : x * (in.hc[g][e] + 1.0f);
           }
           st4(H.dz_critic + row * H.ld_dz_critic + 16 * g + 4 * q, o);
+          raise2(max_dzc, o[0], o[1]);
+          raise2(max_dzc, o[2], o[3]);
         }
       }
       if (q == 0) {
         a.d_value[row * a.ld_dvalue] = dv;
         if (H.value) H.value[row * H.ld_value] = v;
         acc_val += static_cast<double>(vloss);
+        raise2(max_dv, dv, dv);
       }
     }
 
@@ -600,6 +606,8 @@ __global__ __launch_bounds__(64 * WAVES) void ppo_head_kernel(const HeadParams P
       for (int t = 0; t < 2; ++t) {
         const int c = 16 * t + 4 * q;
         if (c < A) {
+          raise2(max_dm, dm[4 * t], dm[4 * t + 1]);  // (zero past the actions)
+          raise2(max_dm, dm[4 * t + 2], dm[4 * t + 3]);
           st4_masked(a.d_mean + row * a.ld_dmean, c, A, f32x4{dm[4 * t], dm[4 * t + 1], dm[4 * t + 2], dm[4 * t + 3]});
           if (H.mean) st4_masked(H.mean + row * H.ld_mean, c, A, f32x4{mu[4 * t], mu[4 * t + 1], mu[4 * t + 2],
                                                                          mu[4 * t + 3]});
@@ -626,11 +634,19 @@ __global__ __launch_bounds__(64 * WAVES) void ppo_head_kernel(const HeadParams P
 #pragma unroll
           for (int e = 0; e < 4; ++e) o[e] = hv[e] > 0.0f ? acc2[e] : acc2[e] * (hv[e] + 1.0f);
           st4(H.dz_actor + row * H.ld_dz_actor + 16 * kt + 4 * q, o);
+          raise2(max_dza, o[0], o[1]);
+          raise2(max_dza, o[2], o[3]);
         }
       }
     }
     if (tile + stride < tiles) head_load_tile(P, tile + stride, lane, in);
   }
+
+  const int slot = WAVES * blockIdx.x + wave;
+  if (P.ranges.dz_actor) amax_publish(P.ranges.dz_actor, max_dza, lane, slot);
+  if (P.ranges.dz_critic) amax_publish(P.ranges.dz_critic, max_dzc, lane, slot);
+  if (P.ranges.d_mean) amax_publish(P.ranges.d_mean, max_dm, lane, slot);
+  if (P.ranges.d_value) amax_publish(P.ranges.d_value, max_dv, lane, slot);
 
   // block partials: wave sums, the per-action std-gradient terms folded over the 16 rows of each quarter, then the
   // waves in a fixed order; column-major [cols][blocks] like ppo_loss_kernel's, for ppo_loss_finalize_kernel
@@ -813,6 +829,14 @@ extern "C" int ppo_gauss_ppo_head(const ppo_loss_args* args, const ppo_policy_he
                                   size_t workspace_bytes, float* d_std_param, ppo_device_state* state,
                                   int32_t adaptive, double desired_kl, double* trace, int32_t trace_rows,
                                   ppo_stream_t stream) {
+  return ppo_gauss_ppo_head_ranged(args, head, nullptr, workspace, workspace_bytes, d_std_param, state, adaptive,
+                                   desired_kl, trace, trace_rows, stream);
+}
+
+extern "C" int ppo_gauss_ppo_head_ranged(const ppo_loss_args* args, const ppo_policy_head* head,
+                                         const ppo_head_ranges* ranges, void* workspace, size_t workspace_bytes,
+                                         float* d_std_param, ppo_device_state* state, int32_t adaptive,
+                                         double desired_kl, double* trace, int32_t trace_rows, ppo_stream_t stream) {
   static const char* who = "ppo_gauss_ppo_head";
   PPO_REQUIRE(args != nullptr && head != nullptr, "%s: null args / head", who);
   PPO_REQUIRE(trace == nullptr || trace_rows > 0, "%s: trace_rows=%d", who, trace_rows);
@@ -840,6 +864,7 @@ extern "C" int ppo_gauss_ppo_head(const ppo_loss_args* args, const ppo_policy_he
                   (h.value == nullptr || h.ld_value >= 1),
               "%s: rows must be 16-byte aligned with leading dimensions that are multiples of 4 floats", who);
   P.h = h;
+  if (ranges != nullptr) P.ranges = *ranges;
   const size_t need = ppo_head_workspace_bytes(a.rows, a.num_actions);
   PPO_REQUIRE(workspace != nullptr && workspace_bytes >= need, "%s: workspace too small (%zu < %zu)", who,
               workspace_bytes, need);

@@ -35,6 +35,15 @@ def _align4(n: int) -> int:
 K_SLACK = 16
 
 
+# Mini-batches of at least this many rows run their GEMMs as fp16x3 (two fp16 parts per operand, csrc/gemm_f16.hpp), the
+# others as bf16x6.  fp16x3 is the faster and the closer to fp64 at every size (24,576 rows, humanoid: 8.9 against 10.0
+# ms per update; weight-grads of 393,216 rows: 4e-7 relative error against 2e-6).  What the line keeps is the trajectory
+# of smaller updates: any other rounding puts a row now and then on the other side of a clip boundary, which moves that
+# step's gradient by about 1 / sqrt(rows), and twenty steps carry it on (humanoid, 16 seeds, two updates: first moments
+# up to 4.5e-2 apart on 8 of them; 393,216 rows: 8e-4 at most on 4).  1 / sqrt(40,000) is 5e-3.
+RANGED_ROWS = 40_000
+
+
 def _pad16(n: int) -> int:
     return (n + 15) // 16 * 16
 
@@ -86,6 +95,10 @@ class ModelBuffers:
         self.h = [buf(w) for w in self.widths[:-1]]     # hidden layers' act(z)
         self.z = None if self.from_output else [buf(w) for w in self.widths[:-1]]
         self.dz = [buf(w) for w in self.widths]
+
+        # largest-magnitude slots of h (hidden layers) and dz (all), set by the engine
+        self.h_max: list[torch.Tensor] = []
+        self.dz_max: list[torch.Tensor] = []
 
     def act_src(self, i: int, R: int) -> torch.Tensor:
         """What the input-grad below hidden layer i reads for act': h (from the output) or z."""
@@ -200,6 +213,7 @@ class UpdateEngine:
                     self.w0_mirrors.append((alg.flat.offsets[id(w)][0], w.shape[0], w.shape[1], wp))
         self.buf_a = ModelBuffers(actor, self.R_max, self.device)
         self.buf_c = ModelBuffers(critic, self.R_max, self.device)
+        self._init_ranges()
         self.loss_ws = torch.empty(ops.loss_workspace_bytes(self.R_max, self.A), dtype=torch.uint8, device=self.device)
         # learn_std=False (distribution.py:166): the std parameter takes no gradient; the loss kernels' gradient for it
         # goes here instead of into the flat gradient, whose slot stays zero, so Adam leaves the parameter (and its
@@ -238,6 +252,49 @@ class UpdateEngine:
         # are enqueued, before the next mini-batch's; the buffers then hold that mini-batch's activations / gradients.
         # It must not change the parameters: within a run the padded first-layer copies follow the Adam steps only
         self.step_hook = None
+
+    # -- largest magnitudes of the GEMMs' operands ----------------------------------------------------------------------
+    def _init_ranges(self) -> None:
+        """Slots for every GEMM operand's largest |x| (ops.amax): with them the GEMMs run as fp16x3.  The table's are
+        written with the gather, the weights' at the start of every mini-batch (one small launch, which also clears
+        the activations' and gradients', raised by the kernels that write those).  Not used with bf16 operands."""
+        la, lc = self._layers()
+        n = len(la)
+        act = self._range_act = ops.new_amax(2 * (2 * n - 1) + self._extra_ranges(), self.device)
+        rows = iter(act)
+        for b in (self.buf_a, self.buf_c):
+            b.h_max = [next(rows) for _ in range(n - 1)]
+            b.dz_max = [next(rows) for _ in range(n)]
+        self._extra_max = list(rows)
+        fixed = ops.new_amax(2 + 2 * n, self.device)
+        self.xa_max, self.xc_max = fixed[0], fixed[0] if self.layout.shared_obs else fixed[1]
+        self.w_max = (list(fixed[2:2 + n]), list(fixed[2 + n:]))
+
+    def _extra_ranges(self) -> int:
+        return 0
+
+    @property
+    def ranged(self) -> bool:
+        return self.R_max >= RANGED_ROWS and not self.alg.use_mixed_precision
+
+    def _table_ranges(self, rows: int) -> None:
+        """Largest magnitudes of the first `rows` table rows' observation blocks, as wide as the first layers read
+        them."""
+        lay, alg = self.layout, self.alg
+        items = []
+        for model, col, slots in ((alg.actor, lay.xa, self.xa_max), (alg.critic, lay.xc, self.xc_max)):
+            wp = self.w0_pad.get(id(model))
+            width = model.obs_dim if wp is None else wp.shape[1]
+            items.append((self.table[:rows, col:col + width], slots))
+        ops.amax(items[:1] if lay.shared_obs else items)
+
+    def _weight_ranges(self, extra: list[tuple] = ()) -> None:
+        items = [(lin.weight, slots) for lins, maxes in zip(self._layers(), self.w_max)
+                 for lin, slots in zip(lins, maxes)] + list(extra)
+        clear = self._range_act
+        for i in range(0, len(items), L.MAX_AMAX_ITEMS):
+            ops.amax(items[i:i + L.MAX_AMAX_ITEMS], clear)
+            clear = None
 
     # -- one update ------------------------------------------------------------------------------------------------
     def _ensure_trace(self) -> None:
@@ -333,6 +390,8 @@ class UpdateEngine:
         dst = self.table[row0:row0 + perm.numel()]
         for i in range(0, len(segs), L.MAX_GATHER_SEGMENTS):
             ops.gather_rows(perm, segs[i:i + L.MAX_GATHER_SEGMENTS], dst)
+        if self.ranged:
+            self._table_ranges(row0 + perm.numel())
 
     def segments(self) -> list[ops.Segment]:
         """The packed table's column blocks and their storage sources ([T * N, width] views)."""
@@ -399,12 +458,14 @@ class UpdateEngine:
         adv_col = self.advantage_column(tab, R)
         if not (self.w0_mirrors and self._w0_current):  # (a caller may have changed the weights since)
             self.refresh_padded_weights()
+        if self.ranged:
+            self._weight_ranges()
         fa, wa0 = self._first_layer(alg.actor, tab, lay.xa, xa)
         fc, wc0 = self._first_layer(alg.critic, tab, lay.xc, xc)
         self.head_forward(fa, fc, R, w0=(wa0, wc0))
         self.loss(tab, R, adv_col)
         self.head_backward(R)
-        self.weight_grads(self.head_dw(xa, xc, R), R, norm=self.grad_norm)
+        self.weight_grads(self.head_dw(xa, xc, R), R, norm=self.grad_norm, ranges=self.dw_ranges())
         self.adam(step, prenorm=self.grad_norm.partials if self.grad_norm is not None else None)
 
     # -- pieces shared with the recurrent engine ----------------------------------------------------------------------
@@ -422,6 +483,17 @@ class UpdateEngine:
             raise NotImplementedError("actor and critic must have the same number of layers")
         return la, lc
 
+    def _input_max(self) -> tuple[torch.Tensor, torch.Tensor]:
+        """Slots of the heads' inputs (actor, critic)."""
+        return self.xa_max, self.xc_max
+
+    def dw_ranges(self) -> list[tuple] | None:
+        """Ranges of head_dw's problems."""
+        if not self.ranged:
+            return None
+        return [(dz, x, None) for b, x0 in zip((self.buf_a, self.buf_c), self._input_max())
+                for dz, x in zip(b.dz_max, (x0, *b.h_max))]
+
     def head_forward(self, xa: torch.Tensor, xc: torch.Tensor, R: int, w0: tuple | None = None) -> None:
         """The MLPs, actor and critic grouped layer by layer (hidden layers keep only elu(z)).  w0: the first layer's
         (actor, critic) weights to use in place of the parameters (zero-padded copies, with inputs as wide)."""
@@ -434,18 +506,23 @@ class UpdateEngine:
             last = i == nl - 1
             wa, wc = w0 if i == 0 and w0 is not None else (la[i].weight, lc[i].weight)
             probs = []
+            rng = [None, None]
+            if self.ranged:
+                rng = [[(x0 if i == 0 else b.h_max[i - 1], w[i], None if last else b.h_max[i])]
+                       for b, x0, w in zip((ba, bc), self._input_max(), self.w_max)]
             for b, x, w, lin in ((ba, ins_a[-1], wa, la[i]), (bc, ins_c[-1], wc, lc[i])):
                 z = b.out[:R] if last else (b.z[i][:R] if b.z is not None else None)
                 probs.append((x, w, lin.bias, z, None if last else b.h[i][:R]))
             tm.start(f"fwd{i}")
             bf16 = self.alg.use_mixed_precision
+            both = rng[0] + rng[1] if self.ranged else None
             if last:
-                ops.linear_fwd(probs, R, act=L.PPO_ACT_NONE, bf16=bf16)
+                ops.linear_fwd(probs, R, act=L.PPO_ACT_NONE, bf16=bf16, ranges=both)
             elif ba.act == bc.act:
-                ops.linear_fwd(probs, R, act=ba.act, bf16=bf16)
+                ops.linear_fwd(probs, R, act=ba.act, bf16=bf16, ranges=both)
             else:  # (actor and critic with different activations: one launch each)
-                ops.linear_fwd(probs[:1], R, act=ba.act, bf16=bf16)
-                ops.linear_fwd(probs[1:], R, act=bc.act, bf16=bf16)
+                ops.linear_fwd(probs[:1], R, act=ba.act, bf16=bf16, ranges=rng[0])
+                ops.linear_fwd(probs[1:], R, act=bc.act, bf16=bf16, ranges=rng[1])
             tm.stop(f"fwd{i}")
             if not last:
                 ins_a.append(ba.h[i][:R])
@@ -502,18 +579,22 @@ class UpdateEngine:
             ops.ppo_head(args, ba.h[-1][:R], la[-1].weight, la[-1].bias, bc.h[-1][:R], lc[-1].weight, lc[-1].bias,
                          ba.dz[-2][:R], bc.dz[-2][:R], self.head_ws, std_grad,
                          alg.device_state, adaptive, alg.desired_kl, self.trace, mean=ba.out[:R],
-                         value=bc.out[:R, 0])
+                         value=bc.out[:R, 0],
+                         ranges=(ba.dz_max[-2], bc.dz_max[-2], ba.dz_max[-1], bc.dz_max[-1]) if self.ranged else None)
             tm.stop("head")
             return
         tm.start("loss")
         ops.ppo_loss(args, self.loss_ws)
         ops.ppo_loss_finalize(args, self.loss_ws, std_grad, alg.device_state, adaptive,
                               alg.desired_kl if alg.desired_kl is not None else 0.0, self.trace)
+        if self.ranged:
+            ops.amax([(ba.dz[-1][:R], ba.dz_max[-1]), (bc.dz[-1][:R], bc.dz_max[-1])])
         tm.stop("loss")
 
-    def dx_layers(self, R: int) -> list[tuple[int, list[tuple], bool, int]]:
+    def dx_layers(self, R: int) -> list[tuple]:
         """The head's input-gradients, top layer first: (layer, grouped actor / critic problems, act' taken from the
-        layer below's output, the activation).  Layer 0 has none (no gradient into the observations)."""
+        layer below's output, the activation, the problems' ranges).  Layer 0 has none (no gradient into the
+        observations)."""
         la, lc = self._layers()
         ba, bc = self.buf_a, self.buf_c
         top = len(la) - 2 if self.fused_head else len(la) - 1  # the fused head produced the output layer's
@@ -521,19 +602,20 @@ class UpdateEngine:
         for i in range(top, 0, -1):
             pa = (ba.dz[i][:R], la[i].weight, ba.act_src(i - 1, R), ba.dz[i - 1][:R])
             pc = (bc.dz[i][:R], lc[i].weight, bc.act_src(i - 1, R), bc.dz[i - 1][:R])
+            ra, rc = ((b.dz_max[i], w[i], b.dz_max[i - 1]) for b, w in zip((ba, bc), self.w_max))
             if (ba.act, ba.from_output) == (bc.act, bc.from_output):
-                out.append((i, [pa, pc], ba.from_output, ba.act))
+                out.append((i, [pa, pc], ba.from_output, ba.act, [ra, rc]))
             else:
-                out += [(i, [pa], ba.from_output, ba.act), (i, [pc], bc.from_output, bc.act)]
+                out += [(i, [pa], ba.from_output, ba.act, [ra]), (i, [pc], bc.from_output, bc.act, [rc])]
         return out
 
     def head_backward(self, R: int) -> None:
         """Input gradients down the chain (actor and critic grouped)."""
         tm = self.timer
-        for i, probs, from_output, act in self.dx_layers(R):
+        for i, probs, from_output, act, rng in self.dx_layers(R):
             tm.start(f"dx{i}")
             ops.linear_bwd_dx(probs, R, self.dx_ws, elu_from_output=from_output, act=act,
-                              bf16=self.alg.use_mixed_precision)
+                              bf16=self.alg.use_mixed_precision, ranges=rng if self.ranged else None)
             tm.stop(f"dx{i}")
 
     def head_dw(self, xa: torch.Tensor, xc: torch.Tensor, R: int) -> list[tuple]:
@@ -547,19 +629,21 @@ class UpdateEngine:
         return dw
 
     def weight_grads(self, dw: list[tuple], R: int, phase: str = "dw", ws: ops.Workspace | None = None,
-                     norm: ops.GradNorm | None = None) -> None:
+                     norm: ops.GradNorm | None = None, ranges: list[tuple] | None = None) -> None:
         """Weight gradients, as few grouped launches as the problem limit allows (with `norm`: one launch that also
-        sums the squares for the clip norms)."""
+        sums the squares for the clip norms).  ranges: the problems' operand ranges."""
         tm = self.timer
         tm.start(phase)
         bf16 = self.alg.use_mixed_precision
         if norm is not None:
             if len(dw) > L.MAX_LINEAR_PROBLEMS:
                 raise RuntimeError("weight_grads: the norm partials need all problems in one launch")
-            ops.linear_bwd_dw(dw, R, ws if ws is not None else self.dw_ws, norm=norm, bf16=bf16)
+            ops.linear_bwd_dw(dw, R, ws if ws is not None else self.dw_ws, norm=norm, bf16=bf16, ranges=ranges)
         else:
             for i in range(0, len(dw), L.MAX_LINEAR_PROBLEMS):
-                ops.linear_bwd_dw(dw[i:i + L.MAX_LINEAR_PROBLEMS], R, ws if ws is not None else self.dw_ws, bf16=bf16)
+                part = slice(i, i + L.MAX_LINEAR_PROBLEMS)
+                ops.linear_bwd_dw(dw[part], R, ws if ws is not None else self.dw_ws, bf16=bf16,
+                                  ranges=None if ranges is None else ranges[part])
         tm.stop(phase)
 
     def _bias_corrections(self, step: int) -> tuple[float, float]:
@@ -729,6 +813,7 @@ class RecurrentUpdateEngine(UpdateEngine):
         self.order = torch.cat(order).to(self.device)
 
     recurrent = True
+    ranged = False
 
     def _recurrent_norm_plan(self) -> dict | None:
         """The clip norms from the weight-grad launch and the gradient unpack (one optimiser launch), when that one
@@ -802,7 +887,8 @@ class RecurrentUpdateEngine(UpdateEngine):
         la, lc = self._layers()
         return super().dx_layers(R) + [(0, [(self.buf_a.dz[0][:R], la[0].weight, None, self.seq_a.dh[:R]),
                                             (self.buf_c.dz[0][:R], lc[0].weight, None, self.seq_c.dh[:R])], False,
-                                        L.PPO_ACT_ELU)]
+                                        L.PPO_ACT_ELU, [(b.dz_max[0], w[0], None)
+                                                        for b, w in zip((self.buf_a, self.buf_c), self.w_max)])]
 
     @property
     def can_fail(self) -> bool:

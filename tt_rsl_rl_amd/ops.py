@@ -345,11 +345,50 @@ def _check_weight(w: torch.Tensor, b: torch.Tensor | None) -> tuple[int, int]:
     return out_f, in_f
 
 
+def new_amax(count: int, device) -> torch.Tensor:
+    """Largest-magnitude slots of `count` tensors (rows of AMAX_WORDS words), zero."""
+    return torch.zeros(count, L.AMAX_WORDS, dtype=torch.int32, device=device)
+
+
+def amax(items: list[tuple], clear: torch.Tensor | None = None) -> None:
+    """items: (x [rows, cols] row-major view, slots[, least]): the slots' maximum becomes max |x| (or `least`, if that is
+    larger); `clear` (slots of other tensors, contiguous) is zeroed by the same launch."""
+    arr = []
+    for x, slots, *least in items:
+        _dev(x)
+        arr.append(L.AmaxItem(x.data_ptr(), _row_major(x, "x"), x.shape[0], x.shape[1], float(*least), _slots(slots)))
+    n = 0
+    if clear is not None:
+        _dev(clear, dtype=torch.int32)
+        if not clear.is_contiguous():
+            raise ValueError("amax: the slots to clear must be contiguous")
+        n = clear.numel()
+    L.call("ppo_amax", L.array(L.AmaxItem, arr), len(arr), _ptr(clear), n, _stream())
+
+
+def _slots(t: torch.Tensor | None) -> int | None:
+    if t is None:
+        return None
+    if t.dtype != torch.int32 or t.numel() != L.AMAX_WORDS or not t.is_contiguous() or not t.is_cuda:
+        raise ValueError("ranges: AMAX_WORDS contiguous int32 words on the GPU per tensor")
+    return t.data_ptr()
+
+
+def _ranges(ranges: list[tuple] | None, count: int):
+    """(a, b, out) slots per problem as the C array, or None."""
+    if ranges is None:
+        return None
+    if len(ranges) != count:
+        raise ValueError("ranges: one (a, b, out) per problem")
+    return L.array(L.GemmRange, [L.GemmRange(*(_slots(t) for t in r)) for r in ranges])
+
+
 def linear_fwd(problems: list[tuple], rows: int, elu: bool = False, act: int | None = None,
-               bf16: bool = False) -> None:
+               bf16: bool = False, ranges: list[tuple] | None = None) -> None:
     """problems: (x [rows, in], w [out, in], b [out], z [rows, out] or None, h [rows, out] or None).
     act: the hidden-layer activation (an L.ACTIVATIONS code; elu=True is L.PPO_ACT_ELU), h = act(z); without one z is
-    required, with one at least one of z / h.  bf16: bf16 operands (ppo_linear_fwd_ex, PPO_GEMM_BF16_OPERANDS)."""
+    required, with one at least one of z / h.  bf16: bf16 operands (ppo_linear_fwd_ex, PPO_GEMM_BF16_OPERANDS).
+    ranges: per problem the largest-magnitude slots of (x, w, output or None) (ppo_linear_fwd_ranged)."""
     act = (L.PPO_ACT_ELU if elu else L.PPO_ACT_NONE) if act is None else int(act)
     elu = act != L.PPO_ACT_NONE
     items = []
@@ -372,7 +411,10 @@ def linear_fwd(problems: list[tuple], rows: int, elu: bool = False, act: int | N
                 raise ValueError("linear_fwd: h too small")
         items.append(L.LinearFwdProblem(x.data_ptr(), ldx, w.data_ptr(), b.data_ptr(), _ptr(z), ldz,
                                         _ptr(h) if elu else None, ldh, in_f, out_f))
-    if bf16:
+    if ranges is not None:
+        L.call("ppo_linear_fwd_ranged", L.array(L.LinearFwdProblem, items), _ranges(ranges, len(items)), len(items), rows,
+               act, L.GEMM_BF16_OPERANDS if bf16 else 0, _stream())
+    elif bf16:
         L.call("ppo_linear_fwd_ex", L.array(L.LinearFwdProblem, items), len(items), rows, act, L.GEMM_BF16_OPERANDS,
                _stream())
     else:
@@ -400,14 +442,18 @@ def _dx_problems(problems: list[tuple], rows: int):
 
 
 def linear_bwd_dx(problems: list[tuple], rows: int, ws: Workspace | None = None, elu_from_output: bool = False,
-                  act: int = L.PPO_ACT_ELU, bf16: bool = False) -> None:
+                  act: int = L.PPO_ACT_ELU, bf16: bool = False, ranges: list[tuple] | None = None) -> None:
     """problems: (dz [rows, out], w [out, in], src [rows, in] or None, dz_prev [rows, in]); src is the activation's
     input z of the layer below, or its output h = act(z) with elu_from_output (monotone activations only).  bf16:
-    bf16 operands (ppo_linear_bwd_dx_ex, PPO_GEMM_BF16_OPERANDS)."""
+    bf16 operands (ppo_linear_bwd_dx_ex, PPO_GEMM_BF16_OPERANDS).  ranges: per problem the largest-magnitude slots of
+    (dz, w, dz_prev or None) (ppo_linear_bwd_dx_ranged)."""
     arr, count, nbytes = _dx_problems(problems, rows)
     buf = (ws or Workspace(problems[0][0].device)).get(nbytes)
     src = L.PPO_ELU_FROM_OUTPUT if elu_from_output else L.PPO_ELU_FROM_INPUT
-    if bf16:
+    if ranges is not None:
+        L.call("ppo_linear_bwd_dx_ranged", arr, _ranges(ranges, count), count, rows, int(act), src,
+               L.GEMM_BF16_OPERANDS if bf16 else 0, buf.data_ptr(), buf.numel(), _stream())
+    elif bf16:
         L.call("ppo_linear_bwd_dx_ex", arr, count, rows, int(act), src, L.GEMM_BF16_OPERANDS, buf.data_ptr(),
                buf.numel(), _stream())
     else:
@@ -431,10 +477,11 @@ def grad_norm_partials(device) -> torch.Tensor:
 
 
 def linear_bwd_dw(problems: list[tuple], rows: int, ws: Workspace | None = None, norm: GradNorm | None = None,
-                  bf16: bool = False) -> None:
+                  bf16: bool = False, ranges: list[tuple] | None = None) -> None:
     """problems: (dz [rows, out], x [rows, in], dw [out, in], db [out] or None for no bias gradient).  With `norm`
     the launch also writes the per-group sums of squares of what it stores (ppo_linear_bwd_dw_norm).  bf16: bf16
-    operands (ppo_linear_bwd_dw_ex, PPO_GEMM_BF16_OPERANDS)."""
+    operands (ppo_linear_bwd_dw_ex, PPO_GEMM_BF16_OPERANDS).  ranges: per problem the largest-magnitude slots of
+    (dz, x, None) (ppo_linear_bwd_dw_ranged)."""
     items = []
     for i, (dz, x, dw, db) in enumerate(problems):
         _dev(dz, x, dw, db)
@@ -452,8 +499,13 @@ def linear_bwd_dw(problems: list[tuple], rows: int, ws: Workspace | None = None,
     if nbytes == 0:
         raise ValueError("linear_bwd_dw: invalid problem set")
     buf = (ws or Workspace(problems[0][0].device)).get(nbytes)
+    flags = L.GEMM_BF16_OPERANDS if bf16 else 0
+    rng = _ranges(ranges, len(items))
     if norm is None:
-        if bf16:
+        if rng is not None:
+            L.call("ppo_linear_bwd_dw_ranged", arr, rng, len(items), rows, flags, buf.data_ptr(), buf.numel(), None,
+                   None, 0, None, _stream())
+        elif bf16:
             L.call("ppo_linear_bwd_dw_ex", arr, len(items), rows, L.GEMM_BF16_OPERANDS, buf.data_ptr(), buf.numel(),
                    None, None, 0, None, _stream())
         else:
@@ -468,7 +520,11 @@ def linear_bwd_dw(problems: list[tuple], rows: int, ws: Workspace | None = None,
         _dev(norm.extra_grads)
         if any(r.begin < 0 or r.end > norm.extra_grads.numel() for r in extra):
             raise ValueError("linear_bwd_dw: extra gradient range outside its buffer")
-    if bf16:
+    if rng is not None:
+        L.call("ppo_linear_bwd_dw_ranged", arr, rng, len(items), rows, flags, buf.data_ptr(), buf.numel(),
+               _ptr(norm.extra_grads) if extra else None, L.array(L.GradRange, extra) if extra else None, len(extra),
+               p.data_ptr(), _stream())
+    elif bf16:
         L.call("ppo_linear_bwd_dw_ex", arr, len(items), rows, L.GEMM_BF16_OPERANDS, buf.data_ptr(), buf.numel(),
                _ptr(norm.extra_grads) if extra else None, L.array(L.GradRange, extra) if extra else None, len(extra),
                p.data_ptr(), _stream())
@@ -604,9 +660,11 @@ def ppo_head(args: L.LossArgs, h_actor: torch.Tensor, w_actor: torch.Tensor, b_a
              h_critic: torch.Tensor, w_critic: torch.Tensor, b_critic: torch.Tensor, dz_actor: torch.Tensor,
              dz_critic: torch.Tensor, ws: torch.Tensor, d_std_param: torch.Tensor, state: torch.Tensor,
              adaptive: bool, desired_kl: float | None, trace: torch.Tensor | None,
-             mean: torch.Tensor | None = None, value: torch.Tensor | None = None) -> None:
+             mean: torch.Tensor | None = None, value: torch.Tensor | None = None,
+             ranges: tuple | None = None) -> None:
     """Output layers + loss + finalize + the output layers' input-grad in one call (ppo_gauss_ppo_head).  args
-    carries the batch columns and d_mean / d_value; its mean / value fields are not read."""
+    carries the batch columns and d_mean / d_value; its mean / value fields are not read.  ranges: the
+    largest-magnitude slots of (dz_actor, dz_critic, d_mean, d_value) to raise (ppo_gauss_ppo_head_ranged)."""
     _dev(h_actor, w_actor, b_actor, h_critic, w_critic, b_critic, dz_actor, dz_critic, mean, value)
     R = int(args.rows)
     for name, t in (("h_actor", h_actor), ("h_critic", h_critic), ("dz_actor", dz_actor), ("dz_critic", dz_critic)):
@@ -629,6 +687,11 @@ def ppo_head(args: L.LossArgs, h_actor: torch.Tensor, w_actor: torch.Tensor, b_a
         dz_critic=dz_critic.data_ptr(), ld_dz_critic=_row_major(dz_critic, "dz_critic"),
         mean=_ptr(mean), ld_mean=_row_major(mean, "mean") if mean is not None else 0,
         value=_ptr(value), ld_value=value.stride(0) if value is not None else 0, k_actor=ka, k_critic=kc)
+    if ranges is not None:
+        L.call("ppo_gauss_ppo_head_ranged", C_ref(args), C_ref(head), C_ref(L.HeadRanges(*(_slots(t) for t in ranges))),
+               ws.data_ptr(), ws.numel(), d_std_param.data_ptr(), state.data_ptr(), 1 if adaptive else 0,
+               float(desired_kl if desired_kl is not None else 0.0), _ptr(trace), _trace_rows(trace), _stream())
+        return
     L.call("ppo_gauss_ppo_head", C_ref(args), C_ref(head), ws.data_ptr(), ws.numel(), d_std_param.data_ptr(),
            state.data_ptr(), 1 if adaptive else 0, float(desired_kl if desired_kl is not None else 0.0), _ptr(trace),
            _trace_rows(trace), _stream())

@@ -301,6 +301,36 @@ int ppo_normalizer_update(const ppo_column_block* blocks, int32_t num_blocks, in
                           size_t workspace_bytes, ppo_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------------------------------
+ * A whole MLP forward in one launch (rollout side; rsl_rl/models/mlp_model.py:82-118): the input blocks side by side
+ * ([rows, width] each), normalised where norm_mean / norm_std are given ((x - mean) / (std + eps) over the concatenated
+ * columns), then the layers, each but the last followed by the activation; out [rows, last out_features].  Inputs of at
+ * most 1,024 features per layer (PPO_EUNSUPPORTED otherwise).  A block of threads carries 16 rows through all layers, so
+ * it is meant for up to some thousands of rows; larger batches are faster as ppo_linear_fwd per layer.
+ * ------------------------------------------------------------------------------------------------------------------ */
+#define PPO_MAX_MLP_PROBLEMS 2
+#define PPO_MAX_MLP_LAYERS 8
+#define PPO_MAX_MLP_BLOCKS 8
+typedef struct ppo_mlp_layer {
+  const float* w; /* [out, in] */
+  const float* b; /* [out] */
+  int32_t in_features;
+  int32_t out_features;
+} ppo_mlp_layer;
+typedef struct ppo_mlp_problem {
+  ppo_column_block x[PPO_MAX_MLP_BLOCKS];
+  ppo_mlp_layer layers[PPO_MAX_MLP_LAYERS];
+  const float* norm_mean; /* [input width] or NULL */
+  const float* norm_std;
+  float* out;
+  int64_t ldo;
+  float norm_eps;
+  int32_t num_blocks;
+  int32_t num_layers;
+  int32_t activation; /* PPO_ACT_*, of the hidden layers */
+} ppo_mlp_problem;
+int ppo_mlp_fwd(const ppo_mlp_problem* problems, int32_t count, int64_t rows, ppo_stream_t stream);
+
+/* ------------------------------------------------------------------------------------------------------------------
  * A8-A11  Gaussian policy head + PPO losses, forward and backward, rsl_rl/algorithms/ppo.py:226-285 with
  * rsl_rl/modules/distribution.py:183-238 (state-independent std).  Per row r of a mini-batch of R rows:
  *   std = clamp(std_param) (scalar) or exp(clamp(log_std_param)) (log);

@@ -241,6 +241,12 @@ class _ForwardBuffers:
         return [b[:rows] for b in self.bufs]
 
 
+# Up to this many rows a model's forward is one launch (ppo_mlp_fwd), above it one GEMM launch per layer: 256 blocks of 16
+# rows, one per compute unit.  48 -> [512, 256, 128] -> 12, one launch / layer by layer: 16 rows 34 / 64 us, 4,096 rows
+# 37 / 63, 8,192 rows 59 / 62, 16,384 rows 112 / 74.
+FUSED_ROWS = 4096
+
+
 class MLPModel(nn.Module):
     """rsl_rl/models/mlp_model.py:19-193 (same signature; registration order normalizer, distribution, mlp)."""
 
@@ -273,6 +279,7 @@ class MLPModel(nn.Module):
         self.mlp = nn.Sequential(*layers)
         self.output_dim = mlp_out
         self._fwd = _ForwardBuffers()
+        self._fused: tuple | None = None  # (addresses the record was built from, the ppo_mlp_fwd record)
 
     # -- structure ---------------------------------------------------------------------------------------------------
     def _get_obs_dim(self, obs: Mapping, obs_groups: dict, obs_set: str) -> tuple[list[str], int]:
@@ -310,7 +317,62 @@ class MLPModel(nn.Module):
                 dst.copy_(x)
             col += w
 
+    def _mlp_record(self, norm) -> "L.MlpProblem | None":
+        """The layers (and the normaliser) as ppo_mlp_fwd takes them; rebuilt when a parameter lives elsewhere.  None:
+        outside what it takes."""
+        layers = [m for m in self.mlp if isinstance(m, nn.Linear)]
+        tensors = [t for l in layers for t in (l.weight, l.bias)]
+        if norm is not None:
+            tensors += [norm._mean, norm._std]
+        key = tuple(t.data_ptr() for t in tensors)
+        if self._fused is not None and self._fused[0] == key:
+            return self._fused[1]
+        rec = None
+        if (len(layers) <= L.MAX_MLP_LAYERS and all(l.in_features <= L.MLP_MAX_WIDTH for l in layers) and
+                all(t.dtype == torch.float32 and t.is_contiguous() and t.is_cuda for t in tensors)):
+            rec = L.MlpProblem(num_layers=len(layers), activation=self.act_code)
+            for i, l in enumerate(layers):
+                rec.layers[i] = L.MlpLayer(l.weight.data_ptr(), l.bias.data_ptr(), l.in_features, l.out_features)
+            if norm is not None:
+                rec.norm_mean, rec.norm_std, rec.norm_eps = norm._mean.data_ptr(), norm._std.data_ptr(), norm.eps
+        self._fused = (key, rec)
+        return rec
+
+    def _fused_forward(self, columns: list[torch.Tensor], norm) -> torch.Tensor | None:
+        """The whole forward on the concatenation of `columns` ([rows, width] each) in one launch; None where the
+        layers run one by one."""
+        rows = columns[0].shape[0]
+        if rows > FUSED_ROWS or rows == 0 or len(columns) > L.MAX_MLP_BLOCKS:
+            return None
+        rec = self._mlp_record(norm)
+        if rec is None:
+            return None
+        width = 0
+        for i, x in enumerate(columns):
+            if x.dtype != torch.float32 or x.shape[0] != rows or not x.is_cuda:
+                return None
+            if x.stride(1) != 1 or (rows > 1 and x.stride(0) < x.shape[1]):
+                x = columns[i] = x.contiguous()
+            b = rec.x[i]
+            b.src, b.stride, b.width = x.data_ptr(), max(x.stride(0), x.shape[1]), x.shape[1]
+            width += x.shape[1]
+        if width != rec.layers[0].in_features:
+            return None
+        rec.num_blocks = len(columns)
+        out = torch.empty(rows, rec.layers[rec.num_layers - 1].out_features, device=columns[0].device)
+        rec.out, rec.ldo = out.data_ptr(), out.stride(0)
+        L.call("ppo_mlp_fwd", ops.C_ref(rec), 1, rows, torch.cuda.current_stream().cuda_stream)
+        return out
+
     def mlp_forward(self, latent: torch.Tensor) -> torch.Tensor:
+        out = self._fused_forward([latent], None)
+        return self._mlp_layers(latent) if out is None else out
+
+    def forward_layers(self, obs: Mapping) -> torch.Tensor:
+        """The deterministic forward with one GEMM launch per layer at every size."""
+        return self._mlp_layers(self.get_latent(obs))
+
+    def _mlp_layers(self, latent: torch.Tensor) -> torch.Tensor:
         rows = latent.shape[0]
         lin = self.linears
         widths = [l.out_features for l in lin[:-1]]
@@ -333,7 +395,13 @@ class MLPModel(nn.Module):
     def forward(self, obs: Mapping, masks=None, hidden_state=None, stochastic_output: bool = False) -> torch.Tensor:
         if masks is not None:
             raise NotImplementedError("padded (recurrent) batches are not supported by the MLP HIP path")
-        out = self.mlp_forward(self.get_latent(obs))
+        out = None
+        if type(self).get_latent is MLPModel.get_latent and type(self).latent_into is MLPModel.latent_into:
+            cols = [obs[g] for g in self.obs_groups]
+            if all(x.is_cuda and x.dim() == 2 for x in cols):
+                out = self._fused_forward(cols, self.obs_normalizer if self.obs_normalization else None)
+        if out is None:
+            out = self.mlp_forward(self.get_latent(obs))
         if self.distribution is not None:
             if stochastic_output:
                 self.distribution.update(out)

@@ -265,7 +265,10 @@ class PPO:
     def compute_returns(self, obs: Mapping) -> None:
         """ppo.py:166-191: bootstrap value, GAE scan and global advantage normalisation on the GPU."""
         critic_hidden_state = self.critic.get_hidden_state()
-        last_values = self.critic(obs).detach().contiguous()
+        # layer by layer at every size: the bootstrap value enters every advantage, and its rounding (another one in the
+        # one-launch forward that act() uses) is carried through all of the update's steps (see RANGED_ROWS in engine.py)
+        plain = type(self.critic).forward in (MLPModel.forward, RNNModel.forward)
+        last_values = (self.critic.forward_layers(obs) if plain else self.critic(obs)).detach().contiguous()
         # the bootstrap forward must not advance the critic's rollout state (ppo.py:170-173)
         self.critic.reset(hidden_state=critic_hidden_state)
         self.compute_returns_from(last_values)

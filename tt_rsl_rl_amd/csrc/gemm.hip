@@ -305,7 +305,7 @@ int launch_nt_pipe(Group& g, int count, hipStream_t s, const char* name) {
 // row and 11.4 with 128 x 64 tiles.  A PPO_HIP_TUNING build reads "PPO_HIP_BX6" = "bn[:stages[:four_lanes]]"
 // (0: off).
 template <int EPI, bool BKM = false>
-int launch_nt_bx6(Group& g, int count, hipStream_t s, const char* name, bool bf16 = false) {
+int launch_nt_bx6(Group& g, int count, hipStream_t s, const char* name) {
   auto fits = [](const float* c, int64_t rows, int64_t ld) {
     return c == nullptr || (w16_ok(c, ld) && rows * ld * 4 < (int64_t(1) << 31));
   };
@@ -348,11 +348,6 @@ int launch_nt_bx6(Group& g, int count, hipStream_t s, const char* name, bool bf1
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, s, g);
     return check_launch(name);
   };
-  if (bf16) {  // the bf16-operand mode: one product per k-group, the default tiles
-    if constexpr (BKM) return go(gemm_nt_bx6_kernel<128, 3, EPI, 2, true, true, true>);
-    if (bn == 64) return go(gemm_nt_bx6_kernel<64, 3, EPI, 2, true, false, true>);
-    return go(gemm_nt_bx6_kernel<128, 3, EPI, 2, true, false, true>);
-  }
   if constexpr (BKM) return go(gemm_nt_bx6_kernel<128, 3, EPI, 2, true, true>);
 #ifdef PPO_HIP_TUNING
   if (bn == 64 || ns == 3 || !q4) {
@@ -398,12 +393,19 @@ int launch_nt_f16(Group& g, int count, hipStream_t s, const char* name) {
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, s, g);
     return check_launch(name);
   };
+  // one product per k-group: registers for three blocks of 128 x 128 per CU (humanoid: 6.69 ms per update; eight waves
+  // of 32 x 64 at four per SIMD 6.9, the bf16x6 kernels' staging with one product, used before, 7.16)
+  if constexpr (AR == ARITH_BF16) {
+    if (bn == 64) return go(gemm_nt_f16_kernel<64, 2, 4, EPI, BKM, AR>, 256);
+    return go(gemm_nt_f16_kernel<128, 2, 3, EPI, BKM, AR>, 256);
+  } else {
   if (bn == 64) return go(gemm_nt_f16_kernel<64, 2, 3, EPI, BKM, AR>, 256);
   // 128 x 128: eight waves of 32 x 64 (128 registers, four waves per SIMD) for the forward, whose epilogue's activation
   // then overlaps other waves' products (512 -> 256 features: 56 us against 63 with four waves of 64 x 64, 240 -> 512:
   // 66 against 73); the input-grad's longer staging and epilogue do not fit 128 registers (74 against 69 us)
   if constexpr (BKM) return go(gemm_nt_f16_kernel<128, 2, 2, EPI, BKM, AR>, 256);
   else return go(gemm_nt_f16_kernel<128, 4, 4, EPI, BKM, AR>, 512);
+  }
 }
 
 // The 128 x 128 (128 x 64 for problems at most 64 columns wide) split-K weight-grad tiles of gemm_f16.hpp; the caller
@@ -630,9 +632,13 @@ extern "C" int ppo_linear_fwd_ranged(const ppo_linear_fwd_problem* problems, con
   bool tracked = false;  // the kernel raised the outputs' slots
   auto plain = [&](auto epi_c, const char* name) {
     constexpr int EPI = decltype(epi_c)::value;
-    const int brc = launch_nt_bx6<EPI>(g, count, s, name, bf16);
+    if (bf16) {
+      const int hrc = launch_nt_f16<EPI, false, ARITH_BF16>(g, count, s, name);
+      if (hrc != PPO_EUNSUPPORTED) return hrc;
+    }
+    const int brc = launch_nt_bx6<EPI>(g, count, s, name);
     if (brc != PPO_EUNSUPPORTED) {
-      tracked = elu && !bf16;
+      tracked = elu;
       return brc;
     }
     const int prc = launch_nt_pipe_tile<EPI>(pipe_tile("PPO_HIP_PIPE_FWD", max_n > 128 ? 1 : 2), g, count, s, name);
@@ -754,7 +760,8 @@ int dx_gemm(const ppo_linear_bwd_dx_problem* problems, int32_t count, int64_t ro
   auto plain = [&](auto epi_c, const char* name) {
     constexpr int EPI = decltype(epi_c)::value;
     // the bf16x6 kernel reads the weights as stored (k-major, 16-byte rows): no transpose
-    const int krc = launch_nt_bx6<EPI, true>(g, count, s, name, bf16);
+    const int krc = bf16 ? launch_nt_f16<EPI, true, ARITH_BF16>(g, count, s, name)
+                         : launch_nt_bx6<EPI, true>(g, count, s, name);
     if (krc != PPO_EUNSUPPORTED) return krc;
     // else w^T (k-contiguous) into the workspace for the other kernels
     if (int rc = launch_transposes(problems, count, ws, offs, s)) return rc;
@@ -762,7 +769,8 @@ int dx_gemm(const ppo_linear_bwd_dx_problem* problems, int32_t count, int64_t ro
       g.p[i].B = ws + offs[i];
       g.p[i].ldb = round4(problems[i].out_features);
     }
-    const int brc = launch_nt_bx6<EPI>(g, count, s, name, bf16);
+    const int brc = bf16 ? launch_nt_f16<EPI, false, ARITH_BF16>(g, count, s, name)
+                         : launch_nt_bx6<EPI>(g, count, s, name);
     if (brc != PPO_EUNSUPPORTED) return brc;
     // measured on MI355X: 64x64 tiles for the 256..512-wide input grads, 128x64 for narrower ones
     const int prc = launch_nt_pipe_tile<EPI>(pipe_tile("PPO_HIP_PIPE_DX", max_n > 128 ? 3 : 2), g, count, s, name);
@@ -880,9 +888,13 @@ int dw_gemm(const ppo_linear_bwd_dw_problem* problems, int32_t count, int64_t ro
     bx6 = bx6 && w16_ok(problems[i].dz, problems[i].lddz) && w16_ok(problems[i].x, problems[i].ldx);
   // with every range known, fp16x3 (its k, the rows, from kF16MinK; the kernel needs one whole slab of 32)
   bool f16 = bx6 && !bf16 && ranges != nullptr && rows >= kF16MinK;
-  for (int i = 0; i < count && f16; ++i)
-    f16 = ranges[i].a != nullptr && ranges[i].b != nullptr &&
-          32 * std::max(problems[i].lddz, problems[i].ldx) * 4 < (int64_t(1) << 31);
+  int64_t max_ld = 0;
+  for (int i = 0; i < count; ++i) {
+    max_ld = std::max(max_ld, std::max(problems[i].lddz, problems[i].ldx));
+    f16 = f16 && ranges[i].a != nullptr && ranges[i].b != nullptr;
+  }
+  f16 = f16 && 32 * max_ld * 4 < (int64_t(1) << 31);
+  const bool b16 = bx6 && bf16 && 32 * max_ld * 4 < (int64_t(1) << 31);
   int occ = f16 ? kDwF16BlocksPerCu : bx6 ? kDwBlocksPerCu : kDwF32BlocksPerCu;
 #ifdef PPO_HIP_TUNING
   const char* cfg = std::getenv("PPO_HIP_DW_CFG");  // tuning aid: other slab depths / stages / occupancies
@@ -947,8 +959,10 @@ int dw_gemm(const ppo_linear_bwd_dw_problem* problems, int32_t count, int64_t ro
 #endif
   if (f16) {
     rc = launch_tn_f16<kDwF16BlocksPerCu, ARITH_F16X3>(g, count, s, "linear_bwd_dw");
+  } else if (b16) {
+    rc = launch_tn_f16<kDwBlocksPerCu, ARITH_BF16>(g, count, s, "linear_bwd_dw");
   } else if (bx6) {
-    rc = launch_tn_bx6<kDwBlocksPerCu>(g, count, s, "linear_bwd_dw", bf16);
+    rc = launch_tn_bx6<kDwBlocksPerCu>(g, count, s, "linear_bwd_dw");
   } else {
     rc = launch_tn<kDwBM, kDwBN, 32, 2, kDwF32BlocksPerCu>(g, count, s, "linear_bwd_dw");
   }

@@ -304,7 +304,7 @@ __global__ __launch_bounds__(WM * 128) __attribute__((amdgpu_waves_per_eu(OCC, O
 // TN (weight-grad): C[m,n] = sum_k A[k,m] B[k,n] over one split's rows, 128 x BN tiles, 32-row k-slabs in two LDS
 // stages of k-major planes, fragments by the transposing LDS read (layouts as in gemm_core.hpp's tn_bx6_tile).  The
 // last slab of a matrix whose rows are not whole slabs is shifted back to end at the matrix's end, its rows before the
-// slab's own start zeroed (the launcher takes matrices of at least 32 rows).
+// slab's own start zeroed (and a matrix of fewer than 32 rows re-reads its last row, zeroed).
 // ------------------------------------------------------------------------------------------------------------------
 template <int BN, int WM, int AR>
 __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, unsigned char* lds) {
@@ -328,17 +328,17 @@ __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, 
   int la[NA], lb[NB];
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
-    aoff[i] = static_cast<uint32_t>(((sk + KPPA * i) * lda + mc_a) * 4);
+    aoff[i] = static_cast<uint32_t>((min(sk + KPPA * i, K - 1) * lda + mc_a) * 4);
     la[i] = tn_chunk_off<BM>(sk + KPPA * i, sc);
   }
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
-    boff[i] = static_cast<uint32_t>(((bsk + KPPB * i) * ldb + mc_b) * 4);
+    boff[i] = static_cast<uint32_t>((min(bsk + KPPB * i, K - 1) * ldb + mc_b) * 4);
     lb[i] = tn_chunk_off<BN>(bsk + KPPB * i, bsc);
   }
   f32x4 va[NA], vb[NB];
   auto load_piece = [&](int kt, int o) __attribute__((always_inline)) {
-    const int64_t k0 = min(k_begin + kt * BK, K - BK);
+    const int64_t k0 = max(min(k_begin + kt * BK, K - BK), 0);
     if (o < NA) {
       va[o < NA ? o : 0] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const unsigned char*>(P.A + k0 * lda) +
                                                            aoff[o < NA ? o : 0]);
@@ -349,7 +349,7 @@ __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, 
   };
   // rows outside [k_begin + 32 kt, k_end): those that a shifted slab repeats, and those past a chunk's end
   auto mask_tail = [&](int kt) __attribute__((always_inline)) {
-    const int own = k_begin + kt * BK, k0 = min(own, K - BK);
+    const int own = k_begin + kt * BK, k0 = max(min(own, K - BK), 0);
     if (own == k0 && own + BK <= k_end) return;
 #pragma unroll
     for (int i = 0; i < NA; ++i) {

@@ -473,6 +473,32 @@ int ppo_gauss_sample(const float* mean, int64_t ld_mean, const float* std_param,
                      ppo_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------------------------------
+ * The rollout storage's writes of one transition (rsl_rl/storage/rollout_storage.py:173-205) in one launch.  Item i
+ * writes a [rows, width] block: F32 copies floats; U8 converts float, byte (also bool) or int64 flags to uint8 as torch
+ * does; BOOTSTRAP (width 1) writes src + gamma * (value * flag), the reward with its time-out bootstrap
+ * (rsl_rl/algorithms/ppo.py:150-155; value and flag: one per row, without gaps), op by op in fp32.  `type`: that of
+ * src (U8) or flag (BOOTSTRAP).  Strides in elements.  Blocks must not overlap one another (a block equal to its
+ * source is left as it is).
+ * ------------------------------------------------------------------------------------------------------------------ */
+#define PPO_MAX_STORE_ITEMS 16
+enum { PPO_STORE_F32 = 0, PPO_STORE_U8 = 1, PPO_STORE_BOOTSTRAP = 2 };
+enum { PPO_STORE_T_F32 = 0, PPO_STORE_T_U8 = 1, PPO_STORE_T_I64 = 2 };
+typedef struct ppo_store_item {
+  const void* src;
+  int64_t src_stride;
+  void* dst;
+  int64_t dst_stride;
+  int64_t rows;
+  int32_t width;
+  int32_t kind;
+  const float* value;
+  const void* flag;
+  float gamma;
+  int32_t type;
+} ppo_store_item;
+int ppo_store_rows(const ppo_store_item* items, int32_t count, ppo_stream_t stream);
+
+/* ------------------------------------------------------------------------------------------------------------------
  * A12+A13  Per-group gradient-norm clipping (torch.nn.utils.clip_grad_norm_, called per model at ppo.py:309-310)
  * fused with Adam (torch.optim.Adam single-tensor path, ppo.py:311) over ONE flat fp32 buffer per kind.
  * Groups are contiguous ranges [group_begin[g], group_begin[g+1]) of the flat buffers.

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 from pathlib import Path
 
 # PPO_HIP_LIB names another build of the same library (the host-sanitizer build of sanitize_host.py)
@@ -104,6 +105,21 @@ OPTIMIZERS = {"adam": OPTIM_ADAM, "adamw": OPTIM_ADAMW, "sgd": OPTIM_SGD, "rmspr
 
 class ColumnBlock(C.Structure):
     _fields_ = [("src", C.c_void_p), ("stride", i64), ("width", i32), ("reserved", i32)]
+
+
+MAX_STORE_ITEMS = 16
+STORE_F32, STORE_U8, STORE_BOOTSTRAP = 0, 1, 2
+STORE_T_F32, STORE_T_U8, STORE_T_I64 = 0, 1, 2
+
+
+class StoreItem(C.Structure):
+    _fields_ = [("src", C.c_void_p), ("src_stride", i64), ("dst", C.c_void_p), ("dst_stride", i64), ("rows", i64),
+                ("width", i32), ("kind", i32), ("value", C.c_void_p), ("flag", C.c_void_p), ("gamma", C.c_float),
+                ("type", i32)]
+
+
+STORE_ITEM = struct.Struct("@PqPqqiiPPfi")  # one StoreItem, packed by hand (a third of the time of its fields)
+assert STORE_ITEM.size == C.sizeof(StoreItem)
 
 
 class LossArgs(C.Structure):
@@ -244,6 +260,7 @@ _SIGNATURES = [
                                             i32, C.c_void_p]),
     ("ppo_gauss_sample", C.c_int, [f32p, i64, f32p, i32, C.c_double, C.c_double, f32p, i64, f32p, i64, f32p, f32p,
                                    i64, i64, i32, C.c_void_p]),
+    ("ppo_store_rows", C.c_int, [C.c_void_p, i32, C.c_void_p]),
     ("ppo_host_randperm", C.c_int, [C.c_void_p, C.c_size_t, i64, C.c_void_p]),
     ("ppo_host_randperm_range", C.c_int, [C.c_void_p, C.c_size_t, i64, i64, i64, C.c_void_p]),
     ("ppo_host_rng_skip", C.c_int, [C.c_void_p, C.c_size_t, i64]),

@@ -162,6 +162,16 @@ class GaussianDistribution(nn.Module):
         self.sample_from(self._mean, noise, actions, None, None)
         return actions
 
+    def sample_scored(self, mean: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+        """``update(mean)``, ``sample()`` and the log-probability of that sample, in one launch."""
+        self._mean = mean
+        noise = self._host_noise.draw(mean.shape, mean.device) if self.host_noise else torch.randn_like(mean)
+        actions, std = torch.empty_like(mean), torch.empty_like(mean)
+        logp = torch.empty(mean.shape[0], device=mean.device)
+        self.sample_from(mean, noise, actions, logp, std)
+        self._std = std
+        return actions, logp
+
     @property
     def mean(self) -> torch.Tensor:
         return self._mean
@@ -245,6 +255,11 @@ class _ForwardBuffers:
 # rows, one per compute unit.  48 -> [512, 256, 128] -> 12, one launch / layer by layer: 16 rows 34 / 64 us, 4,096 rows
 # 37 / 63, 8,192 rows 59 / 62, 16,384 rows 112 / 74.
 FUSED_ROWS = 4096
+
+
+# attributes of a model or distribution that act() goes through; one set on the instance stands for another behaviour
+_STOCHASTIC = frozenset(("forward", "get_output_log_prob", "update", "sample", "log_prob", "sample_from",
+                         "deterministic_output"))
 
 
 class MLPModel(nn.Module):
@@ -408,6 +423,18 @@ class MLPModel(nn.Module):
                 return self.distribution.sample()
             return self.distribution.deterministic_output(out)
         return out
+
+    def acts_plainly(self) -> bool:
+        """Calling this model runs this class's forward on a Gaussian head and nothing else: no subclass, hook, compiled
+        or replaced forward between (``sample_scored`` then gives what the calls of act() give)."""
+        return (type(self) in (MLPModel, RNNModel) and type(self.distribution) is GaussianDistribution and
+                not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks or self._backward_pre_hooks)
+                and not torch.nn.modules.module._has_any_global_hook() and self._compiled_call_impl is None and
+                _STOCHASTIC.isdisjoint(self.__dict__) and _STOCHASTIC.isdisjoint(self.distribution.__dict__))
+
+    def sample_scored(self, obs: Mapping) -> tuple[torch.Tensor, torch.Tensor]:
+        """The stochastic forward and its output's log-probability: (actions, log_prob)."""
+        return self.distribution.sample_scored(self.forward(obs))
 
     # -- upstream model API ------------------------------------------------------------------------------------------
     def reset(self, dones=None, hidden_state=None) -> None:

@@ -85,6 +85,77 @@ def adv_normalize(x: torch.Tensor, out: torch.Tensor, n: int, in_stride: int = 1
 
 
 # ----------------------------------------------------------------------------------------------------------------------
+# rollout storage
+# ----------------------------------------------------------------------------------------------------------------------
+
+STORE_FLAGS = {torch.float32: L.STORE_T_F32, torch.bool: L.STORE_T_U8, torch.uint8: L.STORE_T_U8,
+               torch.int64: L.STORE_T_I64}
+
+
+def _rows_of(t: torch.Tensor) -> tuple[int, int, int] | None:
+    """(rows, width, row stride in elements) of a block whose rows lie one after another; None for other layouts."""
+    if t.is_contiguous():
+        n = t.numel()
+        return (1, n, n) if n else None
+    if t.dim() == 2 and t.stride(1) == 1 and t.stride(0) >= t.shape[1] and t.numel():
+        return t.shape[0], t.shape[1], t.stride(0)
+    return None
+
+
+class RowStores:
+    """Writes ``dst.copy_(src)`` into device buffers, gathered into one ppo_store_rows launch; a pair it does not take
+    (another device, shape, layout or type, tensor subclasses, gradients) is copied by torch at once.  Nothing else may
+    read the destinations before ``flush()``, and a source must stay as it is until then."""
+
+    def __init__(self, device: torch.device) -> None:
+        self.device = None  # no pair fits
+        if device.type == "cuda":
+            index = torch.cuda.current_device()
+            if device.index in (None, index):
+                self.device = torch.device("cuda", index)
+        self.items: list[bytes] = []
+
+    def copy(self, dst: torch.Tensor, src: torch.Tensor) -> None:
+        kind = L.STORE_F32 if dst.dtype == torch.float32 else L.STORE_U8 if dst.dtype == torch.uint8 else None
+        t = STORE_FLAGS.get(src.dtype, -1) if kind == L.STORE_U8 else L.STORE_T_F32
+        if (kind is None or t < 0 or (kind == L.STORE_F32 and src.dtype != torch.float32) or
+                type(src) is not torch.Tensor or type(dst) is not torch.Tensor or src.shape != dst.shape or
+                src.device != self.device or dst.device != self.device or src.requires_grad or dst.requires_grad or
+                dst.numel() >= 1 << 31):
+            dst.copy_(src)
+            return
+        d, s = _rows_of(dst), _rows_of(src)
+        if d is None or s is None:
+            dst.copy_(src)
+            return
+        if d[0] != s[0]:  # one side without gaps: the other's rows
+            rows, width = max(d[:2], s[:2])
+            d = (rows, width, width) if d[0] == 1 else d
+            s = (rows, width, width) if s[0] == 1 else s
+        self._add(L.STORE_ITEM.pack(src.data_ptr(), s[2], dst.data_ptr(), d[2], d[0], d[1], kind, 0, 0, 0.0, t))
+
+    def bootstrap(self, dst: torch.Tensor, rewards: torch.Tensor, gamma: float, values: torch.Tensor,
+                  flags: torch.Tensor) -> None:
+        """dst[i] = rewards[i] + gamma * (values[i] * flags[i]), N contiguous elements each."""
+        n = rewards.numel()
+        if dst.dtype != torch.float32 or dst.numel() != n or not dst.is_contiguous() or dst.device != self.device:
+            dst.copy_((rewards + gamma * (values.view(-1) * flags)).view(dst.shape))
+            return
+        self._add(L.STORE_ITEM.pack(rewards.data_ptr(), 1, dst.data_ptr(), 1, n, 1, L.STORE_BOOTSTRAP, values.data_ptr(),
+                                    flags.data_ptr(), gamma, STORE_FLAGS[flags.dtype]))
+
+    def _add(self, item: bytes) -> None:
+        self.items.append(item)
+        if len(self.items) == L.MAX_STORE_ITEMS:
+            self.flush()
+
+    def flush(self) -> None:
+        if self.items:
+            L.call("ppo_store_rows", b"".join(self.items), len(self.items), _stream())
+            self.items = []
+
+
+# ----------------------------------------------------------------------------------------------------------------------
 # A5 / A7 forward
 # ----------------------------------------------------------------------------------------------------------------------
 

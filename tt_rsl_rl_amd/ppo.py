@@ -33,7 +33,7 @@ from . import _lib as L
 from . import ops
 from .engine import RecurrentUpdateEngine, UpdateEngine
 from .models import MLPModel, RNNModel
-from .storage import RolloutStorage
+from .storage import Bootstrap, RolloutStorage
 
 
 # ----------------------------------------------------------------------------------------------------------------------
@@ -243,21 +243,34 @@ class PPO:
     def act(self, obs: Mapping) -> torch.Tensor:
         """ppo.py:124-135."""
         self.transition.hidden_states = (self.actor.get_hidden_state(), self.critic.get_hidden_state())
-        self.transition.actions = self.actor(obs, stochastic_output=True).detach()
+        logp = None
+        if self.actor.acts_plainly():
+            self.transition.actions, logp = self.actor.sample_scored(obs)
+        else:
+            self.transition.actions = self.actor(obs, stochastic_output=True).detach()
         self.transition.values = self.critic(obs).detach()
-        self.transition.actions_log_prob = self.actor.get_output_log_prob(self.transition.actions).detach()
+        if logp is None:
+            logp = self.actor.get_output_log_prob(self.transition.actions).detach()
+        self.transition.actions_log_prob = logp
         self.transition.distribution_params = tuple(p.detach() for p in self.actor.output_distribution_params)
         self.transition.observations = obs
         return self.transition.actions
 
     def process_env_step(self, obs: Mapping, rewards: torch.Tensor, dones: torch.Tensor, extras: dict) -> None:
         """ppo.py:137-164 (time-out bootstrap with the pre-step value V(s_t))."""
-        self.transition.rewards = rewards.clone()
-        self.transition.dones = dones
+        tr = self.transition
+        tr.dones = dones
+        boot = None
         if "time_outs" in extras:
-            self.transition.rewards += self.gamma * torch.squeeze(
-                self.transition.values * extras["time_outs"].unsqueeze(1).to(self.device), 1)
-        self.storage.add_transition(self.transition)
+            boot = Bootstrap(self.gamma, tr.values, extras["time_outs"])
+        if boot is not None and type(self.storage).add_transition is RolloutStorage.add_transition and boot.fits(rewards):
+            tr.rewards = rewards  # (read by the launch that writes the transition)
+            self.storage.add_transition(tr, boot)
+        else:
+            tr.rewards = rewards.clone()
+            if boot is not None:
+                tr.rewards += self.gamma * torch.squeeze(tr.values * extras["time_outs"].unsqueeze(1).to(self.device), 1)
+            self.storage.add_transition(tr)
         self.transition.clear()
         self.actor.reset(dones)
         self.critic.reset(dones)

@@ -8,9 +8,29 @@ kernel; ``mini_batch_generator`` is kept for API compatibility (it yields the sa
 
 from __future__ import annotations
 
-from typing import Mapping
+from typing import Mapping, NamedTuple
 
 import torch
+
+from . import ops
+
+
+class Bootstrap(NamedTuple):
+    """The time-out bootstrap of a step's rewards, gamma * value * time_out (rsl_rl/algorithms/ppo.py:150-155)."""
+
+    gamma: float
+    values: torch.Tensor
+    time_outs: torch.Tensor
+
+    def fits(self, rewards: torch.Tensor) -> bool:
+        """The launch that writes the transition evaluates it: [N] rewards and time-outs beside [N, 1] values."""
+        v, t = self.values, self.time_outs
+        return (type(rewards) is type(v) is type(t) is torch.Tensor and rewards.dim() == 1 and rewards.is_contiguous() and
+                rewards.dtype == v.dtype == torch.float32 and v.shape == (rewards.shape[0], 1) and v.is_contiguous() and
+                t.shape == rewards.shape and t.is_contiguous() and t.dtype in ops.STORE_FLAGS and
+                rewards.is_cuda and rewards.device == v.device == t.device == torch.device("cuda", torch.cuda.current_device())
+                and 0 < rewards.shape[0] < 1 << 31 and not rewards.requires_grad and not v.requires_grad and
+                not t.requires_grad and isinstance(self.gamma, (int, float)))
 
 
 class RolloutStorage:
@@ -75,23 +95,29 @@ class RolloutStorage:
         self.saved_hidden_state_c = None
         self.step = 0
 
-    def add_transition(self, transition: "RolloutStorage.Transition") -> None:
-        """rollout_storage.py:173-205 (copies into the device buffers)."""
+    def add_transition(self, transition: "RolloutStorage.Transition", bootstrap: "Bootstrap | None" = None) -> None:
+        """rollout_storage.py:173-205 (copies into the device buffers, in one launch; what it does not take, through
+        torch).  ``bootstrap``: added to the rewards on the way (the caller asked ``fits`` of them)."""
         if self.step >= self.num_transitions_per_env:
             raise OverflowError("Rollout buffer overflow! You should call clear() before adding new transitions.")
         s = self.step
         if self.distribution_params is None:
             self._interleave(transition.distribution_params)
+        w = ops.RowStores(self.device)
         for k in self.observations:
-            self.observations[k][s].copy_(transition.observations[k])
-        self.actions[s].copy_(transition.actions)
-        self.rewards[s].copy_(transition.rewards.view(-1, 1))
-        self.dones[s].copy_(transition.dones.view(-1, 1))
-        self.values[s].copy_(transition.values)
-        self.actions_log_prob[s].copy_(transition.actions_log_prob.view(-1, 1))
+            w.copy(self.observations[k][s], transition.observations[k])
+        w.copy(self.actions[s], transition.actions)
+        if bootstrap is None:
+            w.copy(self.rewards[s], transition.rewards.view(-1, 1))
+        else:
+            w.bootstrap(self.rewards[s], transition.rewards, *bootstrap)
+        w.copy(self.dones[s], transition.dones.view(-1, 1))
+        w.copy(self.values[s], transition.values)
+        w.copy(self.actions_log_prob[s], transition.actions_log_prob.view(-1, 1))
         for i, p in enumerate(transition.distribution_params):
-            self.distribution_params[i][s].copy_(p)
-        self._save_hidden_states(transition.hidden_states)
+            w.copy(self.distribution_params[i][s], p)
+        self._save_hidden_states(transition.hidden_states, w)
+        w.flush()
         self.step += 1
 
     def _interleave(self, params) -> None:
@@ -112,7 +138,7 @@ class RolloutStorage:
         else:
             self.distribution_params = tuple(torch.zeros(T, *p.shape, device=self.device) for p in params)
 
-    def _save_hidden_states(self, hidden_states) -> None:
+    def _save_hidden_states(self, hidden_states, writes: ops.RowStores) -> None:
         """rollout_storage.py:333-359: the recurrent models' state before each step's forward, as saved_hidden_state_a /
         _c = [h, c] each [T, num_layers, N, H] (zero where a model had no state yet)."""
         if hidden_states is None or hidden_states == (None, None):
@@ -126,7 +152,7 @@ class RolloutStorage:
             if getattr(self, name) is None:
                 setattr(self, name, [torch.zeros(T, *h.shape, device=self.device) for h in hs])
             for buf, h in zip(getattr(self, name), hs):
-                buf[self.step].copy_(h)
+                writes.copy(buf[self.step], h)
 
     def clear(self) -> None:
         self.step = 0

@@ -4,8 +4,8 @@
 // read across the wavefront (64-lane blocks spread small env counts over many CUs).  HBM-bound: per element 4 B reward + 4 B value + 1 B done in, 4 B return + 4 B
 // advantage out.  Contraction is disabled so the fp32 results are bit-identical to torch's op-by-op evaluation.
 //
-// Advantage normalisation: fp64 block partial sums, a fixed-order second stage (deterministic), then the
-// normalising pass.  Three launches over n floats.
+// Advantage normalisation: fp64 block partial sums, summed in a fixed order (deterministic), then the normalising pass.
+// Three launches over n floats.
 #include "common.hpp"
 
 #pragma clang fp contract(off)
@@ -83,13 +83,43 @@ __device__ inline double block_sum(double x, double* red) {
   return s;  // valid in thread 0
 }
 
-// Pass 1 (mode 0): partial sums of x.  Pass 2 (mode 1): partial sums of (x - mean)^2 with mean from stats[0].
+// Fixed-order sum of up to kNormMaxBlocks partials, by one wavefront: lane l sums partials l, l + 64, ... in order (all
+// of its loads issued before the first add), then a fixed butterfly combines the lanes.
+__device__ inline double sum_partials(const double* __restrict__ partials, int nparts, int lane) {
+  constexpr int kPer = (kNormMaxBlocks + 63) / 64;
+  double v[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) v[j] = partials[min(lane + 64 * j, nparts - 1)];
+  double s = 0.0;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j)
+    if (lane + 64 * j < nparts) s += v[j];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  return s;
+}
+
+// torch's mean() and std(): rounded to fp32
+__device__ inline double mean_of(double sum, int64_t n) { return static_cast<float>(sum / static_cast<double>(n)); }
+__device__ inline double std_of(double sq, int64_t n) { return static_cast<float>(sqrt(sq / static_cast<double>(n - 1))); }
+
+// mode 0: partial sums of x.  mode 1: partial sums of (x - mean)^2, the mean from mode 0's partials, which every block
+// sums for itself, 8 KB from the caches: a launch of one block between the passes, used before, took 1.8 us and its gap
+// (compute_returns of 4,096 x 24 humanoid envs 105.5 -> 100.3 us).
 __global__ __launch_bounds__(kNormThreads) void adv_partials_kernel(const float* __restrict__ x, int64_t stride,
                                                                     int64_t n, int mode,
-                                                                    const double* __restrict__ stats,
+                                                                    const double* __restrict__ sums,
                                                                     double* __restrict__ partials) {
   __shared__ double red[kNormThreads / 64];
-  const double mean = mode ? stats[0] : 0.0;
+  __shared__ double s_mean;
+  double mean = 0.0;
+  if (mode != 0) {
+    if (threadIdx.x < 64) {
+      const double s = sum_partials(sums, gridDim.x, threadIdx.x);
+      if (threadIdx.x == 0) s_mean = mean_of(s, n);
+    }
+    __syncthreads();
+    mean = s_mean;
+  }
   double acc = 0.0;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kNormThreads + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * kNormThreads) {
@@ -105,36 +135,23 @@ __global__ __launch_bounds__(kNormThreads) void adv_partials_kernel(const float*
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
-// Fixed-order reduction of the partials.  mode 0 -> stats[0] = mean (rounded through fp32 like torch's mean());
-// mode 1 -> stats[1] = unbiased std rounded to fp32.
-// One wavefront: lane l sums partials l, l + 64, ... in order (all of its loads issued before the first add), then
-// a fixed butterfly combines the lanes.
-__global__ __launch_bounds__(64) void adv_stats_kernel(const double* __restrict__ partials, int nparts, int64_t n,
-                                                       int mode, double* __restrict__ stats) {
-  constexpr int kPer = (kNormMaxBlocks + 63) / 64;
-  double v[kPer];
-#pragma unroll
-  for (int j = 0; j < kPer; ++j) v[j] = partials[min(static_cast<int>(threadIdx.x) + 64 * j, nparts - 1)];
-  double s = 0.0;
-#pragma unroll
-  for (int j = 0; j < kPer; ++j)
-    if (static_cast<int>(threadIdx.x) + 64 * j < nparts) s += v[j];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if (threadIdx.x != 0) return;
-  if (mode == 0) {
-    stats[0] = static_cast<double>(static_cast<float>(s / static_cast<double>(n)));
-  } else {
-    const double var = s / static_cast<double>(n - 1);
-    stats[1] = static_cast<double>(static_cast<float>(sqrt(var)));
-  }
-}
-
+// The grid is the partials' (one per block of either pass).
 __global__ __launch_bounds__(kNormThreads) void adv_apply_kernel(const float* __restrict__ x, int64_t in_stride,
                                                                  float* __restrict__ out, int64_t out_stride,
                                                                  int64_t n, float eps,
-                                                                 const double* __restrict__ stats) {
-  const float mean = static_cast<float>(stats[0]);
-  const float denom = static_cast<float>(stats[1]) + eps;
+                                                                 const double* __restrict__ sums,
+                                                                 const double* __restrict__ squares) {
+  __shared__ float s_mean, s_denom;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (wave < 2) {
+    const double s = sum_partials(wave == 0 ? sums : squares, gridDim.x, lane);
+    if (lane == 0) {
+      if (wave == 0) s_mean = static_cast<float>(mean_of(s, n));
+      else s_denom = static_cast<float>(std_of(s, n)) + eps;
+    }
+  }
+  __syncthreads();
+  const float mean = s_mean, denom = s_denom;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kNormThreads + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * kNormThreads) {
     out[i * out_stride] = (x[i * in_stride] - mean) / denom;
@@ -186,7 +203,7 @@ extern "C" int ppo_gae(const float* rewards, const float* values, const uint8_t*
 }
 
 extern "C" size_t ppo_adv_normalize_workspace_bytes(int64_t n) {
-  return sizeof(double) * (2 + static_cast<size_t>(n > 0 ? norm_blocks(n) : 1));
+  return sizeof(double) * 2 * static_cast<size_t>(n > 0 ? norm_blocks(n) : 1);
 }
 
 extern "C" int ppo_adv_normalize(const float* x, int64_t in_stride, float* out, int64_t out_stride, int64_t n,
@@ -204,16 +221,12 @@ extern "C" int ppo_adv_normalize(const float* x, int64_t in_stride, float* out, 
   PPO_REQUIRE(workspace && workspace_bytes >= ppo_adv_normalize_workspace_bytes(n),
               "ppo_adv_normalize: workspace too small (%zu < %zu)", workspace_bytes,
               ppo_adv_normalize_workspace_bytes(n));
-  double* stats = static_cast<double*>(workspace);
-  double* partials = stats + 2;
+  double* sums = static_cast<double*>(workspace);
   const int blocks = norm_blocks(n);
-  hipLaunchKernelGGL(adv_partials_kernel, dim3(blocks), dim3(kNormThreads), 0, s, x, in_stride, n, 0, stats,
-                     partials);
-  hipLaunchKernelGGL(adv_stats_kernel, dim3(1), dim3(64), 0, s, partials, blocks, n, 0, stats);
-  hipLaunchKernelGGL(adv_partials_kernel, dim3(blocks), dim3(kNormThreads), 0, s, x, in_stride, n, 1, stats,
-                     partials);
-  hipLaunchKernelGGL(adv_stats_kernel, dim3(1), dim3(64), 0, s, partials, blocks, n, 1, stats);
-  hipLaunchKernelGGL(adv_apply_kernel, dim3(blocks), dim3(kNormThreads), 0, s, x, in_stride, out, out_stride, n,
-                     eps, stats);
+  double* squares = sums + blocks;
+  hipLaunchKernelGGL(adv_partials_kernel, dim3(blocks), dim3(kNormThreads), 0, s, x, in_stride, n, 0, nullptr, sums);
+  hipLaunchKernelGGL(adv_partials_kernel, dim3(blocks), dim3(kNormThreads), 0, s, x, in_stride, n, 1, sums, squares);
+  hipLaunchKernelGGL(adv_apply_kernel, dim3(blocks), dim3(kNormThreads), 0, s, x, in_stride, out, out_stride, n, eps, sums,
+                     squares);
   return check_launch("adv_normalize");
 }

@@ -198,6 +198,7 @@ constexpr int kDwBM = 128, kDwBN = 128, kDwChunk = 64;
 constexpr int kDwBlocksPerCu = 3;     // the bf16x6 kernel (168 VGPRs, 48 KiB LDS)
 constexpr int kDwF16BlocksPerCu = 2;  // the fp16x3 kernel (two accumulators: 256 VGPRs, 64 KiB LDS)
 constexpr int kDwF32BlocksPerCu = 2;  // the fp32 kernel, for operands without 16-byte rows
+constexpr int kDwNarrow = 2, kDwNarrowF16 = 4;  // a narrow problem's tiles in quarters of a full one's (see dw_narrow)
 constexpr int kDwMaxConcurrent = kDwBlocksPerCu * 256;
 
 int dw_query_capacity() {
@@ -230,20 +231,25 @@ struct DwPlan {
   size_t total_floats;
 };
 
-// A problem at most 64 columns wide (in_features) runs on 128 x 64 tiles in the bf16x6 kernel (half a tile's work per
-// block), so it gets half the splits of the others: every block of the launch then has about the same work.
+// A problem at most 64 columns wide (in_features) runs on 128 x 64 tiles: half a tile's products per slab of rows, so in
+// the bf16x6 kernel, which its products bound, it gets half the splits of the others (every block of the launch then has
+// about the same work).  In the fp16x3 kernel, half as many products, a slab takes a narrow tile as long as a full one
+// (loads, barrier), and with half the splits its blocks ran on alone: compute units busy 68 % of 2,017 us (flat48 with
+// 393,216 rows per mini-batch; the update 112.7 ms).  As many splits as the others: the update 104.4 ms (three quarters
+// of them: 105.6 ms, 1,517 us).
 bool dw_narrow(const ppo_linear_bwd_dw_problem& q) { return q.in_features <= kDwBN / 2; }
 
-DwPlan plan_dw(const ppo_linear_bwd_dw_problem* probs, int count, int64_t rows, int capacity) {
+// `weight` and `share`: a narrow tile's work and its problem's split count, in quarters of a full one's.
+DwPlan plan_dw(const ppo_linear_bwd_dw_problem* probs, int count, int64_t rows, int capacity, int weight, int share) {
   DwPlan plan{};
-  int64_t halves = 0;  // work in half tiles (128 x 64)
+  int64_t quarters = 0;
   for (int i = 0; i < count; ++i)
-    halves += ceil_div(probs[i].out_features, kDwBM) *
-              (dw_narrow(probs[i]) ? 1 : 2 * ceil_div(probs[i].in_features, kDwBN));
-  const int s_full = dw_splits((halves + 1) / 2, rows, capacity);
+    quarters += ceil_div(probs[i].out_features, kDwBM) *
+                (dw_narrow(probs[i]) ? weight : 4 * ceil_div(probs[i].in_features, kDwBN));
+  const int s_full = dw_splits((quarters + 3) / 4, rows, capacity);
   size_t off = 0;
   for (int i = 0; i < count; ++i) {
-    const int s = dw_narrow(probs[i]) ? std::max(1, s_full / 2) : s_full;
+    const int s = dw_narrow(probs[i]) ? std::max(1, s_full * share / 4) : s_full;
     const int64_t chunk = ceil_div(ceil_div(rows, s), kDwChunk) * kDwChunk;
     const int splits = static_cast<int>(ceil_div(rows, chunk));
     plan.splits[i] = splits;
@@ -850,7 +856,8 @@ extern "C" size_t ppo_linear_bwd_dw_workspace_bytes(const ppo_linear_bwd_dw_prob
   if (problems == nullptr || count < 1 || count > PPO_MAX_LINEAR_PROBLEMS || !rows_ok(rows)) return 0;
   for (int i = 0; i < count; ++i)
     if (problems[i].in_features <= 0 || problems[i].out_features <= 0) return 0;
-  return plan_dw(problems, count, rows, dw_query_capacity()).total_floats * sizeof(float);
+  // no fewer splits than any launch takes: the most blocks, the least weight and the largest share
+  return plan_dw(problems, count, rows, dw_query_capacity(), kDwNarrow, kDwNarrowF16).total_floats * sizeof(float);
 }
 
 namespace ppo {
@@ -904,7 +911,8 @@ int dw_gemm(const ppo_linear_bwd_dw_problem* problems, int32_t count, int64_t ro
     occ = cfg[std::strlen(cfg) - 1] - '0';
   }
 #endif
-  const DwPlan plan = plan_dw(problems, count, rows, dw_launch_capacity(occ));
+  const int narrow = f16 ? kDwNarrowF16 : kDwNarrow;
+  const DwPlan plan = plan_dw(problems, count, rows, dw_launch_capacity(occ), narrow, narrow);
   PPO_REQUIRE(workspace != nullptr && workspace_bytes >= plan.total_floats * sizeof(float),
               "ppo_linear_bwd_dw: workspace too small (%zu < %zu)", workspace_bytes,
               plan.total_floats * sizeof(float));

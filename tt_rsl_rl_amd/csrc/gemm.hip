@@ -763,11 +763,17 @@ int dx_gemm(const ppo_linear_bwd_dx_problem* problems, int32_t count, int64_t ro
     set_range(p, ranges, i);
     max_n = std::max(max_n, q.in_features);
   }
+  // ELU' from the output has kernels of its own: with the source chosen per four outputs, its expf path lies between
+  // all of them (see nt_epilogue_tiles; with the loads there no longer under a branch of their own, 24,576 rows, humanoid:
+  // 61.4 -> 59.3 us a launch, 393,216 rows, flat48: 754 -> 743 us)
+  const bool out = elu_source == PPO_ELU_FROM_OUTPUT;
   auto plain = [&](auto epi_c, const char* name) {
     constexpr int EPI = decltype(epi_c)::value;
     // the bf16x6 kernel reads the weights as stored (k-major, 16-byte rows): no transpose
-    const int krc = bf16 ? launch_nt_f16<EPI, true, ARITH_BF16>(g, count, s, name)
-                         : launch_nt_bx6<EPI, true>(g, count, s, name);
+    constexpr int OUT = EPI == EPI_ELU_GRAD ? EPI_ELU_GRAD_OUT : EPI;
+    const int krc = bf16 ? (out ? launch_nt_f16<OUT, true, ARITH_BF16>(g, count, s, name)
+                                : launch_nt_f16<EPI, true, ARITH_BF16>(g, count, s, name))
+                         : (out ? launch_nt_bx6<OUT, true>(g, count, s, name) : launch_nt_bx6<EPI, true>(g, count, s, name));
     if (krc != PPO_EUNSUPPORTED) return krc;
     // else w^T (k-contiguous) into the workspace for the other kernels
     if (int rc = launch_transposes(problems, count, ws, offs, s)) return rc;
@@ -786,8 +792,9 @@ int dx_gemm(const ppo_linear_bwd_dx_problem* problems, int32_t count, int64_t ro
   auto run = [&](auto epi_c, const char* name) {
     if (!bf16 && ranges != nullptr) {
       constexpr int EPI = decltype(epi_c)::value;
-      const bool out = elu_source == PPO_ELU_FROM_OUTPUT;
-      const int rc = EPI == EPI_ACT_GRAD && activation == PPO_ACT_TANH && out
+      const int rc = EPI == EPI_ELU_GRAD && out
+                         ? launch_nt_f16<EPI == EPI_ELU_GRAD ? EPI_ELU_GRAD_OUT : EPI, true, ARITH_F16X3>(g, count, s, name)
+                     : EPI == EPI_ACT_GRAD && activation == PPO_ACT_TANH && out
                          ? launch_nt_f16<EPI == EPI_ACT_GRAD ? EPI_TANH_GRAD : EPI, true, ARITH_F16X3>(g, count, s, name)
                      : EPI == EPI_ACT_GRAD && activation == PPO_ACT_RELU
                          ? launch_nt_f16<EPI == EPI_ACT_GRAD ? EPI_RELU_GRAD : EPI, true, ARITH_F16X3>(g, count, s, name)

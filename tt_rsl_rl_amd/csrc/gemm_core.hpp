@@ -51,6 +51,7 @@ enum Epilogue : int {
   EPI_TANH_GRAD = 10,  // product: 48,000 rows x 400 features, two problems, forward 159 us with the call)
   EPI_BIAS_RELU = 11,
   EPI_RELU_GRAD = 12,
+  EPI_ELU_GRAD_OUT = 13,  // EPI_ELU_GRAD from the activation's output (every update; see dx_gemm)
 };
 // The forward epilogues that add the bias and apply an activation, and the input-grad epilogues that multiply by its
 // derivative: ELU's own (the kernels every workload here runs, unchanged by the others' existence) and the generic
@@ -59,7 +60,7 @@ constexpr bool epi_fwd_act(int e) {
   return e == EPI_BIAS_ELU || e == EPI_BIAS_ACT || e == EPI_BIAS_TANH || e == EPI_BIAS_RELU;
 }
 constexpr bool epi_act_grad(int e) {
-  return e == EPI_ELU_GRAD || e == EPI_ACT_GRAD || e == EPI_TANH_GRAD || e == EPI_RELU_GRAD;
+  return e == EPI_ELU_GRAD || e == EPI_ACT_GRAD || e == EPI_TANH_GRAD || e == EPI_RELU_GRAD || e == EPI_ELU_GRAD_OUT;
 }
 constexpr bool epi_generic(int e) { return e == EPI_BIAS_ACT || e == EPI_ACT_GRAD; }
 
@@ -932,11 +933,13 @@ __device__ __forceinline__ void store_b128(__amdgpu_buffer_rsrc_t r, uint32_t of
 // wave's own LDS patch, finished in row order, TM * TN * 4 * OUTS buffer stores in every lane.
 // SCALED (the fp16x3 kernel): the accumulators hold 1 / (s0 s1) times the product, and the activations are the fast
 // forms.  AMAX: returns the largest magnitude among the values this lane wrote (the activation's output of a forward
-// layer).
-template <int TM, int TN, int EPI, bool GEN, bool SCALED = false, bool AMAX = SCALED>
-__device__ __forceinline__ float nt_pipe_epilogue_t(const Problem& P, const f32x16 (&acc)[TM][TN], int row0w,
-                                                    int col0w, float* patch, int lane, float s0 = 1.0f,
-                                                    float s1 = 1.0f) {
+// layer).  STORE_C: a forward epilogue also writes the activation's input.
+// The loop over the tiles has no branch: no wave overlaps a tile's epilogue but the other blocks' of its unit, and a
+// branch per four outputs (the activation gradient's source, rows and columns outside) keeps each four's LDS read, loads
+// and arithmetic from running under the next's.
+template <int TM, int TN, int EPI, bool GEN, bool SCALED, bool AMAX, bool STORE_C>
+__device__ __forceinline__ float nt_epilogue_tiles(const Problem& P, const f32x16 (&acc)[TM][TN], int row0w, int col0w,
+                                                   float* patch, int lane, float s0, float s1) {
   constexpr int PS = 36;
   [[maybe_unused]] float amax = 0.0f;
   const int h = lane >> 5;
@@ -945,27 +948,32 @@ __device__ __forceinline__ float nt_pipe_epilogue_t(const Problem& P, const f32x
   const __amdgpu_buffer_rsrc_t rc = out_buffer(epi_fwd_act(EPI) && P.C == nullptr ? nullptr : P.C, M, P.ldc);
   const __amdgpu_buffer_rsrc_t rc2 = out_buffer(epi_fwd_act(EPI) ? P.C2 : nullptr, M, P.ldc2);
   // every load of the epilogue before its first store: a wait for a load issued after a store would wait for the
-  // store as well (in-order retirement)
+  // store as well (in-order retirement).  Outside the matrix the last row and columns are read (and dropped).
   f32x4 bias[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     bias[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int n = col0w + j * 32 + pc;
-    if ((EPI == EPI_BIAS || epi_fwd_act(EPI)) && n < N) bias[j] = *reinterpret_cast<const f32x4*>(P.vec + n);
+    if (EPI == EPI_BIAS || epi_fwd_act(EPI))
+      bias[j] = *reinterpret_cast<const f32x4*>(P.vec + min(col0w + j * 32 + pc, N - 4));
   }
   f32x4 zsrc[epi_act_grad(EPI) ? TM : 1][epi_act_grad(EPI) ? TN : 1][4];
   if constexpr (epi_act_grad(EPI)) {
+    const float* const aux = P.aux;
+    const int64_t ldaux = P.ldaux;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+      for (int rr = 0; rr < 4; ++rr) {
+        const float* const row = aux + static_cast<int64_t>(min(row0w + i * 32 + pr + 8 * rr, M - 1)) * ldaux;
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int n = col0w + j * 32 + pc, m = row0w + i * 32 + pr + 8 * rr;
-          zsrc[i][j][rr] = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
-          if (m < M && n < N) zsrc[i][j][rr] = *reinterpret_cast<const f32x4*>(P.aux + int64_t(m) * P.ldaux + n);
-        }
+        for (int j = 0; j < TN; ++j)
+          zsrc[i][j][rr] = *reinterpret_cast<const f32x4*>(row + min(col0w + j * 32 + pc, N - 4));
+      }
   }
+  // byte offsets of the lane's first piece; rows and tiles further by wave-uniform steps
+  const uint32_t ldc4 = static_cast<uint32_t>(P.ldc * 4), ldc24 = static_cast<uint32_t>(P.ldc2 * 4);
+  const uint32_t off0 = static_cast<uint32_t>(row0w + pr) * ldc4 + static_cast<uint32_t>(col0w + pc) * 4;
+  const uint32_t off20 = static_cast<uint32_t>(row0w + pr) * ldc24 + static_cast<uint32_t>(col0w + pc) * 4;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -975,8 +983,7 @@ __device__ __forceinline__ float nt_pipe_epilogue_t(const Problem& P, const f32x
         f32x4 x = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
         *reinterpret_cast<f32x4*>(patch + (lane & 31) * PS + 8 * q + 4 * h) = x;
       }
-      const int n = col0w + j * 32 + pc;
-      const bool n_in = n < N;  // N % 4 == 0: columns n .. n + 3 are all in or all out
+      const bool n_in = col0w + j * 32 + pc < N;  // N % 4 == 0: columns n .. n + 3 are all in or all out
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
         const int r = pr + 8 * rr;
@@ -985,9 +992,7 @@ __device__ __forceinline__ float nt_pipe_epilogue_t(const Problem& P, const f32x
 #pragma unroll
           for (int e = 0; e < 4; ++e) x[e] = EPI == EPI_BIAS || epi_fwd_act(EPI) ? x[e] * s0 : x[e] * s0 * s1;
         }
-        const int m = row0w + i * 32 + r;
-        const bool ok = m < M && n_in;
-        const int64_t mm = ok ? m : 0;
+        const bool ok = row0w + i * 32 + r < M && n_in;
         f32x4 o, o2 = {};
         if constexpr (EPI == EPI_BIAS || epi_fwd_act(EPI)) {
 #pragma unroll
@@ -996,15 +1001,17 @@ __device__ __forceinline__ float nt_pipe_epilogue_t(const Problem& P, const f32x
             if constexpr (SCALED) act_fwd4_fast<EPI>(P.act, o, o2);
             else act_fwd4<GEN>(P.act, o, o2);
           }
+        } else if constexpr (EPI == EPI_ELU_GRAD_OUT) {
+          act_grad4<false>(P.act, 1, x, zsrc[i][j][rr], o);
         } else if constexpr (epi_act_grad(EPI)) {
           if constexpr (SCALED) act_grad4_fast<EPI>(P.act, P.elu_from_output, x, zsrc[i][j][rr], o);
           else act_grad4<GEN>(P.act, P.elu_from_output, x, zsrc[i][j][rr], o);
         } else {
           o = x;
         }
-        store_b128(rc, ok ? static_cast<uint32_t>((mm * P.ldc + n) * 4) : kDropOffset, o);
-        if constexpr (epi_fwd_act(EPI))
-          store_b128(rc2, ok ? static_cast<uint32_t>((mm * P.ldc2 + n) * 4) : kDropOffset, o2);
+        const uint32_t row_step = static_cast<uint32_t>(i * 32 + 8 * rr);
+        if constexpr (STORE_C) store_b128(rc, ok ? off0 + row_step * ldc4 + 128 * j : kDropOffset, o);
+        if constexpr (epi_fwd_act(EPI)) store_b128(rc2, ok ? off20 + row_step * ldc24 + 128 * j : kDropOffset, o2);
         if constexpr (AMAX) {
           const f32x4 w = epi_fwd_act(EPI) ? o2 : o;
           float q = amax;
@@ -1018,10 +1025,22 @@ __device__ __forceinline__ float nt_pipe_epilogue_t(const Problem& P, const f32x
   return amax;
 }
 
-template <int TM, int TN, int EPI>
+// COUNTED: the caller's waits count the stores, so a forward epilogue without C issues its (dropped) stores too.
+template <int TM, int TN, int EPI, bool GEN, bool SCALED = false, bool AMAX = SCALED, bool COUNTED = false>
+__device__ __forceinline__ float nt_pipe_epilogue_t(const Problem& P, const f32x16 (&acc)[TM][TN], int row0w,
+                                                    int col0w, float* patch, int lane, float s0 = 1.0f,
+                                                    float s1 = 1.0f) {
+  if constexpr (epi_fwd_act(EPI) && !COUNTED) {
+    if (P.C == nullptr)
+      return nt_epilogue_tiles<TM, TN, EPI, GEN, SCALED, AMAX, false>(P, acc, row0w, col0w, patch, lane, s0, s1);
+  }
+  return nt_epilogue_tiles<TM, TN, EPI, GEN, SCALED, AMAX, true>(P, acc, row0w, col0w, patch, lane, s0, s1);
+}
+
+template <int TM, int TN, int EPI, bool COUNTED = false>
 __device__ __forceinline__ void nt_pipe_epilogue(const Problem& P, const f32x16 (&acc)[TM][TN], int row0w, int col0w,
                                                  float* patch, int lane) {
-  nt_pipe_epilogue_t<TM, TN, EPI, epi_generic(EPI)>(P, acc, row0w, col0w, patch, lane);
+  nt_pipe_epilogue_t<TM, TN, EPI, epi_generic(EPI), false, false, COUNTED>(P, acc, row0w, col0w, patch, lane);
 }
 
 template <int BM, int BN, int BK, int OCC, int EPI>
@@ -1147,7 +1166,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(OCC, O
       }
       cstage ^= 1;
     }
-    nt_pipe_epilogue<TM, TN, EPI>(P, acc, cc.tm * BM + wm * WM, cc.tn * BN + wn * WN, patch, lane);
+    nt_pipe_epilogue<TM, TN, EPI, true>(P, acc, cc.tm * BM + wm * WM, cc.tn * BN + wn * WN, patch, lane);
     if (!next_tile) break;
     ctile += nblk;
     first = false;

@@ -84,3 +84,20 @@ def test_rows_are_independent():
     assert torch.isnan(y[3]).all() and not torch.isfinite(y[20]).all()
     keep = [i for i in range(40) if i not in (3, 20)]
     assert torch.equal(y[keep], clean[keep])
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 250])
+@pytest.mark.parametrize("widths,actions,hidden", [((48,), 12, [512, 256, 128]), ((33, 3), 65, [40, 70]),
+                                                   ((20,), 1, [17, 1000, 30, 64, 18]), ((64,), 130, [128, 64, 66, 200])])
+def test_launches_of_two_layers_give_the_one_launch_forward(monkeypatch, rows, widths, actions, hidden):
+    """Three layers to six (an even and an odd count), slices of whole and of partial tiles, widths off 16 bytes: the
+    same bits."""
+    monkeypatch.setattr(models, "PAIR_WEIGHTS", 0)
+    m = _model(widths, actions, hidden, "elu", True)
+    obs = {f"g{i}": torch.randn(rows, w, device="cuda") for i, w in enumerate(widths)}
+    with torch.inference_mode():
+        monkeypatch.setattr(models, "PAIR_ROWS", 0)
+        one = m(obs)
+        monkeypatch.setattr(models, "PAIR_ROWS", 1024)
+        assert m._fused[2] > 0
+        assert torch.equal(m(obs), one)

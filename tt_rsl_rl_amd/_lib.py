@@ -244,6 +244,8 @@ _SIGNATURES = [
                                            C.c_void_p]),
     ("ppo_obs_normalize", C.c_int, [f32p, i64, f32p, i64, i64, i32, f32p, f32p, C.c_float, C.c_void_p]),
     ("ppo_mlp_fwd", C.c_int, [C.POINTER(MlpProblem), i32, i64, C.c_void_p]),
+    ("ppo_mlp_fwd_pairs_workspace_bytes", C.c_size_t, [C.POINTER(MlpProblem), i32, i64]),
+    ("ppo_mlp_fwd_pairs", C.c_int, [C.POINTER(MlpProblem), i32, i64, C.c_void_p, C.c_size_t, C.c_void_p]),
     ("ppo_normalizer_update_workspace_bytes", C.c_size_t, [i64, i32]),
     ("ppo_normalizer_update", C.c_int, [C.POINTER(ColumnBlock), i32, i64, f32p, f32p, f32p, C.c_void_p, C.c_void_p,
                                         C.c_size_t, C.c_void_p]),

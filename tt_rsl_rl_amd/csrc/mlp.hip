@@ -6,8 +6,8 @@
 // its time on launches, on the host calls before them and on GEMM tiles that filled a fraction of the chip (4,096 rows x
 // [512, 256, 128], actor: normaliser and four GEMMs 80 us of kernel time and 94 us of host time).  Here a block takes 16
 // rows through all layers: the rows' activations stay in LDS (two buffers), the weights come from the caches straight
-// into the MFMA operand registers, 64 k ahead, and nothing is written but the output: one launch of 34 us for 16 to
-// 1,024 rows, 37 for 4,096 (37 / 44 us with 96 normalised inputs and 29 actions; the layers one by one 64 / 77 us).  16 rows give 4,096 rows 256 blocks, one per
+// into the MFMA operand registers, 64 k ahead, and nothing is written but the output: one launch of 33 us for 16 to
+// 2,048 rows, 34 for 4,096 (the layers one by one 64 us).  16 rows give 4,096 rows 256 blocks, one per
 // compute unit.  v_mfma_f32_16x16x4f32 with the weights as the first operand leaves each lane 4 consecutive outputs of one
 // row: one 16-byte LDS store each.  Past some thousands of rows the layers' own GEMMs (weights read once per 128 rows, bf16
 // matrix cores) are faster: the caller's choice.
@@ -27,17 +27,37 @@ struct MlpGroup {
 };
 static_assert(sizeof(MlpGroup) <= 4096, "kernel arguments");
 
-// One layer for the block's 16 rows: x [16][ldx] (columns past K up to the next multiple of 16 zero) -> y, or the
-// output.  TILES 16-wide output tiles per wave at a time.  (Deeper prefetch, eight k-groups and the next tiles' first
-// chunk at two waves per SIMD, measured 44 us against 34 for 16 rows of 48 -> [512, 256, 128] -> 12.)
-template <int TILES, bool VEC>
-__device__ __forceinline__ void mlp_layer(const ppo_mlp_layer& L, bool last, int act, const float* x, float* y, int ldx,
-                                          float* out, int64_t ldo, int64_t row0, int64_t rows, int wave, int lane) {
+// One launch of ppo_mlp_fwd_pairs: layers l0 and, where there is one, l0 + 1 of every problem.
+struct MlpPairs {
+  MlpGroup g;
+  const float* in[PPO_MAX_MLP_PROBLEMS];  // [rows, ld] (NULL: the problem's input blocks)
+  float* to[PPO_MAX_MLP_PROBLEMS];        // [rows, ld] (NULL: its output)
+  int64_t ld[PPO_MAX_MLP_PROBLEMS];
+  int32_t slices[PPO_MAX_MLP_PROBLEMS];  // blocks per 16 rows, kSliceTiles tiles of the second layer each
+  int32_t begin1;                        // the second problem's first block
+  int32_t l0;
+};
+static_assert(sizeof(MlpPairs) <= 4096, "kernel arguments");
+constexpr int kSliceTiles = 4;  // one per SIMD
+
+// Where a layer's outputs go: LDS y, or global rows (`out`).
+struct MlpOut {
+  float* y;  // [16][ldx], used where out is NULL
+  float* out;
+  int64_t ldo, row0, rows;
+};
+
+// Output tiles [t_begin, t_end) of one layer for the block's 16 rows: x [16][ldx] (columns past K up to the next multiple
+// of 16 zero) -> D, after the activation `act` (PPO_ACT_NONE: none).  TILES 16-wide output tiles per wave and AH k-groups
+// of 16 loaded ahead at a time.  (For the one launch of all layers, deeper prefetch, eight k-groups and the next tiles'
+// first chunk at two waves per SIMD, measured 44 us against 34 for 16 rows of 48 -> [512, 256, 128] -> 12.)
+template <int TILES, int AH, bool VEC>
+__device__ __forceinline__ void mlp_layer(const ppo_mlp_layer& L, int act, const float* x, int ldx, const MlpOut& D,
+                                          int t_begin, int t_end, int wave, int lane) {
   const int K = L.in_features, N = L.out_features;
   const int m = lane & 15, q = lane >> 4;
-  const int groups = (K + 15) >> 4, tiles = (N + 15) >> 4;
-  constexpr int AH = 4;  // k-groups of 16 loaded ahead
-  for (int t0 = wave * TILES; t0 < tiles; t0 += kMlpWaves * TILES) {
+  const int groups = (K + 15) >> 4;
+  for (int t0 = t_begin + wave * TILES; t0 < t_end; t0 += kMlpWaves * TILES) {
     const float* wrow[TILES];
 #pragma unroll
     for (int j = 0; j < TILES; ++j) wrow[j] = L.w + static_cast<int64_t>(min(16 * (t0 + j) + m, N - 1)) * K;
@@ -63,6 +83,14 @@ __device__ __forceinline__ void mlp_layer(const ppo_mlp_layer& L, bool last, int
     f32x4 w[2][AH][TILES];
 #pragma unroll
     for (int i = 0; i < AH; ++i) load_w(min(i, groups - 1), w[0][i]);
+    float bias[TILES][4];
+    auto load_bias = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < TILES; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bias[j][e] = L.b[min(16 * (t0 + j) + 4 * q + e, N - 1)];
+    };
+    if constexpr (TILES == 1) load_bias();  // (two tiles' weights fill the registers)
     for (int g0 = 0; g0 < groups; g0 += 2 * AH) {
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
@@ -84,25 +112,73 @@ __device__ __forceinline__ void mlp_layer(const ppo_mlp_layer& L, bool last, int
         }
       }
     }
+    if constexpr (TILES > 1) load_bias();
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {
       const int n = 16 * (t0 + j) + 4 * q;
-      if (16 * (t0 + j) >= N) continue;
+      if (t0 + j >= t_end) continue;
       f32x4 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float z = acc[j][0][e] + acc[j][1][e] + L.b[min(n + e, N - 1)];
-        o[e] = n + e >= N ? 0.0f : last ? z : act == PPO_ACT_ELU ? elu_fast(z) : act_fwd(act, z);
+        const float z = acc[j][0][e] + acc[j][1][e] + bias[j][e];
+        o[e] = n + e >= N ? 0.0f : act == PPO_ACT_NONE ? z : act == PPO_ACT_ELU ? elu_fast(z) : act_fwd(act, z);
       }
-      if (!last) {
-        *reinterpret_cast<f32x4*>(y + m * ldx + n) = o;
-      } else if (row0 + m < rows) {
+      if (D.out == nullptr) {
+        *reinterpret_cast<f32x4*>(D.y + m * ldx + n) = o;
+      } else if (D.row0 + m < D.rows) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (n + e < N) out[(row0 + m) * ldo + n + e] = o[e];
+          if (n + e < N) D.out[(D.row0 + m) * D.ldo + n + e] = o[e];
       }
     }
   }
+}
+
+// DEEP: one tile per wave at a time with eight k-groups ahead (a block has a few tiles, each wave's loads are its time).
+template <bool DEEP>
+__device__ __forceinline__ void mlp_run_layer(const ppo_mlp_layer& L, int act, const float* x, int ldx, const MlpOut& D,
+                                              int t_begin, int t_end, int wave, int lane) {
+  const bool vec = L.in_features % 4 == 0 && reinterpret_cast<uintptr_t>(L.w) % 16 == 0;
+  if (!vec)
+    mlp_layer<1, 4, false>(L, act, x, ldx, D, t_begin, t_end, wave, lane);
+  else if (t_end - t_begin > kMlpWaves)
+    mlp_layer<2, 4, true>(L, act, x, ldx, D, t_begin, t_end, wave, lane);
+  else
+    mlp_layer<1, DEEP ? 8 : 4, true>(L, act, x, ldx, D, t_begin, t_end, wave, lane);
+}
+
+__device__ __forceinline__ int mlp_tiles(const ppo_mlp_layer& L) { return (L.out_features + 15) >> 4; }
+
+// The problem's 16 input rows -> x: 32 threads per row, the blocks side by side, normalised as ppo_obs_normalize does.
+__device__ __forceinline__ void mlp_input(const ppo_mlp_problem& P, float* x, int ldx, int64_t row0, int64_t rows, int tid) {
+  const int r = tid >> 5, c0 = tid & 31;
+  const int64_t row = min(row0 + r, rows - 1);
+  const bool in = row0 + r < rows;
+  int col = 0;
+  for (int s = 0; s < P.num_blocks; ++s) {
+    const ppo_column_block& B = P.x[s];
+    const float* const src = B.src + row * B.stride;
+    for (int c = c0; c < B.width; c += 128) {  // four columns' loads in flight (past the width the last one, dropped)
+      float v[4], mean[4], sd[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int cc = min(c + 32 * u, B.width - 1);
+        v[u] = src[cc];
+        if (P.norm_mean != nullptr) {
+          mean[u] = P.norm_mean[col + cc];
+          sd[u] = P.norm_std[col + cc];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        float q = in ? v[u] : 0.0f;
+        if (P.norm_mean != nullptr) q = (q - mean[u]) / (sd[u] + P.norm_eps);
+        if (c + 32 * u < B.width) x[r * ldx + col + c + 32 * u] = q;
+      }
+    }
+    col += B.width;
+  }
+  for (int c = col + c0; c < (col + 15) / 16 * 16; c += 32) x[r * ldx + c] = 0.0f;
 }
 
 __global__ __launch_bounds__(kMlpThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void mlp_fwd_kernel(const MlpGroup g) {
@@ -114,38 +190,13 @@ __global__ __launch_bounds__(kMlpThreads) __attribute__((amdgpu_waves_per_eu(4, 
   const int ldx = g.ldx;
   float* x = lds;
   float* y = lds + kMlpRows * ldx;
-  // the input rows: 32 threads per row, the blocks side by side, normalised as ppo_obs_normalize does
-  {
-    const int r = tid >> 5, c0 = tid & 31;
-    const int64_t row = row0 + r;
-    int col = 0;
-    for (int s = 0; s < P.num_blocks; ++s) {
-      const ppo_column_block& B = P.x[s];
-      for (int c = c0; c < B.width; c += 32) {
-        float v = row < g.rows ? B.src[row * B.stride + c] : 0.0f;
-        if (P.norm_mean != nullptr) v = (v - P.norm_mean[col + c]) / (P.norm_std[col + c] + P.norm_eps);
-        x[r * ldx + col + c] = v;
-      }
-      col += B.width;
-    }
-    for (int c = col + c0; c < (col + 15) / 16 * 16; c += 32) x[r * ldx + c] = 0.0f;
-  }
+  mlp_input(P, x, ldx, row0, g.rows, tid);
   __syncthreads();
   for (int l = 0; l < P.num_layers; ++l) {
     const ppo_mlp_layer& L = P.layers[l];
     const bool last = l == P.num_layers - 1;
-    const bool vec = L.in_features % 4 == 0 && reinterpret_cast<uintptr_t>(L.w) % 16 == 0;
-    const bool wide = L.out_features > 16 * kMlpWaves;
-    auto run = [&](auto tiles_c, auto vec_c) __attribute__((always_inline)) {
-      mlp_layer<decltype(tiles_c)::value, decltype(vec_c)::value>(L, last, P.activation, x, y, ldx, P.out, P.ldo, row0,
-                                                                  g.rows, wave, lane);
-    };
-    if (vec) {
-      if (wide) run(IntC<2>{}, BoolC<true>{});
-      else run(IntC<1>{}, BoolC<true>{});
-    } else {
-      run(IntC<1>{}, BoolC<false>{});
-    }
+    mlp_run_layer<false>(L, last ? PPO_ACT_NONE : P.activation, x, ldx, {y, last ? P.out : nullptr, P.ldo, row0, g.rows}, 0,
+                         mlp_tiles(L), wave, lane);
     __syncthreads();
     float* const t = x;
     x = y;
@@ -153,43 +204,83 @@ __global__ __launch_bounds__(kMlpThreads) __attribute__((amdgpu_waves_per_eu(4, 
   }
 }
 
+// A launch of few rows leaves all but a few compute units idle and takes the time of one block's products and load
+// latencies (16 rows of 48 -> [512, 256, 128] -> 12: 33 us in one launch, 10 of them fp32 MFMA).  Here each 16 rows have
+// as many blocks as the pair's second layer has groups of four tiles, each computing the first layer for itself: two
+// launches of 13.4 us for the four layers, no waits between blocks.
+// Layers l0 (all of it, in LDS) and l0 + 1 (the block's slice of tiles, to global memory), or a slice of l0 alone.
+__global__ __launch_bounds__(kMlpThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void mlp_pairs_kernel(const MlpPairs a) {
+  extern __shared__ __align__(16) float lds[];
+  const int pi = static_cast<int>(blockIdx.x) >= a.begin1 ? 1 : 0;
+  const ppo_mlp_problem& P = a.g.p[pi];
+  const int b = static_cast<int>(blockIdx.x) - (pi ? a.begin1 : 0);
+  const int slices = a.slices[pi], rb = b / slices, slice = b - rb * slices;
+  const int64_t row0 = static_cast<int64_t>(rb) * kMlpRows, rows = a.g.rows;
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
+  const int ldx = a.g.ldx;
+  float* x = lds;
+  float* y = lds + kMlpRows * ldx;
+  if (a.l0 >= P.num_layers) return;  // (the other problem has more layers)
+  if (a.in[pi] == nullptr) {
+    mlp_input(P, x, ldx, row0, rows, tid);
+  } else {  // a previous launch's rows, whole 16-byte pieces
+    const int K = P.layers[a.l0].in_features, pieces = (K + 15) / 16 * 4;
+    const int64_t ld = a.ld[pi];
+    for (int i = tid; i < kMlpRows * pieces; i += kMlpThreads) {
+      const int r = i / pieces, c = 4 * (i - r * pieces);
+      const f32x4 v = *reinterpret_cast<const f32x4*>(a.in[pi] + min(row0 + r, rows - 1) * ld + min(c, static_cast<int>(ld) - 4));
+      f32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = c + e < K ? v[e] : 0.0f;
+      *reinterpret_cast<f32x4*>(x + r * ldx + c) = o;
+    }
+  }
+  __syncthreads();
+  int l = a.l0;
+  if (l + 1 < P.num_layers) {
+    mlp_run_layer<true>(P.layers[l], P.activation, x, ldx, {y, nullptr, 0, row0, rows}, 0, mlp_tiles(P.layers[l]), wave, lane);
+    __syncthreads();
+    x = y;
+    ++l;
+  }
+  const bool last = l == P.num_layers - 1;
+  const int t0 = slice * kSliceTiles, t1 = min(t0 + kSliceTiles, mlp_tiles(P.layers[l]));
+  mlp_run_layer<true>(P.layers[l], last ? PPO_ACT_NONE : P.activation, x, ldx,
+                      {nullptr, last ? P.out : a.to[pi], last ? P.ldo : a.ld[pi], row0, rows}, t0, t1, wave, lane);
+}
+
 int64_t round16(int64_t n) { return (n + 15) / 16 * 16; }
 
-}  // namespace
-}  // namespace ppo
-
-using namespace ppo;
-
-extern "C" int ppo_mlp_fwd(const ppo_mlp_problem* problems, int32_t count, int64_t rows, ppo_stream_t stream) {
-  PPO_REQUIRE(problems != nullptr && count >= 1 && count <= PPO_MAX_MLP_PROBLEMS, "ppo_mlp_fwd: count=%d outside [1, %d]",
-              count, PPO_MAX_MLP_PROBLEMS);
-  PPO_REQUIRE(rows > 0 && rows <= INT32_MAX / 4, "ppo_mlp_fwd: rows=%lld", (long long)rows);
-  MlpGroup g{};
+// The checked problems as kernel arguments.
+int mlp_group(const ppo_mlp_problem* problems, int32_t count, int64_t rows, const char* who, MlpGroup& g) {
   int64_t widest = 0;
+  PPO_REQUIRE(problems != nullptr && count >= 1 && count <= PPO_MAX_MLP_PROBLEMS, "%s: count=%d outside [1, %d]", who,
+              count, PPO_MAX_MLP_PROBLEMS);
+  PPO_REQUIRE(rows > 0 && rows <= INT32_MAX / 4, "%s: rows=%lld", who, (long long)rows);
   for (int i = 0; i < count; ++i) {
     const ppo_mlp_problem& q = problems[i];
     PPO_REQUIRE(q.num_blocks >= 1 && q.num_blocks <= PPO_MAX_MLP_BLOCKS && q.num_layers >= 1 &&
                     q.num_layers <= PPO_MAX_MLP_LAYERS,
-                "ppo_mlp_fwd: problem %d: %d input blocks (at most %d), %d layers (at most %d)", i, q.num_blocks,
+                "%s: problem %d: %d input blocks (at most %d), %d layers (at most %d)", who, i, q.num_blocks,
                 PPO_MAX_MLP_BLOCKS, q.num_layers, PPO_MAX_MLP_LAYERS);
-    PPO_REQUIRE(q.activation >= PPO_ACT_NONE && q.activation < PPO_ACT_COUNT, "ppo_mlp_fwd: activation=%d", q.activation);
-    PPO_REQUIRE((q.norm_mean == nullptr) == (q.norm_std == nullptr), "ppo_mlp_fwd: problem %d: one of mean / std", i);
+    PPO_REQUIRE(q.activation >= PPO_ACT_NONE && q.activation < PPO_ACT_COUNT, "%s: activation=%d", who, q.activation);
+    PPO_REQUIRE((q.norm_mean == nullptr) == (q.norm_std == nullptr), "%s: problem %d: one of mean / std", who, i);
     int64_t width = 0;
     for (int s = 0; s < q.num_blocks; ++s) {
-      PPO_REQUIRE(q.x[s].src && q.x[s].width > 0 && q.x[s].stride >= q.x[s].width, "ppo_mlp_fwd: problem %d: input block %d",
-                  i, s);
+      PPO_REQUIRE(q.x[s].src && q.x[s].width > 0 && q.x[s].stride >= q.x[s].width, "%s: problem %d: input block %d",
+                  who, i, s);
       width += q.x[s].width;
     }
     for (int l = 0; l < q.num_layers; ++l) {
       const ppo_mlp_layer& L = q.layers[l];
       PPO_REQUIRE(L.w && L.b && L.in_features == width && L.out_features > 0,
-                  "ppo_mlp_fwd: problem %d layer %d: %d -> %d features after %lld", i, l, L.in_features, L.out_features,
+                  "%s: problem %d layer %d: %d -> %d features after %lld", who, i, l, L.in_features, L.out_features,
                   (long long)width);
-      if (width > kMlpMaxWidth) return fail(PPO_EUNSUPPORTED, "ppo_mlp_fwd: layers of at most %d features", kMlpMaxWidth);
+      if (width > kMlpMaxWidth) return fail(PPO_EUNSUPPORTED, "%s: layers of at most %d features", who, kMlpMaxWidth);
       widest = std::max(widest, width);
       width = L.out_features;
     }
-    PPO_REQUIRE(q.out && q.ldo >= width, "ppo_mlp_fwd: problem %d output", i);
+    PPO_REQUIRE(q.out && q.ldo >= width, "%s: problem %d output", who, i);
     g.p[i] = q;
   }
   g.count = count;
@@ -197,10 +288,80 @@ extern "C" int ppo_mlp_fwd(const ppo_mlp_problem* problems, int32_t count, int64
   g.blocks = static_cast<int>(ceil_div(rows, static_cast<int64_t>(kMlpRows)));
   // rows of whole 64 floats plus 4: a 16-byte read of the same columns of 16 rows falls on all 64 banks
   g.ldx = static_cast<int>((round16(widest) + 63) / 64 * 64 + 4);
+  return PPO_OK;
+}
+
+template <typename K, typename A>
+int launch_mlp(K kernel, int64_t blocks, const MlpGroup& g, const A& args, hipStream_t s, const char* name) {
   const size_t lds = 2 * static_cast<size_t>(kMlpRows) * g.ldx * sizeof(float);
   if (lds > 64 * 1024)
-    PPO_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mlp_fwd_kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kMlpRows * (kMlpMaxWidth + 4) * 4));
-  hipLaunchKernelGGL(mlp_fwd_kernel, dim3(count * g.blocks), dim3(kMlpThreads), lds, static_cast<hipStream_t>(stream), g);
-  return check_launch("mlp_fwd_kernel");
+    PPO_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      2 * kMlpRows * (kMlpMaxWidth + 4) * 4));
+  PPO_REQUIRE(blocks <= INT32_MAX, "%s: too many rows", name);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kMlpThreads), lds, s, args);
+  return check_launch(name);
+}
+
+// Floats per row of one of a problem's two intermediate buffers: its widest layer of odd index but the last (0: none).
+int64_t pairs_width(const ppo_mlp_problem& q) {
+  int64_t w = 0;
+  for (int l = 1; l + 1 < q.num_layers && l < PPO_MAX_MLP_LAYERS; l += 2)
+    w = std::max<int64_t>(w, (q.layers[l].out_features + 3) / 4 * 4);
+  return w;
+}
+
+}  // namespace
+}  // namespace ppo
+
+using namespace ppo;
+
+extern "C" int ppo_mlp_fwd(const ppo_mlp_problem* problems, int32_t count, int64_t rows, ppo_stream_t stream) {
+  MlpGroup g{};
+  if (int rc = mlp_group(problems, count, rows, "ppo_mlp_fwd", g)) return rc;
+  return launch_mlp(mlp_fwd_kernel, static_cast<int64_t>(count) * g.blocks, g, g, static_cast<hipStream_t>(stream),
+                    "mlp_fwd_kernel");
+}
+
+extern "C" size_t ppo_mlp_fwd_pairs_workspace_bytes(const ppo_mlp_problem* problems, int32_t count, int64_t rows) {
+  if (problems == nullptr || count < 1 || count > PPO_MAX_MLP_PROBLEMS || rows <= 0) return 0;
+  int64_t floats = 0;
+  for (int i = 0; i < count; ++i) floats += 2 * pairs_width(problems[i]);
+  return static_cast<size_t>(floats) * static_cast<size_t>(rows) * sizeof(float);
+}
+
+extern "C" int ppo_mlp_fwd_pairs(const ppo_mlp_problem* problems, int32_t count, int64_t rows, void* workspace,
+                                 size_t workspace_bytes, ppo_stream_t stream) {
+  MlpPairs a{};
+  if (int rc = mlp_group(problems, count, rows, "ppo_mlp_fwd_pairs", a.g)) return rc;
+  const size_t need = ppo_mlp_fwd_pairs_workspace_bytes(problems, count, rows);
+  PPO_REQUIRE(need == 0 || (workspace != nullptr && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0),
+              "ppo_mlp_fwd_pairs: workspace of %zu bytes (%zu, 16-byte aligned, needed)", workspace_bytes, need);
+  float* buf[PPO_MAX_MLP_PROBLEMS][2] = {};
+  int layers = 0;
+  float* ws = static_cast<float*>(workspace);
+  for (int i = 0; i < count; ++i) {
+    a.ld[i] = pairs_width(problems[i]);
+    for (int k = 0; k < 2; ++k) {
+      buf[i][k] = ws;
+      if (ws != nullptr) ws += rows * a.ld[i];
+    }
+    layers = std::max(layers, problems[i].num_layers);
+  }
+  for (int l0 = 0, p = 0; l0 < layers; l0 += 2, ++p) {
+    int64_t blocks = 0;
+    for (int i = 0; i < count; ++i) {
+      const ppo_mlp_problem& q = problems[i];
+      const int l = std::min(l0 + 1, q.num_layers - 1);  // the sliced layer
+      a.in[i] = p == 0 ? nullptr : buf[i][(p - 1) & 1];
+      a.to[i] = buf[i][p & 1];
+      a.slices[i] = static_cast<int>(ceil_div(ceil_div(q.layers[l].out_features, 16), kSliceTiles));
+      if (i == 1) a.begin1 = static_cast<int>(blocks);
+      if (l0 < q.num_layers) blocks += static_cast<int64_t>(a.g.blocks) * a.slices[i];
+      PPO_REQUIRE(blocks <= INT32_MAX, "ppo_mlp_fwd_pairs: too many rows");
+    }
+    if (count == 1) a.begin1 = INT32_MAX;
+    a.l0 = l0;
+    if (int rc = launch_mlp(mlp_pairs_kernel, blocks, a.g, a, static_cast<hipStream_t>(stream), "mlp_pairs_kernel")) return rc;
+  }
+  return PPO_OK;
 }

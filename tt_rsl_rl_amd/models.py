@@ -255,6 +255,11 @@ class _ForwardBuffers:
 # rows, one per compute unit.  48 -> [512, 256, 128] -> 12, one launch / layer by layer: 16 rows 34 / 64 us, 4,096 rows
 # 37 / 63, 8,192 rows 59 / 62, 16,384 rows 112 / 74.
 FUSED_ROWS = 4096
+# Up to this many rows that forward is a launch per two layers, the second one's outputs spread over several blocks
+# (ppo_mlp_fwd_pairs), where those second layers (but the last) hold at least PAIR_WEIGHTS weights: fewer do not pay for
+# the further launch.  48 inputs, 16 rows, two launches / one: hidden 512-256-128 (131,072 weights) 26.7 / 33.3 us,
+# 256-256-256 (65,536) 27.4 / 29.3, 128-128 (16,384) 21.6 / 17.1; 512-256-128 with 1,024 rows 27.6 / 33.8, 2,048 35.5 / 33.9.
+PAIR_ROWS, PAIR_WEIGHTS = 1024, 65536
 
 
 # attributes of a model or distribution that act() goes through; one set on the instance stands for another behaviour
@@ -294,7 +299,7 @@ class MLPModel(nn.Module):
         self.mlp = nn.Sequential(*layers)
         self.output_dim = mlp_out
         self._fwd = _ForwardBuffers()
-        self._fused: tuple | None = None  # (addresses the record was built from, the ppo_mlp_fwd record)
+        self._fused: tuple | None = None  # (addresses it was built from, the ppo_mlp_fwd record, workspace bytes per row)
 
     # -- structure ---------------------------------------------------------------------------------------------------
     def _get_obs_dim(self, obs: Mapping, obs_groups: dict, obs_set: str) -> tuple[list[str], int]:
@@ -350,7 +355,11 @@ class MLPModel(nn.Module):
                 rec.layers[i] = L.MlpLayer(l.weight.data_ptr(), l.bias.data_ptr(), l.in_features, l.out_features)
             if norm is not None:
                 rec.norm_mean, rec.norm_std, rec.norm_eps = norm._mean.data_ptr(), norm._std.data_ptr(), norm.eps
-        self._fused = (key, rec)
+        second = sum(l.in_features * l.out_features for l in layers[1:-1:2])
+        per_row = 0
+        if rec is not None and second >= PAIR_WEIGHTS:
+            per_row = L.load().ppo_mlp_fwd_pairs_workspace_bytes(ops.C_ref(rec), 1, 1)
+        self._fused = (key, rec, per_row)
         return rec
 
     def _fused_forward(self, columns: list[torch.Tensor], norm) -> torch.Tensor | None:
@@ -376,7 +385,13 @@ class MLPModel(nn.Module):
         rec.num_blocks = len(columns)
         out = torch.empty(rows, rec.layers[rec.num_layers - 1].out_features, device=columns[0].device)
         rec.out, rec.ldo = out.data_ptr(), out.stride(0)
-        L.call("ppo_mlp_fwd", ops.C_ref(rec), 1, rows, torch.cuda.current_stream().cuda_stream)
+        stream = torch.cuda.current_stream().cuda_stream
+        nbytes = rows * self._fused[2]
+        if rows <= PAIR_ROWS and nbytes:
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=out.device)
+            L.call("ppo_mlp_fwd_pairs", ops.C_ref(rec), 1, rows, ws.data_ptr(), nbytes, stream)
+        else:
+            L.call("ppo_mlp_fwd", ops.C_ref(rec), 1, rows, stream)
         return out
 
     def mlp_forward(self, latent: torch.Tensor) -> torch.Tensor:

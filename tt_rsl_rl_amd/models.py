@@ -142,7 +142,7 @@ class GaussianDistribution(nn.Module):
                None if noise is None else noise.data_ptr(), 0 if noise is None else noise.stride(0),
                actions.data_ptr(), actions.stride(0), None if logp is None else logp.data_ptr(),
                None if std_out is None else std_out.data_ptr(), 0 if std_out is None else std_out.stride(0),
-               mean.shape[0], self.output_dim, torch.cuda.current_stream().cuda_stream)
+               mean.shape[0], self.output_dim, ops._stream())
 
     def update(self, mean: torch.Tensor) -> None:
         """Record the distribution of the last forward (the std broadcast per row, as upstream's Normal does)."""
@@ -371,6 +371,7 @@ class MLPModel(nn.Module):
         rec = self._mlp_record(norm)
         if rec is None:
             return None
+        rec, per_row = L.MlpProblem.from_buffer_copy(rec), self._fused[2]  # (this call's own: its buffers go into it)
         width = 0
         for i, x in enumerate(columns):
             if x.dtype != torch.float32 or x.shape[0] != rows or not x.is_cuda:
@@ -385,8 +386,8 @@ class MLPModel(nn.Module):
         rec.num_blocks = len(columns)
         out = torch.empty(rows, rec.layers[rec.num_layers - 1].out_features, device=columns[0].device)
         rec.out, rec.ldo = out.data_ptr(), out.stride(0)
-        stream = torch.cuda.current_stream().cuda_stream
-        nbytes = rows * self._fused[2]
+        stream = ops._stream()
+        nbytes = rows * per_row
         if rows <= PAIR_ROWS and nbytes:
             ws = torch.empty(nbytes, dtype=torch.uint8, device=out.device)
             L.call("ppo_mlp_fwd_pairs", ops.C_ref(rec), 1, rows, ws.data_ptr(), nbytes, stream)

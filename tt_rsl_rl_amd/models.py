@@ -267,6 +267,14 @@ _STOCHASTIC = frozenset(("forward", "get_output_log_prob", "update", "sample", "
                          "deterministic_output"))
 
 
+class _FusedRecord(tuple):
+    """(addresses it was built from, the ppo_mlp_fwd record, workspace bytes per row).  The record holds pointers: a
+    copied or pickled model starts without one."""
+
+    def __reduce__(self):
+        return type(None), ()
+
+
 class MLPModel(nn.Module):
     """rsl_rl/models/mlp_model.py:19-193 (same signature; registration order normalizer, distribution, mlp)."""
 
@@ -299,7 +307,7 @@ class MLPModel(nn.Module):
         self.mlp = nn.Sequential(*layers)
         self.output_dim = mlp_out
         self._fwd = _ForwardBuffers()
-        self._fused: tuple | None = None  # (addresses it was built from, the ppo_mlp_fwd record, workspace bytes per row)
+        self._fused: _FusedRecord | None = None
 
     # -- structure ---------------------------------------------------------------------------------------------------
     def _get_obs_dim(self, obs: Mapping, obs_groups: dict, obs_set: str) -> tuple[list[str], int]:
@@ -359,7 +367,7 @@ class MLPModel(nn.Module):
         per_row = 0
         if rec is not None and second >= PAIR_WEIGHTS:
             per_row = L.load().ppo_mlp_fwd_pairs_workspace_bytes(ops.C_ref(rec), 1, 1)
-        self._fused = (key, rec, per_row)
+        self._fused = _FusedRecord((key, rec, per_row))
         return rec
 
     def _fused_forward(self, columns: list[torch.Tensor], norm) -> torch.Tensor | None:

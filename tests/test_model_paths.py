@@ -48,3 +48,46 @@ def test_a_model_that_ran_copies_and_pickles():
         assert m._fused is not None and m._fused[1] is not None
         for c in _copies(m):
             assert torch.equal(c(obs), y)
+
+
+class _Doubled(torch.nn.Module):
+    """A parametrisation: the weight is computed on each access."""
+
+    def forward(self, w):
+        return 2.0 * w
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", ["eps", "activation", "shape", "transposed", "parametrised"])
+def test_the_record_follows_what_it_was_made_from(change):
+    """A changed normaliser eps or activation, a weight of another shape or layout at the same address, weights computed
+    on access: the one-launch forward gives what the layers give."""
+    m = _model(width=32, hidden=(32, 16)).to("cuda")
+    obs = {"g": torch.randn(100, 32, device="cuda")}
+    with torch.no_grad():
+        before = m(obs)
+        if change == "eps":
+            m.obs_normalizer.eps = 0.5
+        elif change == "activation":
+            m.act_code = L.ACTIVATIONS["tanh"]
+        elif change == "shape":  # the same memory as another layer stack: 32 -> 16 -> 16 -> 4
+            first, second = m.mlp[0], m.mlp[2]
+            first.weight.data = first.weight.data[:16]
+            first.bias.data = first.bias.data[:16]
+            second.weight.data = second.weight.data.view(-1)[:256].view(16, 16)
+            first.out_features, second.in_features = 16, 16
+        elif change == "transposed":  # (the layers take contiguous weights only)
+            m.mlp[0].weight.data = m.mlp[0].weight.data.t()
+            for call in (m, m.forward_layers):
+                with pytest.raises(ValueError, match="contiguous"):
+                    call(obs)
+            return
+        elif change == "parametrised":
+            torch.nn.utils.parametrize.register_parametrization(m.mlp[2], "weight", _Doubled())
+        else:
+            m.mlp[0].weight.data = m.mlp[0].weight.data.clone()
+        after, want = m(obs), m.forward_layers(obs)
+        assert float((after - want).norm() / want.norm()) < 1e-5
+        assert not torch.equal(before, after)
+        for _ in range(20):  # (memory handed round between the computed weights, the output and the workspace)
+            assert torch.equal(m(obs), after)

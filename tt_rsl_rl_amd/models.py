@@ -268,8 +268,8 @@ _STOCHASTIC = frozenset(("forward", "get_output_log_prob", "update", "sample", "
 
 
 class _FusedRecord(tuple):
-    """(addresses it was built from, the ppo_mlp_fwd record, workspace bytes per row).  The record holds pointers: a
-    copied or pickled model starts without one."""
+    """(what it was built from, the ppo_mlp_fwd record, workspace bytes per row).  The record holds pointers: a copied
+    or pickled model starts without one."""
 
     def __reduce__(self):
         return type(None), ()
@@ -345,30 +345,40 @@ class MLPModel(nn.Module):
                 dst.copy_(x)
             col += w
 
-    def _mlp_record(self, norm) -> "L.MlpProblem | None":
-        """The layers (and the normaliser) as ppo_mlp_fwd takes them; rebuilt when a parameter lives elsewhere.  None:
-        outside what it takes."""
+    def _mlp_record(self, norm) -> tuple:
+        """The layers (and the normaliser) as ppo_mlp_fwd takes them, or None where it does not; the workspace bytes per
+        row of its launches by pairs; and the tensors the record points into, which the caller holds until its launch
+        (a parametrised weight is a new tensor on each access).  Kept from call to call, rebuilt when anything it was
+        made from changed: a tensor's address, shape, strides or type, the activation, the normaliser's eps."""
         layers = [m for m in self.mlp if isinstance(m, nn.Linear)]
         tensors = [t for l in layers for t in (l.weight, l.bias)]
         if norm is not None:
             tensors += [norm._mean, norm._std]
-        key = tuple(t.data_ptr() for t in tensors)
+        if any(t is None for t in tensors):
+            return None, 0, tensors
+        key = (self.act_code, None if norm is None else norm.eps,
+               *[(t.data_ptr(), t.shape, t.stride(), t.dtype) for t in tensors])
         if self._fused is not None and self._fused[0] == key:
-            return self._fused[1]
-        rec = None
-        if (len(layers) <= L.MAX_MLP_LAYERS and all(l.in_features <= L.MLP_MAX_WIDTH for l in layers) and
+            return self._fused[1], self._fused[2], tensors
+        rec, per_row = None, 0
+        shapes = [t.shape for t in tensors]
+        if (len(layers) <= L.MAX_MLP_LAYERS and
+                all(len(w) == 2 and b == w[:1] and w[1] <= L.MLP_MAX_WIDTH for w, b in
+                    zip(shapes[0:2 * len(layers):2], shapes[1:2 * len(layers):2])) and
+                (norm is None or norm._mean.numel() == norm._std.numel() == shapes[0][1]) and
                 all(t.dtype == torch.float32 and t.is_contiguous() and t.is_cuda for t in tensors)):
             rec = L.MlpProblem(num_layers=len(layers), activation=self.act_code)
-            for i, l in enumerate(layers):
-                rec.layers[i] = L.MlpLayer(l.weight.data_ptr(), l.bias.data_ptr(), l.in_features, l.out_features)
+            second = 0
+            for i in range(len(layers)):
+                w, b = tensors[2 * i], tensors[2 * i + 1]
+                rec.layers[i] = L.MlpLayer(w.data_ptr(), b.data_ptr(), w.shape[1], w.shape[0])
+                second += w.numel() if i % 2 == 1 and i < len(layers) - 1 else 0
             if norm is not None:
                 rec.norm_mean, rec.norm_std, rec.norm_eps = norm._mean.data_ptr(), norm._std.data_ptr(), norm.eps
-        second = sum(l.in_features * l.out_features for l in layers[1:-1:2])
-        per_row = 0
-        if rec is not None and second >= PAIR_WEIGHTS:
-            per_row = L.load().ppo_mlp_fwd_pairs_workspace_bytes(ops.C_ref(rec), 1, 1)
+            if second >= PAIR_WEIGHTS:
+                per_row = L.load().ppo_mlp_fwd_pairs_workspace_bytes(ops.C_ref(rec), 1, 1)
         self._fused = _FusedRecord((key, rec, per_row))
-        return rec
+        return rec, per_row, tensors
 
     def _fused_forward(self, columns: list[torch.Tensor], norm) -> torch.Tensor | None:
         """The whole forward on the concatenation of `columns` ([rows, width] each) in one launch; None where the
@@ -376,10 +386,10 @@ class MLPModel(nn.Module):
         rows = columns[0].shape[0]
         if rows > FUSED_ROWS or rows == 0 or len(columns) > L.MAX_MLP_BLOCKS:
             return None
-        rec = self._mlp_record(norm)
+        rec, per_row, held = self._mlp_record(norm)  # (held: until the launch below is issued)
         if rec is None:
             return None
-        rec, per_row = L.MlpProblem.from_buffer_copy(rec), self._fused[2]  # (this call's own: its buffers go into it)
+        rec = L.MlpProblem.from_buffer_copy(rec)  # (this call's own: its buffers go into it)
         width = 0
         for i, x in enumerate(columns):
             if x.dtype != torch.float32 or x.shape[0] != rows or not x.is_cuda:

@@ -9,6 +9,7 @@ import pickle
 
 import pytest
 import torch
+import torch.nn.utils.parametrize
 
 from tt_rsl_rl_amd import _lib as L
 from tt_rsl_rl_amd import models
@@ -84,10 +85,110 @@ def test_the_record_follows_what_it_was_made_from(change):
             return
         elif change == "parametrised":
             torch.nn.utils.parametrize.register_parametrization(m.mlp[2], "weight", _Doubled())
-        else:
-            m.mlp[0].weight.data = m.mlp[0].weight.data.clone()
         after, want = m(obs), m.forward_layers(obs)
         assert float((after - want).norm() / want.norm()) < 1e-5
         assert not torch.equal(before, after)
         for _ in range(20):  # (memory handed round between the computed weights, the output and the workspace)
             assert torch.equal(m(obs), after)
+
+
+class _OwnMlp(MLPModel):
+    def mlp_forward(self, latent):
+        return 3.0 * super().mlp_forward(latent)
+
+
+class _OwnCall(MLPModel):
+    def __call__(self, obs, **kw):
+        return 3.0 * super().__call__(obs, **kw)
+
+
+def _own_on_instance(m, name):
+    f = getattr(m, name)
+    setattr(m, name, {"latent_into": lambda obs, out: (f(obs, out), out.mul_(0.5))[0]}.get(name, lambda *a, **k: 3.0 * f(*a, **k)))
+
+
+def _overridden(how):
+    if how in ("mlp_forward", "call"):
+        return _model({"mlp_forward": _OwnMlp, "call": _OwnCall}[how]).to("cuda")
+    m = _model().to("cuda")
+    if how == "hook":
+        m.register_forward_hook(lambda mod, args, out: 3.0 * out)
+    elif how == "pre_hook":
+        m.register_forward_pre_hook(lambda mod, args: ({"g": 0.5 * args[0]["g"]},))
+    else:
+        _own_on_instance(m, how.split(".")[1])
+    return m
+
+
+_WAYS = ["mlp_forward", "call", "hook", "pre_hook", "instance.forward", "instance.mlp_forward", "instance.get_latent",
+         "instance.latent_into"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", _WAYS)
+@pytest.mark.parametrize("rows", [50, 5000])
+def test_overrides_and_hooks_run_at_every_size(how, rows):
+    """What a user puts in a method's place or between runs on few rows (the one-launch forward) as on many."""
+    m = _overridden(how)
+    obs = {"g": torch.randn(rows, 20, device="cuda")}
+    with torch.no_grad():
+        plain, got = _model().to("cuda")(obs), m(obs)
+        factor = {"pre_hook": None, "instance.latent_into": None, "instance.get_latent": None}.get(how, 3.0)
+        if factor is None:
+            assert float((got - plain).norm() / plain.norm()) > 0.05
+            z = torch.cat([m(obs) for _ in range(2)])
+            assert torch.equal(z[:rows], z[rows:])
+        else:
+            assert float((got - factor * plain).norm() / plain.norm()) < 1e-5
+        # the layers themselves, through the same methods
+        big = {"g": obs["g"].repeat(-(-5000 // rows), 1)}
+        assert float((m(big)[:rows] - got).norm() / got.norm()) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", [None, *_WAYS])
+def test_the_bootstrap_value_is_the_critics_call(how):
+    """compute_returns takes V(s_T) from calling the critic, as act() takes V(s_t), whatever stands in the call."""
+    from types import SimpleNamespace
+
+    from tt_rsl_rl_amd.ppo import PPO
+
+    n = 64
+    model = dict(class_name="MLPModel", hidden_dims=[32, 16], activation="elu")
+    cfg = dict(algorithm=dict(class_name="tt_rsl_rl_amd.ppo:PPO"),
+               actor=dict(model, distribution_cfg=dict(class_name="GaussianDistribution")), critic=model,
+               obs_groups={"actor": ["g"], "critic": ["g"]}, num_steps_per_env=1)
+    alg = PPO.construct_algorithm({"g": torch.zeros(n, 20)}, SimpleNamespace(num_envs=n, num_actions=3), cfg, "cuda:0")
+    if how is not None:
+        alg.critic = _overridden(how)
+    seen = []
+    alg.compute_returns_from = lambda v: seen.append(v.clone())
+    obs = {"g": torch.randn(n, 20, device="cuda")}
+    with torch.inference_mode():
+        want = alg.critic(obs)
+        alg.compute_returns(obs)
+    assert float((seen[0] - want).norm() / want.norm()) < 1e-5
+    assert alg.critic.forwards_plainly() is (how is None)
+
+
+@pytest.mark.gpu
+def test_a_storage_with_its_own_add_transition_gets_the_transition_alone():
+    from types import SimpleNamespace
+
+    from tt_rsl_rl_amd.ppo import PPO
+
+    n = 16
+    model = dict(class_name="MLPModel", hidden_dims=[16], activation="elu")
+    cfg = dict(algorithm=dict(class_name="tt_rsl_rl_amd.ppo:PPO", gamma=0.5),
+               actor=dict(model, distribution_cfg=dict(class_name="GaussianDistribution")), critic=model,
+               obs_groups={"actor": ["g"], "critic": ["g"]}, num_steps_per_env=1)
+    alg = PPO.construct_algorithm({"g": torch.zeros(n, 5)}, SimpleNamespace(num_envs=n, num_actions=3), cfg, "cuda:0")
+    seen, own = [], alg.storage.add_transition
+    alg.storage.add_transition = lambda tr: (seen.append(tr.rewards.clone()), own(tr))[1]
+    obs = {"g": torch.randn(n, 5, device="cuda")}
+    with torch.inference_mode():
+        alg.act(obs)
+        v = alg.transition.values.clone()
+        r, t = torch.randn(n, device="cuda"), torch.ones(n, device="cuda")
+        alg.process_env_step(obs, r, t, {"time_outs": t})
+    assert torch.equal(seen[0], r + 0.5 * v[:, 0]) and torch.equal(alg.storage.rewards[0, :, 0], seen[0])

@@ -445,7 +445,7 @@ class MLPModel(nn.Module):
         if masks is not None:
             raise NotImplementedError("padded (recurrent) batches are not supported by the MLP HIP path")
         out = None
-        if type(self).get_latent is MLPModel.get_latent and type(self).latent_into is MLPModel.latent_into:
+        if self._own(MLPModel, "get_latent", "latent_into", "mlp_forward"):
             cols = [obs[g] for g in self.obs_groups]
             if all(x.is_cuda and x.dim() == 2 for x in cols):
                 out = self._fused_forward(cols, self.obs_normalizer if self.obs_normalization else None)
@@ -458,13 +458,30 @@ class MLPModel(nn.Module):
             return self.distribution.deterministic_output(out)
         return out
 
+    def _own(self, cls: type, *names: str) -> bool:
+        """These methods are `cls`'s: neither a subclass nor the instance has one of its own."""
+        return all(getattr(type(self), n) is getattr(cls, n) and n not in self.__dict__ for n in names)
+
+    def _called_directly(self) -> bool:
+        """Nothing stands between a call of this model and its forward: no hook, no compiled call."""
+        return not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks or self._backward_pre_hooks) \
+            and not torch.nn.modules.module._has_any_global_hook() and self._compiled_call_impl is None
+
     def acts_plainly(self) -> bool:
         """Calling this model runs this class's forward on a Gaussian head and nothing else: no subclass, hook, compiled
         or replaced forward between (``sample_scored`` then gives what the calls of act() give)."""
         return (type(self) in (MLPModel, RNNModel) and type(self.distribution) is GaussianDistribution and
-                not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks or self._backward_pre_hooks)
-                and not torch.nn.modules.module._has_any_global_hook() and self._compiled_call_impl is None and
+                self._called_directly() and
                 _STOCHASTIC.isdisjoint(self.__dict__) and _STOCHASTIC.isdisjoint(self.distribution.__dict__))
+
+    def forwards_plainly(self) -> bool:
+        """Calling this model runs the package's layers and nothing else (``forward_layers`` then gives what the call
+        gives, but for the rounding)."""
+        cls = RNNModel if isinstance(self, RNNModel) else MLPModel
+        return self._called_directly() and \
+            self._own(cls, "__call__", "forward", "get_latent", "latent_into", "mlp_forward") and \
+            (self.distribution is None or (type(self.distribution) is GaussianDistribution and
+                                           _STOCHASTIC.isdisjoint(self.distribution.__dict__)))
 
     def sample_scored(self, obs: Mapping) -> tuple[torch.Tensor, torch.Tensor]:
         """The stochastic forward and its output's log-probability: (actions, log_prob)."""

@@ -244,7 +244,7 @@ class PPO:
         """ppo.py:124-135."""
         self.transition.hidden_states = (self.actor.get_hidden_state(), self.critic.get_hidden_state())
         logp = None
-        if self.actor.acts_plainly():
+        if isinstance(self.actor, MLPModel) and self.actor.acts_plainly():
             self.transition.actions, logp = self.actor.sample_scored(obs)
         else:
             self.transition.actions = self.actor(obs, stochastic_output=True).detach()
@@ -263,7 +263,9 @@ class PPO:
         boot = None
         if "time_outs" in extras:
             boot = Bootstrap(self.gamma, tr.values, extras["time_outs"])
-        if boot is not None and type(self.storage).add_transition is RolloutStorage.add_transition and boot.fits(rewards):
+        # (an add_transition of a subclass's or the instance's own takes the transition alone)
+        own = getattr(self.storage.add_transition, "__func__", None) is RolloutStorage.add_transition
+        if boot is not None and own and boot.fits(rewards):
             tr.rewards = rewards  # (read by the launch that writes the transition)
             self.storage.add_transition(tr, boot)
         else:
@@ -280,7 +282,8 @@ class PPO:
         critic_hidden_state = self.critic.get_hidden_state()
         # layer by layer at every size: the bootstrap value enters every advantage, and its rounding (another one in the
         # one-launch forward that act() uses) is carried through all of the update's steps (see RANGED_ROWS in engine.py)
-        plain = type(self.critic).forward in (MLPModel.forward, RNNModel.forward)
+        # where something stands between (a hook, a compiled call, a method of the user's own), the call itself
+        plain = isinstance(self.critic, MLPModel) and self.critic.forwards_plainly()
         last_values = (self.critic.forward_layers(obs) if plain else self.critic(obs)).detach().contiguous()
         # the bootstrap forward must not advance the critic's rollout state (ppo.py:170-173)
         self.critic.reset(hidden_state=critic_hidden_state)

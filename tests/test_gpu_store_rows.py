@@ -91,3 +91,18 @@ def test_act_and_step_match_the_general_path(cuda, envs, actions, rnn):
 
     for i, (x, y) in enumerate(zip(collect(False), collect(True), strict=True)):
         assert torch.equal(x, y), i
+
+
+def test_sources_made_for_the_call(cuda):
+    """Observations that a mapping computes on access are freed with the call that took them: each destination still gets
+    its own."""
+    from tt_rsl_rl_amd import ops
+
+    src = [torch.full((512, 8), float(i), device=cuda) for i in range(6)]
+    dst = [torch.empty(512, 8, device=cuda) for _ in src]
+    w = ops.RowStores(cuda)
+    for d, s in zip(dst, src):
+        w.copy(d, s.clone())
+    w.bootstrap(dst[0][:, :1].clone(), src[0][:, 0].clone(), 0.5, src[1][:, :1].clone(), src[2][:, 0].clone())
+    w.flush()
+    assert all(torch.equal(d, s) for d, s in zip(dst, src)) and not w.items and not w.held

@@ -110,7 +110,8 @@ def _rows_of(t: torch.Tensor) -> tuple[int, int, int] | None:
 class RowStores:
     """Writes ``dst.copy_(src)`` into device buffers, gathered into one ppo_store_rows launch; a pair it does not take
     (another device, shape, layout or type, tensor subclasses, gradients) is copied by torch at once.  Nothing else may
-    read the destinations before ``flush()``, and a source must stay as it is until then."""
+    read the destinations before ``flush()``, and a source's values must stay as they are until then; the tensors
+    themselves are held (a source that was made for the call alone would be freed, its memory another source's)."""
 
     def __init__(self, device: torch.device) -> None:
         self.device = None  # no pair fits
@@ -119,6 +120,7 @@ class RowStores:
             if device.index in (None, index):
                 self.device = torch.device("cuda", index)
         self.items: list[bytes] = []
+        self.held: list[tuple] = []
 
     def copy(self, dst: torch.Tensor, src: torch.Tensor) -> None:
         kind = L.STORE_F32 if dst.dtype == torch.float32 else L.STORE_U8 if dst.dtype == torch.uint8 else None
@@ -137,7 +139,7 @@ class RowStores:
             rows, width = max(d[:2], s[:2])
             d = (rows, width, width) if d[0] == 1 else d
             s = (rows, width, width) if s[0] == 1 else s
-        self._add(L.STORE_ITEM.pack(src.data_ptr(), s[2], dst.data_ptr(), d[2], d[0], d[1], kind, 0, 0, 0.0, t))
+        self._add(L.STORE_ITEM.pack(src.data_ptr(), s[2], dst.data_ptr(), d[2], d[0], d[1], kind, 0, 0, 0.0, t), dst, src)
 
     def bootstrap(self, dst: torch.Tensor, rewards: torch.Tensor, gamma: float, values: torch.Tensor,
                   flags: torch.Tensor) -> None:
@@ -147,17 +149,18 @@ class RowStores:
             dst.copy_((rewards + gamma * (values.view(-1) * flags)).view(dst.shape))
             return
         self._add(L.STORE_ITEM.pack(rewards.data_ptr(), 1, dst.data_ptr(), 1, n, 1, L.STORE_BOOTSTRAP, values.data_ptr(),
-                                    flags.data_ptr(), gamma, STORE_FLAGS[flags.dtype]))
+                                    flags.data_ptr(), gamma, STORE_FLAGS[flags.dtype]), dst, rewards, values, flags)
 
-    def _add(self, item: bytes) -> None:
+    def _add(self, item: bytes, *tensors: torch.Tensor) -> None:
         self.items.append(item)
+        self.held.append(tensors)
         if len(self.items) == L.MAX_STORE_ITEMS:
             self.flush()
 
     def flush(self) -> None:
         if self.items:
             L.call("ppo_store_rows", b"".join(self.items), len(self.items), _stream())
-            self.items = []
+            self.items, self.held = [], []
 
 
 # ----------------------------------------------------------------------------------------------------------------------

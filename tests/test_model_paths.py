@@ -192,3 +192,28 @@ def test_a_storage_with_its_own_add_transition_gets_the_transition_alone():
         r, t = torch.randn(n, device="cuda"), torch.ones(n, device="cuda")
         alg.process_env_step(obs, r, t, {"time_outs": t})
     assert torch.equal(seen[0], r + 0.5 * v[:, 0]) and torch.equal(alg.storage.rewards[0, :, 0], seen[0])
+
+
+# (inputs, hidden layers), rows, the fastest of the routes as measured (us): one launch, by pairs, layer by layer
+@pytest.mark.parametrize("width,hidden,rows,us", [
+    (48, [512, 256, 128], 16, (33.4, 27.0, 50.9)), (48, [512, 256, 128], 4096, (33.8, 56.0, 51.3)),
+    (460, [512, 256, 128], 1024, (52.9, 48.5, 83.2)), (460, [512, 256, 128], 4096, (53.9, 130.0, 87.2)),
+    (235, [512, 256, 128], 16, (75.4, 69.3, 64.7)), (235, [512, 256, 128], 4096, (75.9, 220.0, 73.5)),
+    (48, [1024, 512, 256], 16, (94.3, 49.1, 74.4)), (48, [1024, 512, 256], 1024, (94.3, 72.5, 75.9)),
+    (48, [1024, 512, 256], 4096, (95.2, 207.8, 80.9)), (48, [1024, 1024, 1024], 16, (263.1, 160.4, 112.3)),
+    (48, [1024, 1024, 1024], 4096, (264.9, 500.2, 156.5)), (235, [1024, 512, 256, 128], 1024, (184.7, 251.2, 109.6)),
+    (1000, [512, 512], 1024, (90.1, 131.0, 118.8)), (49, [1023, 511], 1024, (178.8, 114.3, 133.9)),
+    (49, [1023, 511], 4096, (179.2, 420.3, 138.9)), (99, [256, 128, 64], 4096, (24.9, 41.7, 50.6))])
+def test_wide_networks_keep_the_route_that_is_faster(width, hidden, rows, us):
+    dims = [width, *hidden, 12]
+    second = sum(a * b for i, (a, b) in enumerate(zip(dims[:-1], dims[1:])) if i % 2 == 1 and i < len(dims) - 2)
+    chosen = models._Route.of(dims).choose(rows, second >= models.PAIR_WEIGHTS)
+    assert dict(zip(("one", "pairs", "layers"), us))[chosen] <= 1.08 * min(us)
+
+
+@pytest.mark.gpu
+def test_a_wide_network_of_few_rows_runs_layer_by_layer():
+    m = _model(hidden=(1024, 1024, 1024), norm=False).to("cuda")
+    obs = {"g": torch.randn(100, 20, device="cuda")}
+    with torch.no_grad():
+        assert torch.equal(m(obs), m.forward_layers(obs))

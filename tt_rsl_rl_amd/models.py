@@ -10,7 +10,7 @@ pass on the GPU runs the HIP kernels of libppo_hip.so; CPU tensors are rejected.
 from __future__ import annotations
 
 import copy
-from typing import Mapping
+from typing import Mapping, NamedTuple
 
 import numpy as np
 import torch
@@ -251,8 +251,8 @@ class _ForwardBuffers:
         return [b[:rows] for b in self.bufs]
 
 
-# Up to this many rows a model's forward is one launch (ppo_mlp_fwd), above it one GEMM launch per layer: 256 blocks of 16
-# rows, one per compute unit.  48 -> [512, 256, 128] -> 12, one launch / layer by layer: 16 rows 33 / 64 us, 4,096 rows
+# Up to this many rows a model's forward is one launch (ppo_mlp_fwd) where its weights are few enough (_Route), above it one
+# GEMM launch per layer: 256 blocks of 16 rows, one per compute unit.  48 -> [512, 256, 128] -> 12, one launch / layer by layer: 16 rows 33 / 64 us, 4,096 rows
 # 34 / 63, 8,192 rows 59 / 62, 16,384 rows 112 / 74.
 FUSED_ROWS = 4096
 # Up to this many rows that forward is a launch per two layers, the second one's outputs spread over several blocks
@@ -262,14 +262,53 @@ FUSED_ROWS = 4096
 PAIR_ROWS, PAIR_WEIGHTS = 1024, 65536
 
 
+class _Route(NamedTuple):
+    """Estimated times (us) of one model's forward: in one launch, by pairs of layers (one wave of blocks), layer by layer;
+    and the blocks per 16 rows of its widest pair."""
+
+    one: float
+    pairs: float
+    layers: float
+    slices: int
+
+    @staticmethod
+    def of(dims: list[int]) -> "_Route":
+        """dims: the inputs, each layer's outputs.  A block of the one-launch forward reads every weight for its 16 rows:
+        0.115 us per 1,000 of them, 0.36 where a row is not whole 16 bytes, which is what a wide network's time is;
+        layer by layer it is mostly launches, with a k chain of 0.02 us per column (0.06 off 16 columns).  Fitted to 13
+        networks of 16 and 4,096 rows; one launch / layers measured: 48-[512, 256, 128] 34 / 51 (estimated 34 / 59),
+        460-[512, 256, 128] 53 / 87 (58 / 85), 235-[512, 256, 128] 76 / 72 (74 / 72), 48-[1024, 512, 256] 95 / 81 (93 /
+        76), 48-[1024, 1024, 1024] 263 / 112 (260 / 102), 49-[1023, 511] 179 / 139 (220 / 126)."""
+        one, pairs, layers, slices = 12.0, 0.0, 7.0, 1
+        shapes = list(zip(dims[:-1], dims[1:]))
+        for i, (k, n) in enumerate(shapes):
+            vec = k % 4 == 0
+            one += k * n * (0.115e-3 if vec else 0.36e-3)
+            layers += 8.2 + k * (0.02 if k % 16 == 0 else 0.06)
+            if i % 2 == 0 and i + 1 < len(shapes):
+                pairs += k * n * (0.1e-3 if vec else 0.42e-3)
+            else:  # (a pair's second layer, or a last one alone: 64 outputs per block)
+                pairs += 8.0 + k * (0.01 if vec else 0.03)
+                slices = max(slices, -(-n // 64))
+        return _Route(one, pairs, layers, slices)
+
+    def choose(self, rows: int, pairs_fit: bool) -> str:
+        """"one", "pairs" or "layers".  More blocks by pairs than the 256 compute units take run one after another."""
+        waves = -(-(-(-rows // 16) * self.slices) // 256)
+        by_pairs = self.pairs * max(1.0, 0.75 * waves)
+        if pairs_fit and rows <= PAIR_ROWS and (waves == 1 or by_pairs < self.one):
+            return "pairs" if by_pairs <= self.layers else "layers"
+        return "one" if self.one <= self.layers else "layers"
+
+
 # attributes of a model or distribution that act() goes through; one set on the instance stands for another behaviour
 _STOCHASTIC = frozenset(("forward", "get_output_log_prob", "update", "sample", "log_prob", "sample_from",
                          "deterministic_output"))
 
 
 class _FusedRecord(tuple):
-    """(what it was built from, the ppo_mlp_fwd record, workspace bytes per row).  The record holds pointers: a copied
-    or pickled model starts without one."""
+    """(what it was built from, the ppo_mlp_fwd record, workspace bytes per row, the _Route).  The record holds pointers:
+    a copied or pickled model starts without one."""
 
     def __reduce__(self):
         return type(None), ()
@@ -346,21 +385,21 @@ class MLPModel(nn.Module):
             col += w
 
     def _mlp_record(self, norm) -> tuple:
-        """The layers (and the normaliser) as ppo_mlp_fwd takes them, or None where it does not; the workspace bytes per
-        row of its launches by pairs; and the tensors the record points into, which the caller holds until its launch
-        (a parametrised weight is a new tensor on each access).  Kept from call to call, rebuilt when anything it was
+        """The cached (key, record, workspace bytes per row by pairs, route) of this model, the record None where
+        ppo_mlp_fwd does not take the layers, and the tensors the record points into, which the caller holds until its
+        launch (a parametrised weight is a new tensor on each access).  Kept from call to call, rebuilt when anything it was
         made from changed: a tensor's address, shape, strides or type, the activation, the normaliser's eps."""
         layers = [m for m in self.mlp if isinstance(m, nn.Linear)]
         tensors = [t for l in layers for t in (l.weight, l.bias)]
         if norm is not None:
             tensors += [norm._mean, norm._std]
         if any(t is None for t in tensors):
-            return None, 0, tensors
+            return (None, None, 0, None), tensors
         key = (self.act_code, None if norm is None else norm.eps,
                *[(t.data_ptr(), t.shape, t.stride(), t.dtype) for t in tensors])
         if self._fused is not None and self._fused[0] == key:
-            return self._fused[1], self._fused[2], tensors
-        rec, per_row = None, 0
+            return self._fused, tensors
+        rec, per_row, route = None, 0, None
         shapes = [t.shape for t in tensors]
         if (len(layers) <= L.MAX_MLP_LAYERS and
                 all(len(w) == 2 and b == w[:1] and w[1] <= L.MLP_MAX_WIDTH for w, b in
@@ -377,17 +416,21 @@ class MLPModel(nn.Module):
                 rec.norm_mean, rec.norm_std, rec.norm_eps = norm._mean.data_ptr(), norm._std.data_ptr(), norm.eps
             if second >= PAIR_WEIGHTS:
                 per_row = L.load().ppo_mlp_fwd_pairs_workspace_bytes(ops.C_ref(rec), 1, 1)
-        self._fused = _FusedRecord((key, rec, per_row))
-        return rec, per_row, tensors
+            route = _Route.of([shapes[0][1], *[w[0] for w in shapes[0:2 * len(layers):2]]])
+        self._fused = _FusedRecord((key, rec, per_row, route))
+        return self._fused, tensors
 
     def _fused_forward(self, columns: list[torch.Tensor], norm) -> torch.Tensor | None:
-        """The whole forward on the concatenation of `columns` ([rows, width] each) in one launch; None where the
-        layers run one by one."""
+        """The whole forward on the concatenation of `columns` ([rows, width] each) in one launch, or one per two layers;
+        None where the layers run one by one."""
         rows = columns[0].shape[0]
         if rows > FUSED_ROWS or rows == 0 or len(columns) > L.MAX_MLP_BLOCKS:
             return None
-        rec, per_row, held = self._mlp_record(norm)  # (held: until the launch below is issued)
+        (_, rec, per_row, route), held = self._mlp_record(norm)  # (held: until the launch below is issued)
         if rec is None:
+            return None
+        by = route.choose(rows, per_row > 0)
+        if by == "layers":
             return None
         rec = L.MlpProblem.from_buffer_copy(rec)  # (this call's own: its buffers go into it)
         width = 0
@@ -405,8 +448,8 @@ class MLPModel(nn.Module):
         out = torch.empty(rows, rec.layers[rec.num_layers - 1].out_features, device=columns[0].device)
         rec.out, rec.ldo = out.data_ptr(), out.stride(0)
         stream = ops._stream()
-        nbytes = rows * per_row
-        if rows <= PAIR_ROWS and nbytes:
+        if by == "pairs":
+            nbytes = rows * per_row
             ws = torch.empty(nbytes, dtype=torch.uint8, device=out.device)
             L.call("ppo_mlp_fwd_pairs", ops.C_ref(rec), 1, rows, ws.data_ptr(), nbytes, stream)
         else:

@@ -247,11 +247,13 @@ int ppo_linear_bwd_dw_ex(const ppo_linear_bwd_dw_problem* problems, int32_t coun
                          void* workspace, size_t workspace_bytes, const float* extra_grads,
                          const ppo_grad_range* extra, int32_t num_extra, double* norm_partials, ppo_stream_t stream);
 
-/* Largest magnitudes.  PPO_AMAX_WORDS words per tensor: PPO_AMAX_SLOTS slots, one per 128-byte line (its first word; the
- * others are unused), the maximum over the slots being the fp32 bits of max |x| over the tensor's finite values (an
- * upper bound serves as well).  ppo_amax writes the slots of each item (x: [rows, cols], row
- * stride ld) and clears `clear_words` words at `clear`, the slots that kernels after it on the stream add to; both in
- * one launch.  No counterpart in the reference. */
+/* Ranges.  PPO_AMAX_WORDS words per tensor: PPO_AMAX_SLOTS slots, one per 128-byte line.  A slot's first word holds fp32
+ * bits whose maximum over the slots is max |x| over the tensor's finite values (an upper bound serves as well; the slots
+ * that a GEMM or the head raises also count infinities), its second word what the smallest nonzero max |x| among the
+ * tensor's parts is (csrc/amax.hpp); the others are unused.  ppo_amax finds them: parts are rows (of up to 256 columns) and
+ * columns (within a block's rows), coarse items take several rows at a time for a part.  It writes every slot of each item
+ * (x: [rows, cols], row stride ld), or with `raise` raises them from what they hold, and clears `clear_words` words at
+ * `clear`, the slots that kernels after it on the stream add to; both in one launch.  No counterpart in the reference. */
 #define PPO_AMAX_SLOTS 64
 #define PPO_AMAX_WORDS (PPO_AMAX_SLOTS * 32)
 #define PPO_MAX_AMAX_ITEMS 16
@@ -260,16 +262,22 @@ typedef struct ppo_amax_item {
   int64_t rows;
   int32_t cols;
   float least;    /* the slots' maximum is at least this (>= 0) */
-  uint32_t* slots;
+  uint32_t* slots; /* 8-byte aligned */
+  int32_t coarse;
+  int32_t reserved;
+  const uint32_t* source[2]; /* NULL, or the slots of tensors x was computed from: one beyond fp16x3's range, so is x */
 } ppo_amax_item;
-int ppo_amax(const ppo_amax_item* items, int32_t count, uint32_t* clear, int64_t clear_words, ppo_stream_t stream);
+int ppo_amax(const ppo_amax_item* items, int32_t count, uint32_t* clear, int64_t clear_words, int32_t raise,
+             ppo_stream_t stream);
 
-/* The three GEMMs with the operands' largest magnitudes known (ranges: one per problem, in the problems' order; a / b:
- * the slots of the first and the second operand -- x and w, dz and w, dz and x -- and out: NULL, or slots that the
- * forward and the input-grad raise by the largest |output| they write, h where there is an activation).  Launches whose
- * ranges are all given and whose operands have 16-byte rows run on the fp16 matrix cores with each operand element
- * scaled and split into two fp16 parts (fp32 accuracy, csrc/gemm_f16.hpp); any other launch is the plain entry point's,
- * followed by a pass over its outputs where `out` is given.  flags as above. */
+/* The three GEMMs with the operands' ranges known (ranges: one per problem, in the problems' order; a / b: the slots of the
+ * first and the second operand -- x and w, dz and w, dz and x -- and out: NULL, or slots that the forward and the
+ * input-grad raise by the |output| they write, h where there is an activation).  Launches whose ranges are all given and
+ * whose operands have 16-byte rows run on the fp16 matrix cores with each operand element scaled and split into two fp16
+ * parts (fp32 accuracy, csrc/gemm_f16.hpp); a problem of theirs with an operand whose parts lie more than 2^28 apart, that
+ * holds an infinity or reaches 2^61 runs in three bf16 parts instead, as the plain entry point's kernels do, decided on the
+ * device; any other launch is the plain entry point's, followed by a pass over its outputs where `out` is given.  flags as
+ * above. */
 typedef struct ppo_gemm_range {
   const uint32_t* a;
   const uint32_t* b;
@@ -453,13 +461,15 @@ int ppo_gauss_ppo_head(const ppo_loss_args* args, const ppo_policy_head* head, v
                        size_t workspace_bytes, float* d_std_param, ppo_device_state* state, int32_t adaptive,
                        double desired_kl, double* trace, int32_t trace_rows, ppo_stream_t stream);
 
-/* The same, also raising the slots (PPO_AMAX_WORDS each, NULL: not wanted) of what it writes by their largest
- * magnitudes: dz_actor, dz_critic and the loss arguments' d_mean and d_value. */
+/* The same, also raising the slots (PPO_AMAX_WORDS each) of what it writes: dz_actor, dz_critic and the loss arguments'
+ * d_mean and d_value.  h_actor, h_critic: the slots of the hidden layers it reads. */
 typedef struct ppo_head_ranges {
   uint32_t* dz_actor;
   uint32_t* dz_critic;
   uint32_t* d_mean;
   uint32_t* d_value;
+  const uint32_t* h_actor;
+  const uint32_t* h_critic;
 } ppo_head_ranges;
 int ppo_gauss_ppo_head_ranged(const ppo_loss_args* args, const ppo_policy_head* head, const ppo_head_ranges* ranges,
                               void* workspace, size_t workspace_bytes, float* d_std_param, ppo_device_state* state,

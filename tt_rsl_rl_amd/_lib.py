@@ -62,7 +62,7 @@ MAX_AMAX_ITEMS = 16
 
 class AmaxItem(C.Structure):
     _fields_ = [("x", C.c_void_p), ("ld", i64), ("rows", i64), ("cols", i32), ("least", C.c_float),
-                ("slots", C.c_void_p)]
+                ("slots", C.c_void_p), ("coarse", i32), ("reserved", i32), ("source", C.c_void_p * 2)]
 
 
 class GemmRange(C.Structure):
@@ -146,7 +146,8 @@ class PolicyHead(C.Structure):
 
 
 class HeadRanges(C.Structure):
-    _fields_ = [("dz_actor", C.c_void_p), ("dz_critic", C.c_void_p), ("d_mean", C.c_void_p), ("d_value", C.c_void_p)]
+    _fields_ = [("dz_actor", C.c_void_p), ("dz_critic", C.c_void_p), ("d_mean", C.c_void_p), ("d_value", C.c_void_p),
+                ("h_actor", C.c_void_p), ("h_critic", C.c_void_p)]
 
 
 class DeviceState(C.Structure):
@@ -234,7 +235,7 @@ _SIGNATURES = [
                                        C.c_size_t, C.c_void_p]),
     ("ppo_linear_bwd_dw_ex", C.c_int, [C.POINTER(LinearBwdDwProblem), i32, i64, i32, C.c_void_p, C.c_size_t, f32p,
                                        C.POINTER(GradRange), i32, C.c_void_p, C.c_void_p]),
-    ("ppo_amax", C.c_int, [C.POINTER(AmaxItem), i32, C.c_void_p, i64, C.c_void_p]),
+    ("ppo_amax", C.c_int, [C.POINTER(AmaxItem), i32, C.c_void_p, i64, i32, C.c_void_p]),
     ("ppo_linear_fwd_ranged", C.c_int, [C.POINTER(LinearFwdProblem), C.POINTER(GemmRange), i32, i64, i32, i32,
                                         C.c_void_p]),
     ("ppo_linear_bwd_dx_ranged", C.c_int, [C.POINTER(LinearBwdDxProblem), C.POINTER(GemmRange), i32, i64, i32, i32,

@@ -1,4 +1,6 @@
-// Largest magnitudes of tensors, as the kernels that write them leave them and the fp16x3 GEMMs read them.
+// Ranges of tensors, as the kernels that write them leave them and the fp16x3 GEMMs read them.  A slot's first word is the
+// largest magnitude (fp32 bits), its second the smallest among the nonzero largest magnitudes of the tensor's parts, as
+// part_code() of it (0: no such part).
 #pragma once
 
 #include "common.hpp"
@@ -30,12 +32,47 @@ __device__ __forceinline__ int amax_exponent(uint32_t u) {
 }
 __device__ __forceinline__ float pow2(int e) { return __builtin_bit_cast(float, static_cast<uint32_t>(e + 127) << 23); }
 
-// The wave's largest magnitude into the tensor's slots.
-__device__ __forceinline__ void amax_publish(uint32_t* slots, float m, int lane, int slot) {
-  const uint32_t u = wave_max(__builtin_bit_cast(uint32_t, m));
-  if (lane == 0) atomicMax(slots + (slot & (kAmaxSlots - 1)) * kAmaxStride, u);
+// The second word for a part whose largest magnitude has the bits u: larger for a smaller part (an atomic maximum finds the
+// smallest), and as a float negative, so that the words' largest float is the first word's.
+__device__ __forceinline__ uint32_t part_code(uint32_t u) { return u == 0 ? 0u : 0x80000000u | (0x7f800000u - u); }
+
+// A tensor as fp16x3 operand.  Scaled by its largest magnitude, an element is held to 2^-50 of that, so one part far above
+// the others (a sentinel in one row, a column of another unit) would cost the others their digits: to 2^-22 of a part 2^28
+// below the largest, whence kMaxSpread.  The parts of the inputs and the weights are single rows and columns, those of
+// activations and gradients the tiles of the waves that write them (16 to 64 rows): an outlier there comes of one in the
+// inputs or the weights, which amax_publish hands on, or of single rows of the loss.  Operands beyond it, with an infinity, or so large (2^61) that the two scales taken
+// out one after the other could overflow in between, are multiplied in three bf16 parts, which have fp32's exponents.
+constexpr int kMaxSpread = 28, kMaxExponent = 127 + 60;
+struct Range {
+  uint32_t top, low;
+  __device__ __forceinline__ bool narrow() const {
+    const int smallest = low == 0 ? 255 : static_cast<int>((0x7f800000u - (low & 0x7fffffffu)) >> 23);
+    return static_cast<int>(top >> 23) <= kMaxExponent && static_cast<int>(top >> 23) - smallest <= kMaxSpread;
+  }
+};
+__device__ __forceinline__ Range load_range(const uint32_t* slots, int lane) {
+  const uint2 u = *reinterpret_cast<const uint2*>(slots + lane * kAmaxStride);
+  return Range{wave_max(u.x), wave_max(u.y)};
 }
 
+// A wave's range into the tensor's slots.
+__device__ __forceinline__ void publish_range(uint32_t* slots, uint32_t top, uint32_t low, int lane, int slot) {
+  if (lane != 0 || top == 0) return;
+  uint32_t* const w = slots + (slot & (kAmaxSlots - 1)) * kAmaxStride;
+  atomicMax(w, top);
+  atomicMax(w + 1, low);
+}
+
+// The same where the wave's values are one part.  wide: the tensor comes of one that is not narrow, so that outliers may lie
+// in every part: it counts as not narrow itself, and so does what follows from it.
+constexpr uint32_t kWideCode = 0x80000000u | (0x7f800000u - 1u);
+__device__ __forceinline__ void amax_publish(uint32_t* slots, float m, bool wide, int lane, int slot) {
+  const uint32_t u = wave_max(__builtin_bit_cast(uint32_t, m));
+  publish_range(slots, u, wide ? kWideCode : part_code(u), lane, slot);
+}
+__device__ __forceinline__ bool wide_source(const uint32_t* slots, int lane) {
+  return slots != nullptr && !load_range(slots, lane).narrow();
+}
 
 // m = max(m, |a|, |b|); a NaN does not count.
 __device__ __forceinline__ void raise2(float& m, float a, float b) {

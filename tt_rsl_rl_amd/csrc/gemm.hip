@@ -405,12 +405,18 @@ int launch_nt_f16(Group& g, int count, hipStream_t s, const char* name) {
     if (bn == 64) return go(gemm_nt_f16_kernel<64, 2, 4, EPI, BKM, AR>, 256);
     return go(gemm_nt_f16_kernel<128, 2, 3, EPI, BKM, AR>, 256);
   } else {
-  if (bn == 64) return go(gemm_nt_f16_kernel<64, 2, 3, EPI, BKM, AR>, 256);
+  // (then the problems it left: gemm_nt_wide_kernel)
+  auto both = [&](auto kernel, int threads, auto wide) {
+    if (int rc = go(kernel, threads)) return rc;
+    hipLaunchKernelGGL(wide, dim3(std::min(blocks, device_info().cus)), dim3(512), 0, s, g, blocks);
+    return check_launch(name);
+  };
+  if (bn == 64) return both(gemm_nt_f16_kernel<64, 2, 3, EPI, BKM, AR>, 256, gemm_nt_wide_kernel<64, EPI, BKM>);
   // 128 x 128: eight waves of 32 x 64 (128 registers, four waves per SIMD) for the forward, whose epilogue's activation
   // then overlaps other waves' products (512 -> 256 features: 56 us against 63 with four waves of 64 x 64, 240 -> 512:
   // 66 against 73); the input-grad's longer staging and epilogue do not fit 128 registers (74 against 69 us)
-  if constexpr (BKM) return go(gemm_nt_f16_kernel<128, 2, 2, EPI, BKM, AR>, 256);
-  else return go(gemm_nt_f16_kernel<128, 4, 4, EPI, BKM, AR>, 512);
+  if constexpr (BKM) return both(gemm_nt_f16_kernel<128, 2, 2, EPI, BKM, AR>, 256, gemm_nt_wide_kernel<128, EPI, BKM>);
+  else return both(gemm_nt_f16_kernel<128, 4, 4, EPI, BKM, AR>, 512, gemm_nt_wide_kernel<128, EPI, BKM>);
   }
 }
 
@@ -430,73 +436,119 @@ int launch_tn_f16(Group& g, int count, hipStream_t s, const char* name) {
   }
   if (blocks == 0) return PPO_OK;
   hipLaunchKernelGGL((gemm_tn_f16_kernel<2, OCC, AR>), dim3(blocks), dim3(256), 0, s, g);
-  return check_launch(name);
+  if (int rc = check_launch(name)) return rc;
+  if (AR == ARITH_F16X3) {  // then the problems it left
+    hipLaunchKernelGGL(gemm_tn_wide_kernel, dim3(std::min(blocks, device_info().cus)), dim3(512), 0, s, g, blocks);
+    return check_launch(name);
+  }
+  return PPO_OK;
 }
 
-// Largest magnitudes of a few tensors: block b of kAmaxSlots per item writes slot b (or raises it), 64 rows apart;
-// the last grid row clears the caller's words.
+// Ranges of a few tensors: one block row per item, the last grid row clears the caller's words.  A block takes `chunk` rows
+// of an item, its waves whole rows (or as many side by side as 64 lanes of four columns hold).  The parts are each row's up
+// to 256 columns (coarse items: a wave's rows at a time) and each column's rows within a block.
 struct AmaxGroup {
   ppo_amax_item it[PPO_MAX_AMAX_ITEMS];
-  int32_t count, raise;
+  int32_t count;
+  int32_t raise;  // blocks beyond kAmaxSlots share slots, raised from what they hold; else block b writes slot b
   uint32_t* clear;
   int64_t clear_words;
 };
+constexpr int kAmaxRows = 16;  // per block at least
 __global__ __launch_bounds__(256) void amax_kernel(const AmaxGroup g) {
-  const int b = blockIdx.x;
+  constexpr int kPanel = 256, kUnroll = 4;
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (static_cast<int>(blockIdx.y) == g.count) {
-    for (int64_t i = int64_t(b) * 256 + threadIdx.x; i < g.clear_words; i += int64_t(kAmaxSlots) * 256) g.clear[i] = 0;
+    for (int64_t i = int64_t(b) * 256 + tid; i < g.clear_words; i += int64_t(gridDim.x) * 256) g.clear[i] = 0;
     return;
   }
   const ppo_amax_item& T = g.it[blockIdx.y];
-  float m = T.least;
-  auto take = [&](float x) {
-    x = fabsf(x);
-    if (x < __builtin_inff()) m = fmaxf(m, x);
-  };
+  const int64_t chunk = max(ceil_div(T.rows, static_cast<int64_t>(gridDim.x)), static_cast<int64_t>(kAmaxRows));
+  const int64_t r0 = b * chunk, r1 = min(T.rows, r0 + chunk);
   const bool vec = reinterpret_cast<uintptr_t>(T.x) % 16 == 0 && T.ld % 4 == 0;
-  const int q4 = vec ? T.cols >> 2 : 0;  // 16-byte pieces of a row, then its last columns one by one
-  const int rest = T.cols - 4 * q4;
-  const int64_t pieces = T.rows * q4, step = int64_t(kAmaxSlots) * 256;
-  for (int64_t i = int64_t(b) * 256 + threadIdx.x; i < pieces; i += 4 * step) {
-    f32x4 v[4];
+  __shared__ float s_col[4][kPanel];
+  __shared__ uint32_t s_top[4], s_low[4];
+  uint32_t top = __builtin_bit_cast(uint32_t, T.least), low = 0;
+  for (int c0 = 0; c0 < T.cols && r0 < r1; c0 += kPanel) {
+    const int width = min(T.cols - c0, kPanel);
+    int lanes = 1;  // per row
+    while (4 * lanes < width) lanes *= 2;
+    const int sub = lane / lanes, rows = 64 / lanes, col = 4 * (lane & (lanes - 1)), left = width - col;
+    float cm[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int64_t r = r0 + wave * rows; r < r1; r += 4 * kUnroll * rows) {
+      float v[kUnroll][4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t k = min(i + j * step, pieces - 1);
-      v[j] = *reinterpret_cast<const f32x4*>(T.x + (k / q4) * T.ld + 4 * (k % q4));
+      for (int u = 0; u < kUnroll; ++u) {  // (rows past the block's: its last one again)
+        const float* const row = T.x + min(r + sub + 4 * u * rows, r1 - 1) * T.ld + c0 + col;
+        if (vec && left >= 4) {
+          const f32x4 q = *reinterpret_cast<const f32x4*>(row);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[u][e] = q[e];
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[u][e] = e < left ? row[e] : 0.0f;
+        }
+      }
+      float some = 0.0f;
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        float rm = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x = fabsf(v[u][e]);
+          const float q = x < __builtin_inff() ? x : 0.0f;
+          cm[e] = fmaxf(cm[e], q);
+          rm = fmaxf(rm, q);
+        }
+        some = fmaxf(some, rm);
+        if (!T.coarse) {
+          for (int o = 1; o < lanes; o *= 2) rm = fmaxf(rm, __shfl_xor(rm, o, 64));
+          low = max(low, part_code(__builtin_bit_cast(uint32_t, rm)));
+        }
+      }
+      const uint32_t u = wave_max(__builtin_bit_cast(uint32_t, some));
+      top = max(top, u);
+      if (T.coarse) low = max(low, part_code(u));
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) take(v[j][c]);
+    for (int e = 0; e < 4; ++e) {
+      for (int o = lanes; o < 64; o *= 2) cm[e] = fmaxf(cm[e], __shfl_xor(cm[e], o, 64));
+      if (lane < lanes) s_col[wave][col + e] = cm[e];
+    }
+    __syncthreads();
+    if (tid < width) {
+      const float m = fmaxf(fmaxf(s_col[0][tid], s_col[1][tid]), fmaxf(s_col[2][tid], s_col[3][tid]));
+      low = max(low, part_code(__builtin_bit_cast(uint32_t, m)));
+    }
+    __syncthreads();
   }
-  if (rest > 0)
-    for (int64_t i = int64_t(b) * 256 + threadIdx.x; i < T.rows * rest; i += step)
-      take(T.x[(i / rest) * T.ld + 4 * q4 + i % rest]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  __shared__ float red[4];
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  low = wave_max(low);
+  if (wide_source(T.source[0], lane) || wide_source(T.source[1], lane)) low = kWideCode;
+  if (lane == 0) {
+    s_top[wave] = top;
+    s_low[wave] = low;
+  }
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  if (g.raise) atomicMax(T.slots + b * kAmaxStride, __builtin_bit_cast(uint32_t, m));
-  else T.slots[b * kAmaxStride] = __builtin_bit_cast(uint32_t, m);
-}
-
-// A contiguous tensor counts as one row.
-void add_amax(AmaxGroup& g, const float* x, int64_t ld, int64_t rows, int cols, uint32_t* slots) {
-  ppo_amax_item& t = g.it[g.count++];
-  t.x = x; t.slots = slots;
-  t.rows = rows; t.cols = cols; t.ld = ld;
-  if (ld == cols && rows * cols <= INT32_MAX) {
-    t.cols = static_cast<int32_t>(rows * cols);
-    t.ld = (t.cols + 3) / 4 * 4;
-    t.rows = 1;
+  if (tid != 0) return;
+  top = max(max(s_top[0], s_top[1]), max(s_top[2], s_top[3]));
+  low = max(max(s_low[0], s_low[1]), max(s_low[2], s_low[3]));
+  if (g.raise) {
+    publish_range(T.slots, top, low, 0, b);
+  } else {
+    T.slots[b * kAmaxStride] = top;
+    T.slots[b * kAmaxStride + 1] = low;
   }
 }
 
+// Blocks per item: one per slot where they write; where they raise, enough to fill the chip with rows in flight (98,304 x
+// 235: 97 us with 64 blocks).
 int launch_amax(const AmaxGroup& g, hipStream_t s, const char* who) {
-  hipLaunchKernelGGL(amax_kernel, dim3(kAmaxSlots, g.count + (g.clear_words > 0 ? 1 : 0)), dim3(256), 0, s, g);
+  int64_t rows = 0;
+  for (int i = 0; i < g.count; ++i) rows = std::max(rows, g.it[i].rows);
+  const int64_t blocks = g.raise ? std::min<int64_t>(std::max<int64_t>(ceil_div(rows, 4 * kAmaxRows), kAmaxSlots), 1024)
+                                 : kAmaxSlots;
+  hipLaunchKernelGGL(amax_kernel, dim3(static_cast<unsigned>(blocks), g.count + (g.clear_words > 0 ? 1 : 0)), dim3(256), 0, s,
+                     g);
   return check_launch(who);
 }
 
@@ -571,15 +623,23 @@ void set_range(Problem& p, const ppo_gemm_range* ranges, int i) {
   p.amax_c = ranges[i].out;
 }
 
-// After a launch of kernels that do not track their outputs' largest magnitude: a pass over the outputs that want it.
+// After a launch of kernels that do not track their outputs' range: a pass over the outputs that want it.
 int raise_outputs(const Group& g, int count, bool c2, hipStream_t s, const char* who) {
   AmaxGroup ag{};
   ag.raise = 1;
   for (int i = 0; i < count; ++i) {
     const Problem& p = g.p[i];
     if (p.amax_c == nullptr) continue;
-    const float* x = c2 && p.C2 != nullptr ? p.C2 : p.C;
-    add_amax(ag, x, x == p.C2 ? p.ldc2 : p.ldc, p.M, p.N, p.amax_c);
+    const bool h = c2 && p.C2 != nullptr;
+    ppo_amax_item& t = ag.it[ag.count++];
+    t.x = h ? p.C2 : p.C;
+    t.ld = h ? p.ldc2 : p.ldc;
+    t.rows = p.M;
+    t.cols = p.N;
+    t.slots = p.amax_c;
+    t.coarse = 1;
+    t.source[0] = p.amax_a;
+    t.source[1] = p.amax_b;
   }
   return ag.count > 0 ? launch_amax(ag, s, who) : PPO_OK;
 }
@@ -839,7 +899,7 @@ extern "C" int ppo_linear_bwd_dx_ranged(const ppo_linear_bwd_dx_problem* problem
                  "ppo_linear_bwd_dx_ranged", flags, ranges);
 }
 
-extern "C" int ppo_amax(const ppo_amax_item* items, int32_t count, uint32_t* clear, int64_t clear_words,
+extern "C" int ppo_amax(const ppo_amax_item* items, int32_t count, uint32_t* clear, int64_t clear_words, int32_t raise,
                         ppo_stream_t stream) {
   PPO_REQUIRE(count >= 0 && count <= PPO_MAX_AMAX_ITEMS && (count == 0 || items != nullptr),
               "ppo_amax: count=%d outside [0, %d]", count, PPO_MAX_AMAX_ITEMS);
@@ -848,10 +908,13 @@ extern "C" int ppo_amax(const ppo_amax_item* items, int32_t count, uint32_t* cle
   AmaxGroup g{};
   for (int i = 0; i < count; ++i) {
     const ppo_amax_item& q = items[i];
-    PPO_REQUIRE(q.x && q.slots && q.rows > 0 && q.cols > 0 && q.ld >= q.cols && q.least >= 0.0f, "ppo_amax: item %d", i);
-    add_amax(g, q.x, q.ld, q.rows, q.cols, q.slots);
-    g.it[i].least = q.least;
+    PPO_REQUIRE(q.x && q.slots && reinterpret_cast<uintptr_t>(q.slots) % 8 == 0 && q.rows > 0 && q.cols > 0 &&
+                    q.ld >= q.cols && q.least >= 0.0f &&
+                    reinterpret_cast<uintptr_t>(q.source[0]) % 8 == 0 && reinterpret_cast<uintptr_t>(q.source[1]) % 8 == 0,
+                "ppo_amax: item %d", i);
+    g.it[g.count++] = q;
   }
+  g.raise = raise;
   g.clear = clear;
   g.clear_words = clear_words;
   if (g.count == 0 && clear_words == 0) return PPO_OK;

@@ -91,9 +91,9 @@ struct Problem {
   const float* vec;  // bias [N]
   const float* aux;  // ELU'-source z_prev [M, N]
   double* colsum;    // [splits, M] sums of A over each split's k range (fp64: bias grads cancel heavily)
-  const uint32_t* amax_a;  // fp16x3 kernels: the operands' largest magnitudes (PPO_AMAX_SLOTS words each)
+  const uint32_t* amax_a;  // fp16x3 kernels: the operands' ranges (PPO_AMAX_WORDS words each)
   const uint32_t* amax_b;
-  uint32_t* amax_c;        // where the NT kernels leave the output's (null: not wanted)
+  uint32_t* amax_c;        // where the NT kernels leave the output's range (null: not wanted)
   int64_t lda, ldb, ldc, ldc2, ldaux;
   int64_t partial_stride;  // floats between split partials of C
   int32_t M, N, K;
@@ -310,8 +310,9 @@ struct TileCoord {
   int pi, split, tm, tn;
 };
 
-__device__ inline TileCoord locate(const Group& g) {
-  const int b = g.xcds > 1 ? xcd_remap(blockIdx.x, gridDim.x, g.xcds) : static_cast<int>(blockIdx.x);
+// Tile `block` of `blocks`.
+__device__ inline TileCoord locate_at(const Group& g, int block, int blocks) {
+  const int b = g.xcds > 1 ? xcd_remap(block, blocks, g.xcds) : block;
   int pi = 0;
 #pragma unroll
   for (int i = 1; i < PPO_MAX_LINEAR_PROBLEMS; ++i) {
@@ -328,6 +329,8 @@ __device__ inline TileCoord locate(const Group& g) {
   t.tn = r - t.tm * P.tiles_n;
   return t;
 }
+
+__device__ inline TileCoord locate(const Group& g) { return locate_at(g, blockIdx.x, gridDim.x); }
 
 // Direct global->LDS copy through a raw buffer: every lane moves BYTES from byte offset `off` of buffer r to
 // lds_wave + lane * BYTES (lds_wave wave-uniform), and an offset at or past the buffer's record count reads zeros.
@@ -2020,12 +2023,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(OCC, O
   if (kt < nk) step(kt, cs, RB_EVEN, 1 - RB_EVEN);
   float* const patch = reinterpret_cast<float*>(lds) + wave * 32 * PS;  // every wave is past the last barrier
   if constexpr (epi_fwd_act(EPI)) {
-    const float m = nt_pipe_epilogue_t<TM, TN, EPI, epi_generic(EPI), false, true>(P, acc, row0 + wm * 64,
-                                                                                  col0 + wn * (BN / 2), patch, lane);
-    if (P.amax_c != nullptr) amax_publish(P.amax_c, m, lane, 4 * blockIdx.x + wave);
-  } else {
-    nt_pipe_epilogue<TM, TN, EPI>(P, acc, row0 + wm * 64, col0 + wn * (BN / 2), patch, lane);
+    if (P.amax_c != nullptr) {
+      const float m = nt_pipe_epilogue_t<TM, TN, EPI, epi_generic(EPI), false, true>(P, acc, row0 + wm * 64,
+                                                                                    col0 + wn * (BN / 2), patch, lane);
+      const bool wide = wide_source(P.amax_a, lane) || wide_source(P.amax_b, lane);
+      amax_publish(P.amax_c, m, wide, lane, 4 * blockIdx.x + wave);
+      return;
+    }
   }
+  nt_pipe_epilogue<TM, TN, EPI>(P, acc, row0 + wm * 64, col0 + wn * (BN / 2), patch, lane);
 }
 
 // 16-byte direct loads need a 16-byte aligned base and a leading dimension that is a multiple of 4.

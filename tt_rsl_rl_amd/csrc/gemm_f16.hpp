@@ -39,12 +39,14 @@ __device__ __forceinline__ void split_f16x2(float x0, float x1, float s, float k
 enum Arith : int {
   ARITH_F16X3 = 0,  // two fp16 parts, three products, two accumulators
   ARITH_BF16 = 1,   // bf16 operands (PPO_GEMM_BF16_OPERANDS): one part, one product
+  ARITH_BF16X6 = 2, // three bf16 parts, six products (gemm_core.hpp): the problems whose operands span too much for fp16x3
 };
 
 template <int AR>
 struct Parts {
-  static constexpr int planes = AR == ARITH_F16X3 ? 2 : 1;
+  static constexpr int planes = AR == ARITH_F16X3 ? 2 : AR == ARITH_BF16X6 ? 3 : 1;
   static constexpr int accs = AR == ARITH_F16X3 ? 2 : 1;
+  static constexpr int products = AR == ARITH_F16X3 ? 3 : AR == ARITH_BF16X6 ? 6 : 1;
 };
 
 // Splits 4 consecutive elements and writes each part's 8 bytes (at c and c + plane).
@@ -56,6 +58,13 @@ __device__ __forceinline__ void stage_piece(const f32x4& v, float s, float k2048
     split_f16x2(v[2], v[3], s, k2048, h[1], l[1]);
     *reinterpret_cast<u32x2*>(c) = u32x2{h[0], h[1]};
     *reinterpret_cast<u32x2*>(c + plane) = u32x2{l[0], l[1]};
+  } else if constexpr (AR == ARITH_BF16X6) {
+    uint32_t h[2], m[2], l[2];
+    split_bf16x3(v[0], v[1], h[0], m[0], l[0]);
+    split_bf16x3(v[2], v[3], h[1], m[1], l[1]);
+    *reinterpret_cast<u32x2*>(c) = u32x2{h[0], h[1]};
+    *reinterpret_cast<u32x2*>(c + plane) = u32x2{m[0], m[1]};
+    *reinterpret_cast<u32x2*>(c + 2 * plane) = u32x2{l[0], l[1]};
   } else {
     *reinterpret_cast<u32x2*>(c) = u32x2{round_bf16x2(v[0], v[1]), round_bf16x2(v[2], v[3])};
   }
@@ -75,6 +84,7 @@ template <int AR, int TM, int TN, bool FLIP>
 __device__ __forceinline__ void products(f32x16 (&acc)[Parts<AR>::accs][TM][TN], const u32x4 (&fa)[TM][Parts<AR>::planes],
                                          const u32x4 (&fb)[TN][Parts<AR>::planes], int t) {
   constexpr int pa[3] = {1, 0, 0}, pb[3] = {0, 1, 0};
+  constexpr int pa6[6] = {2, 1, 0, 1, 0, 0}, pb6[6] = {0, 1, 2, 0, 1, 0};
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -82,6 +92,9 @@ __device__ __forceinline__ void products(f32x16 (&acc)[Parts<AR>::accs][TM][TN],
       if constexpr (AR == ARITH_F16X3) {
         f32x16& c = acc[t < 2 ? 1 : 0][i][j];
         c = FLIP ? mfma16<AR>(fb[j][pb[t]], fa[i][pa[t]], c) : mfma16<AR>(fa[i][pa[t]], fb[j][pb[t]], c);
+      } else if constexpr (AR == ARITH_BF16X6) {
+        f32x16& c = acc[0][i][j];
+        c = FLIP ? mfma16<AR>(fb[j][pb6[t]], fa[i][pa6[t]], c) : mfma16<AR>(fa[i][pa6[t]], fb[j][pb6[t]], c);
       } else {
         f32x16& c = acc[0][i][j];
         c = FLIP ? mfma16<AR>(fb[j][0], fa[i][0], c) : mfma16<AR>(fa[i][0], fb[j][0], c);
@@ -112,18 +125,22 @@ __device__ __forceinline__ void join_acc(f32x16 (&acc)[Parts<AR>::accs][TM][TN])
 // LDS planes: [row][32 k] halves, the 16-byte chunk index XOR-ed with (row / 4) % 4 (the 16 rows that a ds_read_b128
 // serves at a time fall on all 64 banks); BKM's B: [32 k][BN n], as the weight-grad's.
 // ------------------------------------------------------------------------------------------------------------------
-template <int BN, int WM, int OCC, int EPI, bool BKM, int AR>
-__global__ __launch_bounds__(WM * 128) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemm_nt_f16_kernel(
-    const Group g) {
+template <int BN, int WM, int AR>
+struct NtF16 {
+  static constexpr int stage = Parts<AR>::planes * (128 + BN) * 32 * 2;
+  static constexpr int patch = WM * 2 * 32 * 36 * 4;
+  static constexpr int lds = 2 * stage > patch ? 2 * stage : patch;
+};
+
+// slot: of the output's range.  fp16x3: a problem with an operand that is not narrow() is left to the launch after it.
+template <int BN, int WM, int EPI, bool BKM, int AR>
+__device__ __forceinline__ void nt_f16_tile(const Group& g, const TileCoord tc, unsigned char* lds, int slot) {
   static_assert(EPI == EPI_BIAS || epi_fwd_act(EPI) || epi_act_grad(EPI) || EPI == EPI_STORE, "NT epilogues");
   constexpr int BM = 128, BK = 32, THREADS = WM * 128, TM = 4 / WM, TN = BN / 64, NPL = Parts<AR>::planes;
   constexpr int PLANE_A = BM * BK * 2, PLANE_B = BN * BK * 2;
-  constexpr int STAGE = NPL * (PLANE_A + PLANE_B);
+  constexpr int STAGE = NtF16<BN, WM, AR>::stage;
   constexpr int PS = 36;
-  constexpr int PATCH = (THREADS / 64) * 32 * PS * 4, LDS = 2 * STAGE > PATCH ? 2 * STAGE : PATCH;
-  __shared__ __align__(16) unsigned char lds[LDS];
 
-  const TileCoord tc = locate(g);
   const Problem& P = g.p[tc.pi];
   const int64_t lda = P.lda, ldb = P.ldb;
   const int row0 = tc.tm * BM, col0 = tc.tn * BN;
@@ -197,9 +214,10 @@ __global__ __launch_bounds__(WM * 128) __attribute__((amdgpu_waves_per_eu(OCC, O
   for (int o = 0; o < NA + NB; ++o) load_piece(0, o);
   int ea = 0, eb = 0;
   if constexpr (AR == ARITH_F16X3) {
-    const uint32_t ua = P.amax_a[lane * kAmaxStride], ub = P.amax_b[lane * kAmaxStride];
-    ea = amax_exponent(wave_max(ua));
-    eb = amax_exponent(wave_max(ub));
+    const Range ra = load_range(P.amax_a, lane), rb = load_range(P.amax_b, lane);
+    if (!ra.narrow() || !rb.narrow()) return;
+    ea = amax_exponent(ra.top);
+    eb = amax_exponent(rb.top);
   }
   const float sa = pow2(ea), sb = pow2(eb);
   const float k2048 = 2048.0f;
@@ -246,7 +264,7 @@ __global__ __launch_bounds__(WM * 128) __attribute__((amdgpu_waves_per_eu(OCC, O
     }
     lds_barrier();
   }
-  constexpr int NT = AR == ARITH_F16X3 ? 3 : 1;
+  constexpr int NT = Parts<AR>::products;
   u32x4 fa[TM][NPL], fb[TN][NPL];
   auto read = [&](const unsigned char* st, int kg) __attribute__((always_inline)) {
 #pragma unroll
@@ -291,12 +309,46 @@ __global__ __launch_bounds__(WM * 128) __attribute__((amdgpu_waves_per_eu(OCC, O
   join_acc<AR, TM, TN>(acc);
   float* const patch = reinterpret_cast<float*>(lds) + wave * 32 * PS;  // every wave is past the last barrier
   const int rw = row0 + wm * (128 / WM), cw = col0 + wn * (BN / 2);
-  if constexpr (AR == ARITH_F16X3) {
+  if constexpr (AR != ARITH_BF16) {
     const float m = nt_pipe_epilogue_t<TM, TN, EPI, epi_generic(EPI), true>(P, acc[0], rw, cw, patch, lane,
                                                                                pow2(-ea), pow2(-eb));
-    if (P.amax_c != nullptr) amax_publish(P.amax_c, m, lane, (THREADS / 64) * blockIdx.x + wave);
+    if (P.amax_c != nullptr) amax_publish(P.amax_c, m, AR == ARITH_BF16X6, lane, (THREADS / 64) * slot + wave);
   } else {
     nt_pipe_epilogue<TM, TN, EPI>(P, acc[0], rw, cw, patch, lane);
+  }
+}
+
+template <int BN, int WM, int OCC, int EPI, bool BKM, int AR>
+__global__ __launch_bounds__(WM * 128) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemm_nt_f16_kernel(
+    const Group g) {
+  __shared__ __align__(16) unsigned char lds[NtF16<BN, WM, AR>::lds];
+  nt_f16_tile<BN, WM, EPI, BKM, AR>(g, locate(g), lds, blockIdx.x);
+}
+
+// The problems (bit i: problem i) with an operand that fp16x3 does not take.
+__device__ __forceinline__ uint32_t wide_problems(const Group& g, int lane) {
+  uint32_t wide = 0;
+  for (int i = 0; i < g.count; ++i) {
+    const Range ra = load_range(g.p[i].amax_a, lane), rb = load_range(g.p[i].amax_b, lane);
+    if (!ra.narrow() || !rb.narrow()) wide |= 1u << i;
+  }
+  return wide;
+}
+
+// The launch after an fp16x3 one: its wide problems, on the same tiles in bf16x6, a block per compute unit going through
+// them; nothing where there are none (the usual case: a launch of 3 us).  Three planes take 96 KB of LDS: one block per
+// compute unit, eight waves.
+template <int BN, int EPI, bool BKM>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_nt_wide_kernel(const Group g,
+                                                                                                      int tiles) {
+  __shared__ __align__(16) unsigned char lds[NtF16<BN, 4, ARITH_BF16X6>::lds];
+  const uint32_t wide = wide_problems(g, threadIdx.x & 63);
+  if (wide == 0) return;
+  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const TileCoord tc = locate_at(g, t, tiles);
+    if (((wide >> tc.pi) & 1) == 0) continue;
+    nt_f16_tile<BN, 4, EPI, BKM, ARITH_BF16X6>(g, tc, lds, t);
+    __syncthreads();  // (the next tile's stages lie where this one's patches are)
   }
 }
 
@@ -366,9 +418,10 @@ __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, 
   for (int o = 0; o < NA + NB; ++o) load_piece(0, o);
   int ea = 0, eb = 0;
   if constexpr (AR == ARITH_F16X3) {
-    const uint32_t ua = P.amax_a[lane * kAmaxStride], ub = P.amax_b[lane * kAmaxStride];
-    ea = amax_exponent(wave_max(ua));
-    eb = amax_exponent(wave_max(ub));
+    const Range ra = load_range(P.amax_a, lane), rb = load_range(P.amax_b, lane);
+    if (!ra.narrow() || !rb.narrow()) return;
+    ea = amax_exponent(ra.top);
+    eb = amax_exponent(rb.top);
   }
   const float sa = pow2(ea), sb = pow2(eb);
   const float k2048 = 2048.0f;
@@ -418,7 +471,7 @@ __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, 
     }
     lds_barrier();
   }
-  constexpr int NT = AR == ARITH_F16X3 ? 3 : 1;
+  constexpr int NT = Parts<AR>::products;
   u32x4 fa[TM][NPL], fb[TN][NPL];
   auto read = [&](const unsigned char* st, int kg) __attribute__((always_inline)) {
 #pragma unroll
@@ -499,6 +552,24 @@ __global__ __launch_bounds__(WM * 128) __attribute__((amdgpu_waves_per_eu(OCC, O
     tn_f16_tile<64, WM, AR>(g, tc, lds);
   } else {
     tn_f16_tile<128, WM, AR>(g, tc, lds);
+  }
+}
+
+// As gemm_nt_wide_kernel, for the weight-grad.
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tn_wide_kernel(const Group g,
+                                                                                                      int tiles) {
+  __shared__ __align__(16) unsigned char lds[2 * Parts<ARITH_BF16X6>::planes * 2 * 32 * 128 * 2];
+  const uint32_t wide = wide_problems(g, threadIdx.x & 63);
+  if (wide == 0) return;
+  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const TileCoord tc = locate_at(g, t, tiles);
+    if (((wide >> tc.pi) & 1) == 0) continue;
+    if (g.p[tc.pi].tn64) {
+      tn_f16_tile<64, 4, ARITH_BF16X6>(g, tc, lds);
+    } else {
+      tn_f16_tile<128, 4, ARITH_BF16X6>(g, tc, lds);
+    }
+    __syncthreads();
   }
 }
 

@@ -464,9 +464,11 @@ __global__ __launch_bounds__(64 * WAVES) void ppo_head_kernel(const HeadParams P
   double acc_dstd[8];
 #pragma unroll
   for (int v = 0; v < 8; ++v) acc_dstd[v] = 0.0;
-  float max_dza = 0.0f, max_dzc = 0.0f, max_dm = 0.0f, max_dv = 0.0f;
+  // what the ranges want: the largest magnitudes and the smallest of the tiles' (16 rows)
+  uint32_t top[4] = {0, 0, 0, 0}, low[4] = {0, 0, 0, 0};
 
   for (; tile < tiles; tile += stride) {
+    float max_dza = 0.0f, max_dzc = 0.0f, max_dm = 0.0f, max_dv = 0.0f;
     const int64_t row = tile * kHeadRows + m;
     const bool valid = row < R;
 
@@ -640,13 +642,26 @@ __global__ __launch_bounds__(64 * WAVES) void ppo_head_kernel(const HeadParams P
       }
     }
     if (tile + stride < tiles) head_load_tile(P, tile + stride, lane, in);
+    if (P.ranges.dz_actor != nullptr) {  // (all of them, or none)
+      const float m[4] = {max_dza, max_dzc, max_dm, max_dv};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t u = wave_max(__builtin_bit_cast(uint32_t, m[k]));
+        top[k] = max(top[k], u);
+        low[k] = max(low[k], part_code(u));
+      }
+    }
   }
 
-  const int slot = WAVES * blockIdx.x + wave;
-  if (P.ranges.dz_actor) amax_publish(P.ranges.dz_actor, max_dza, lane, slot);
-  if (P.ranges.dz_critic) amax_publish(P.ranges.dz_critic, max_dzc, lane, slot);
-  if (P.ranges.d_mean) amax_publish(P.ranges.d_mean, max_dm, lane, slot);
-  if (P.ranges.d_value) amax_publish(P.ranges.d_value, max_dv, lane, slot);
+  if (P.ranges.dz_actor != nullptr) {
+    const int slot = WAVES * blockIdx.x + wave;
+    if (wide_source(P.ranges.h_actor, lane)) low[0] = low[2] = kWideCode;
+    if (wide_source(P.ranges.h_critic, lane)) low[1] = low[3] = kWideCode;
+    publish_range(P.ranges.dz_actor, top[0], low[0], lane, slot);
+    publish_range(P.ranges.dz_critic, top[1], low[1], lane, slot);
+    publish_range(P.ranges.d_mean, top[2], low[2], lane, slot);
+    publish_range(P.ranges.d_value, top[3], low[3], lane, slot);
+  }
 
   // block partials: wave sums, the per-action std-gradient terms folded over the 16 rows of each quarter, then the
   // waves in a fixed order; column-major [cols][blocks] like ppo_loss_kernel's, for ppo_loss_finalize_kernel
@@ -864,7 +879,12 @@ extern "C" int ppo_gauss_ppo_head_ranged(const ppo_loss_args* args, const ppo_po
                   (h.value == nullptr || h.ld_value >= 1),
               "%s: rows must be 16-byte aligned with leading dimensions that are multiples of 4 floats", who);
   P.h = h;
-  if (ranges != nullptr) P.ranges = *ranges;
+  if (ranges != nullptr) {
+    PPO_REQUIRE(ranges->dz_actor && ranges->dz_critic && ranges->d_mean && ranges->d_value && ranges->h_actor &&
+                    ranges->h_critic,
+                "%s: all six ranges", who);
+    P.ranges = *ranges;
+  }
   const size_t need = ppo_head_workspace_bytes(a.rows, a.num_actions);
   PPO_REQUIRE(workspace != nullptr && workspace_bytes >= need, "%s: workspace too small (%zu < %zu)", who,
               workspace_bytes, need);

@@ -96,7 +96,7 @@ class ModelBuffers:
         self.z = None if self.from_output else [buf(w) for w in self.widths[:-1]]
         self.dz = [buf(w) for w in self.widths]
 
-        # largest-magnitude slots of h (hidden layers) and dz (all), set by the engine
+        # range slots of h (hidden layers) and dz (all), set by an engine that uses them
         self.h_max: list[torch.Tensor] = []
         self.dz_max: list[torch.Tensor] = []
 
@@ -253,44 +253,42 @@ class UpdateEngine:
         # It must not change the parameters: within a run the padded first-layer copies follow the Adam steps only
         self.step_hook = None
 
-    # -- largest magnitudes of the GEMMs' operands ----------------------------------------------------------------------
+    # -- ranges of the GEMMs' operands -----------------------------------------------------------------------------------
     def _init_ranges(self) -> None:
-        """Slots for every GEMM operand's largest |x| (ops.amax): with them the GEMMs run as fp16x3.  The table's are
-        written with the gather, the weights' at the start of every mini-batch (one small launch, which also clears
-        the activations' and gradients', raised by the kernels that write those).  Not used with bf16 operands."""
-        la, lc = self._layers()
-        n = len(la)
-        act = self._range_act = ops.new_amax(2 * (2 * n - 1) + self._extra_ranges(), self.device)
+        """Slots for every GEMM operand's range (ops.amax): with them the GEMMs run as fp16x3.  The table's are written
+        with the gather, the weights' at the start of every mini-batch (one small launch, which also clears the
+        activations' and gradients', raised by the kernels that write those).  Not used with bf16 operands."""
+        n = len(self._layers()[0])
+        act = self._range_act = ops.new_amax(2 * (2 * n - 1), self.device)
         rows = iter(act)
         for b in (self.buf_a, self.buf_c):
             b.h_max = [next(rows) for _ in range(n - 1)]
             b.dz_max = [next(rows) for _ in range(n)]
-        self._extra_max = list(rows)
-        fixed = ops.new_amax(2 + 2 * n, self.device)
-        self.xa_max, self.xc_max = fixed[0], fixed[0] if self.layout.shared_obs else fixed[1]
-        self.w_max = (list(fixed[2:2 + n]), list(fixed[2 + n:]))
-
-    def _extra_ranges(self) -> int:
-        return 0
+        self._range_table = ops.new_amax(1 if self.layout.shared_obs else 2, self.device)
+        self.xa_max, self.xc_max = self._range_table[0], self._range_table[-1]
+        weights = ops.new_amax(2 * n, self.device)
+        self.w_max = (list(weights[:n]), list(weights[n:]))
 
     @property
     def ranged(self) -> bool:
         return self.R_max >= RANGED_ROWS and not self.alg.use_mixed_precision
 
-    def _table_ranges(self, rows: int) -> None:
-        """Largest magnitudes of the first `rows` table rows' observation blocks, as wide as the first layers read
-        them."""
+    def _table_ranges(self, row0: int, rows: int) -> None:
+        """Raise the ranges of the table's observation blocks, as wide as the first layers read them, by rows
+        [row0, row0 + rows) (from row 0: cleared first)."""
         lay, alg = self.layout, self.alg
+        if row0 == 0:
+            ops.amax([], self._range_table)
         items = []
         for model, col, slots in ((alg.actor, lay.xa, self.xa_max), (alg.critic, lay.xc, self.xc_max)):
             wp = self.w0_pad.get(id(model))
             width = model.obs_dim if wp is None else wp.shape[1]
-            items.append((self.table[:rows, col:col + width], slots))
-        ops.amax(items[:1] if lay.shared_obs else items)
+            items.append((self.table[row0:row0 + rows, col:col + width], slots))
+        ops.amax(items[:1] if lay.shared_obs else items, raising=True)
 
-    def _weight_ranges(self, extra: list[tuple] = ()) -> None:
+    def _weight_ranges(self) -> None:
         items = [(lin.weight, slots) for lins, maxes in zip(self._layers(), self.w_max)
-                 for lin, slots in zip(lins, maxes)] + list(extra)
+                 for lin, slots in zip(lins, maxes)]
         clear = self._range_act
         for i in range(0, len(items), L.MAX_AMAX_ITEMS):
             ops.amax(items[i:i + L.MAX_AMAX_ITEMS], clear)
@@ -391,7 +389,7 @@ class UpdateEngine:
         for i in range(0, len(segs), L.MAX_GATHER_SEGMENTS):
             ops.gather_rows(perm, segs[i:i + L.MAX_GATHER_SEGMENTS], dst)
         if self.ranged:
-            self._table_ranges(row0 + perm.numel())
+            self._table_ranges(row0, perm.numel())
 
     def segments(self) -> list[ops.Segment]:
         """The packed table's column blocks and their storage sources ([T * N, width] views)."""
@@ -580,7 +578,8 @@ class UpdateEngine:
                          ba.dz[-2][:R], bc.dz[-2][:R], self.head_ws, std_grad,
                          alg.device_state, adaptive, alg.desired_kl, self.trace, mean=ba.out[:R],
                          value=bc.out[:R, 0],
-                         ranges=(ba.dz_max[-2], bc.dz_max[-2], ba.dz_max[-1], bc.dz_max[-1]) if self.ranged else None)
+                         ranges=(ba.dz_max[-2], bc.dz_max[-2], ba.dz_max[-1], bc.dz_max[-1], ba.h_max[-1], bc.h_max[-1])
+                         if self.ranged else None)
             tm.stop("head")
             return
         tm.start("loss")
@@ -588,7 +587,8 @@ class UpdateEngine:
         ops.ppo_loss_finalize(args, self.loss_ws, std_grad, alg.device_state, adaptive,
                               alg.desired_kl if alg.desired_kl is not None else 0.0, self.trace)
         if self.ranged:
-            ops.amax([(ba.dz[-1][:R], ba.dz_max[-1]), (bc.dz[-1][:R], bc.dz_max[-1])])
+            ops.amax([(ba.dz[-1][:R], ba.dz_max[-1]), (bc.dz[-1][:R], bc.dz_max[-1])], raising=True, coarse=True,
+                     sources=[ba.h_max[-1], bc.h_max[-1]])
         tm.stop("loss")
 
     def dx_layers(self, R: int) -> list[tuple]:
@@ -602,7 +602,8 @@ class UpdateEngine:
         for i in range(top, 0, -1):
             pa = (ba.dz[i][:R], la[i].weight, ba.act_src(i - 1, R), ba.dz[i - 1][:R])
             pc = (bc.dz[i][:R], lc[i].weight, bc.act_src(i - 1, R), bc.dz[i - 1][:R])
-            ra, rc = ((b.dz_max[i], w[i], b.dz_max[i - 1]) for b, w in zip((ba, bc), self.w_max))
+            ra, rc = ((b.dz_max[i], w[i], b.dz_max[i - 1]) for b, w in zip((ba, bc), self.w_max)) if self.ranged \
+                else (None, None)
             if (ba.act, ba.from_output) == (bc.act, bc.from_output):
                 out.append((i, [pa, pc], ba.from_output, ba.act, [ra, rc]))
             else:
@@ -887,8 +888,7 @@ class RecurrentUpdateEngine(UpdateEngine):
         la, lc = self._layers()
         return super().dx_layers(R) + [(0, [(self.buf_a.dz[0][:R], la[0].weight, None, self.seq_a.dh[:R]),
                                             (self.buf_c.dz[0][:R], lc[0].weight, None, self.seq_c.dh[:R])], False,
-                                        L.PPO_ACT_ELU, [(b.dz_max[0], w[0], None)
-                                                        for b, w in zip((self.buf_a, self.buf_c), self.w_max)])]
+                                        L.PPO_ACT_ELU, [None, None])]
 
     @property
     def can_fail(self) -> bool:

@@ -425,24 +425,28 @@ def _check_weight(w: torch.Tensor, b: torch.Tensor | None) -> tuple[int, int]:
 
 
 def new_amax(count: int, device) -> torch.Tensor:
-    """Largest-magnitude slots of `count` tensors (rows of AMAX_WORDS words), zero."""
+    """Range slots of `count` tensors (rows of AMAX_WORDS words), zero."""
     return torch.zeros(count, L.AMAX_WORDS, dtype=torch.int32, device=device)
 
 
-def amax(items: list[tuple], clear: torch.Tensor | None = None) -> None:
-    """items: (x [rows, cols] row-major view, slots[, least]): the slots' maximum becomes max |x| (or `least`, if that is
-    larger); `clear` (slots of other tensors, contiguous) is zeroed by the same launch."""
+def amax(items: list[tuple], clear: torch.Tensor | None = None, raising: bool = False, coarse: bool = False,
+         sources: list[torch.Tensor] | None = None) -> None:
+    """items: (x [rows, cols] row-major view, slots[, least]): the slots become the range of x (the maximum max |x|, or
+    `least`, if that is larger), or with `raising` are raised by it; `clear` (slots of other tensors, contiguous) is zeroed
+    by the same launch.  coarse: for the spread between parts (csrc/amax.hpp), several rows count as one.  sources: per
+    item the slots of a tensor it was computed from."""
     arr = []
-    for x, slots, *least in items:
+    for i, (x, slots, *least) in enumerate(items):
         _dev(x)
-        arr.append(L.AmaxItem(x.data_ptr(), _row_major(x, "x"), x.shape[0], x.shape[1], float(*least), _slots(slots)))
+        arr.append(L.AmaxItem(x.data_ptr(), _row_major(x, "x"), x.shape[0], x.shape[1], float(*least), _slots(slots),
+                              int(coarse), 0, (None if sources is None else _slots(sources[i]), None)))
     n = 0
     if clear is not None:
         _dev(clear, dtype=torch.int32)
         if not clear.is_contiguous():
             raise ValueError("amax: the slots to clear must be contiguous")
         n = clear.numel()
-    L.call("ppo_amax", L.array(L.AmaxItem, arr), len(arr), _ptr(clear), n, _stream())
+    L.call("ppo_amax", L.array(L.AmaxItem, arr) if arr else None, len(arr), _ptr(clear), n, int(raising), _stream())
 
 
 def _slots(t: torch.Tensor | None) -> int | None:
@@ -467,7 +471,7 @@ def linear_fwd(problems: list[tuple], rows: int, elu: bool = False, act: int | N
     """problems: (x [rows, in], w [out, in], b [out], z [rows, out] or None, h [rows, out] or None).
     act: the hidden-layer activation (an L.ACTIVATIONS code; elu=True is L.PPO_ACT_ELU), h = act(z); without one z is
     required, with one at least one of z / h.  bf16: bf16 operands (ppo_linear_fwd_ex, PPO_GEMM_BF16_OPERANDS).
-    ranges: per problem the largest-magnitude slots of (x, w, output or None) (ppo_linear_fwd_ranged)."""
+    ranges: per problem the range slots of (x, w, output or None) (ppo_linear_fwd_ranged)."""
     act = (L.PPO_ACT_ELU if elu else L.PPO_ACT_NONE) if act is None else int(act)
     elu = act != L.PPO_ACT_NONE
     items = []
@@ -524,7 +528,7 @@ def linear_bwd_dx(problems: list[tuple], rows: int, ws: Workspace | None = None,
                   act: int = L.PPO_ACT_ELU, bf16: bool = False, ranges: list[tuple] | None = None) -> None:
     """problems: (dz [rows, out], w [out, in], src [rows, in] or None, dz_prev [rows, in]); src is the activation's
     input z of the layer below, or its output h = act(z) with elu_from_output (monotone activations only).  bf16:
-    bf16 operands (ppo_linear_bwd_dx_ex, PPO_GEMM_BF16_OPERANDS).  ranges: per problem the largest-magnitude slots of
+    bf16 operands (ppo_linear_bwd_dx_ex, PPO_GEMM_BF16_OPERANDS).  ranges: per problem the range slots of
     (dz, w, dz_prev or None) (ppo_linear_bwd_dx_ranged)."""
     arr, count, nbytes = _dx_problems(problems, rows)
     buf = (ws or Workspace(problems[0][0].device)).get(nbytes)
@@ -559,7 +563,7 @@ def linear_bwd_dw(problems: list[tuple], rows: int, ws: Workspace | None = None,
                   bf16: bool = False, ranges: list[tuple] | None = None) -> None:
     """problems: (dz [rows, out], x [rows, in], dw [out, in], db [out] or None for no bias gradient).  With `norm`
     the launch also writes the per-group sums of squares of what it stores (ppo_linear_bwd_dw_norm).  bf16: bf16
-    operands (ppo_linear_bwd_dw_ex, PPO_GEMM_BF16_OPERANDS).  ranges: per problem the largest-magnitude slots of
+    operands (ppo_linear_bwd_dw_ex, PPO_GEMM_BF16_OPERANDS).  ranges: per problem the range slots of
     (dz, x, None) (ppo_linear_bwd_dw_ranged)."""
     items = []
     for i, (dz, x, dw, db) in enumerate(problems):
@@ -743,7 +747,8 @@ def ppo_head(args: L.LossArgs, h_actor: torch.Tensor, w_actor: torch.Tensor, b_a
              ranges: tuple | None = None) -> None:
     """Output layers + loss + finalize + the output layers' input-grad in one call (ppo_gauss_ppo_head).  args
     carries the batch columns and d_mean / d_value; its mean / value fields are not read.  ranges: the
-    largest-magnitude slots of (dz_actor, dz_critic, d_mean, d_value) to raise (ppo_gauss_ppo_head_ranged)."""
+    range slots of (dz_actor, dz_critic, d_mean, d_value) to raise and of (h_actor, h_critic)
+    (ppo_gauss_ppo_head_ranged)."""
     _dev(h_actor, w_actor, b_actor, h_critic, w_critic, b_critic, dz_actor, dz_critic, mean, value)
     R = int(args.rows)
     for name, t in (("h_actor", h_actor), ("h_critic", h_critic), ("dz_actor", dz_actor), ("dz_critic", dz_critic)):

@@ -353,3 +353,26 @@ def test_update_with_a_sentinel_observation(activation, every, actions, monkeypa
         assert torch.equal(torch.isfinite(a), torch.isfinite(b))
         if float(b.norm()) > 0:
             assert float((a - b).norm() / b.norm()) < 1e-4
+
+
+def test_an_engine_that_uses_no_ranges_allocates_none():
+    """Small and recurrent updates run without slots; an engine made with mixed precision has them for when that is off."""
+    from types import SimpleNamespace
+
+    from tt_rsl_rl_amd import engine
+    from tt_rsl_rl_amd.ppo import PPO
+
+    def made(n, mixed=False, **model):
+        model = dict(dict(class_name="MLPModel", hidden_dims=[16], activation="elu"), **model)
+        cfg = dict(algorithm=dict(class_name="tt_rsl_rl_amd.ppo:PPO", num_mini_batches=1, use_mixed_precision=mixed),
+                   actor=dict(model, distribution_cfg=dict(class_name="GaussianDistribution")), critic=model,
+                   obs_groups={"actor": ["g"], "critic": ["g"]}, num_steps_per_env=2)
+        alg = PPO.construct_algorithm({"g": torch.zeros(n, 4)}, SimpleNamespace(num_envs=n, num_actions=2), cfg, "cuda:0")
+        alg.storage.distribution_params = ()
+        return alg._get_engine()
+
+    lstm = dict(class_name="RNNModel", rnn_type="lstm", rnn_hidden_dim=16, rnn_num_layers=1)
+    n = engine.RANGED_ROWS // 2
+    for e, slots in ((made(100), False), (made(n, **lstm), False), (made(n), True), (made(n, mixed=True), True)):
+        assert hasattr(e, "w_max") is slots
+        assert not e.ranged or slots

@@ -213,7 +213,8 @@ class UpdateEngine:
                     self.w0_mirrors.append((alg.flat.offsets[id(w)][0], w.shape[0], w.shape[1], wp))
         self.buf_a = ModelBuffers(actor, self.R_max, self.device)
         self.buf_c = ModelBuffers(critic, self.R_max, self.device)
-        self._init_ranges()
+        if self.R_max >= RANGED_ROWS and not self.recurrent:  # (mixed precision may be switched from update to update)
+            self._init_ranges()
         self.loss_ws = torch.empty(ops.loss_workspace_bytes(self.R_max, self.A), dtype=torch.uint8, device=self.device)
         # learn_std=False (distribution.py:166): the std parameter takes no gradient; the loss kernels' gradient for it
         # goes here instead of into the flat gradient, whose slot stays zero, so Adam leaves the parameter (and its

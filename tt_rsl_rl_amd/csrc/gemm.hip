@@ -405,18 +405,12 @@ int launch_nt_f16(Group& g, int count, hipStream_t s, const char* name) {
     if (bn == 64) return go(gemm_nt_f16_kernel<64, 2, 4, EPI, BKM, AR>, 256);
     return go(gemm_nt_f16_kernel<128, 2, 3, EPI, BKM, AR>, 256);
   } else {
-  // (then the problems it left: gemm_nt_wide_kernel)
-  auto both = [&](auto kernel, int threads, auto wide) {
-    if (int rc = go(kernel, threads)) return rc;
-    hipLaunchKernelGGL(wide, dim3(std::min(blocks, device_info().cus)), dim3(512), 0, s, g, blocks);
-    return check_launch(name);
-  };
-  if (bn == 64) return both(gemm_nt_f16_kernel<64, 2, 3, EPI, BKM, AR>, 256, gemm_nt_wide_kernel<64, EPI, BKM>);
+  if (bn == 64) return go(gemm_nt_f16_kernel<64, 2, 3, EPI, BKM, AR>, 256);
   // 128 x 128: eight waves of 32 x 64 (128 registers, four waves per SIMD) for the forward, whose epilogue's activation
   // then overlaps other waves' products (512 -> 256 features: 56 us against 63 with four waves of 64 x 64, 240 -> 512:
   // 66 against 73); the input-grad's longer staging and epilogue do not fit 128 registers (74 against 69 us)
-  if constexpr (BKM) return both(gemm_nt_f16_kernel<128, 2, 2, EPI, BKM, AR>, 256, gemm_nt_wide_kernel<128, EPI, BKM>);
-  else return both(gemm_nt_f16_kernel<128, 4, 4, EPI, BKM, AR>, 512, gemm_nt_wide_kernel<128, EPI, BKM>);
+  if constexpr (BKM) return go(gemm_nt_f16_kernel<128, 2, 2, EPI, BKM, AR>, 256);
+  else return go(gemm_nt_f16_kernel<128, 4, 4, EPI, BKM, AR>, 512);
   }
 }
 
@@ -436,12 +430,7 @@ int launch_tn_f16(Group& g, int count, hipStream_t s, const char* name) {
   }
   if (blocks == 0) return PPO_OK;
   hipLaunchKernelGGL((gemm_tn_f16_kernel<2, OCC, AR>), dim3(blocks), dim3(256), 0, s, g);
-  if (int rc = check_launch(name)) return rc;
-  if (AR == ARITH_F16X3) {  // then the problems it left
-    hipLaunchKernelGGL(gemm_tn_wide_kernel, dim3(std::min(blocks, device_info().cus)), dim3(512), 0, s, g, blocks);
-    return check_launch(name);
-  }
-  return PPO_OK;
+  return check_launch(name);
 }
 
 // Ranges of a few tensors: one block row per item, the last grid row clears the caller's words.  A block takes `chunk` rows

@@ -310,9 +310,8 @@ struct TileCoord {
   int pi, split, tm, tn;
 };
 
-// Tile `block` of `blocks`.
-__device__ inline TileCoord locate_at(const Group& g, int block, int blocks) {
-  const int b = g.xcds > 1 ? xcd_remap(block, blocks, g.xcds) : block;
+__device__ inline TileCoord locate(const Group& g) {
+  const int b = g.xcds > 1 ? xcd_remap(blockIdx.x, gridDim.x, g.xcds) : static_cast<int>(blockIdx.x);
   int pi = 0;
 #pragma unroll
   for (int i = 1; i < PPO_MAX_LINEAR_PROBLEMS; ++i) {
@@ -329,8 +328,6 @@ __device__ inline TileCoord locate_at(const Group& g, int block, int blocks) {
   t.tn = r - t.tm * P.tiles_n;
   return t;
 }
-
-__device__ inline TileCoord locate(const Group& g) { return locate_at(g, blockIdx.x, gridDim.x); }
 
 // Direct global->LDS copy through a raw buffer: every lane moves BYTES from byte offset `off` of buffer r to
 // lds_wave + lane * BYTES (lds_wave wave-uniform), and an offset at or past the buffer's record count reads zeros.

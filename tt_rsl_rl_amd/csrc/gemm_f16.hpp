@@ -39,7 +39,7 @@ __device__ __forceinline__ void split_f16x2(float x0, float x1, float s, float k
 enum Arith : int {
   ARITH_F16X3 = 0,  // two fp16 parts, three products, two accumulators
   ARITH_BF16 = 1,   // bf16 operands (PPO_GEMM_BF16_OPERANDS): one part, one product
-  ARITH_BF16X6 = 2, // three bf16 parts, six products (gemm_core.hpp): the problems whose operands span too much for fp16x3
+  ARITH_BF16X6 = 2, // three bf16 parts, six products (gemm_core.hpp): problems whose operands span too much for fp16x3
 };
 
 template <int AR>
@@ -84,7 +84,7 @@ template <int AR, int TM, int TN, bool FLIP>
 __device__ __forceinline__ void products(f32x16 (&acc)[Parts<AR>::accs][TM][TN], const u32x4 (&fa)[TM][Parts<AR>::planes],
                                          const u32x4 (&fb)[TN][Parts<AR>::planes], int t) {
   constexpr int pa[3] = {1, 0, 0}, pb[3] = {0, 1, 0};
-  constexpr int pa6[6] = {2, 1, 0, 1, 0, 0}, pb6[6] = {0, 1, 2, 0, 1, 0};
+  constexpr int pa6[6] = {2, 1, 0, 1, 0, 0}, pb6[6] = {0, 1, 2, 0, 1, 0};  // (small terms first, as gemm_core.hpp's)
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -125,22 +125,39 @@ __device__ __forceinline__ void join_acc(f32x16 (&acc)[Parts<AR>::accs][TM][TN])
 // LDS planes: [row][32 k] halves, the 16-byte chunk index XOR-ed with (row / 4) % 4 (the 16 rows that a ds_read_b128
 // serves at a time fall on all 64 banks); BKM's B: [32 k][BN n], as the weight-grad's.
 // ------------------------------------------------------------------------------------------------------------------
-template <int BN, int WM, int AR>
-struct NtF16 {
-  static constexpr int stage = Parts<AR>::planes * (128 + BN) * 32 * 2;
-  static constexpr int patch = WM * 2 * 32 * 36 * 4;
-  static constexpr int lds = 2 * stage > patch ? 2 * stage : patch;
-};
+// fp16x3: a problem with an operand that is not narrow() (amax.hpp) takes its tiles in bf16x6, one slab at a time, three
+// planes in the memory of the two stages.  It is there for outliers, and a function of its own so that the usual path keeps
+// its registers (as a branch with a loop inside the kernel it cost 17 to 22 spilled ones; as a launch of its own after each
+// of these, 3 us and a gap where there is nothing to do).  98,304 rows, 240 -> 512, with an outlier / without / the plain
+// kernels: forward 201 / 144 / 164 us, input-grad 179 / 139 / 162, weight-grad 196 / 143 / 162.
+using LdsBytes = __attribute__((address_space(3))) unsigned char;
+using GroupArgument = const __attribute__((address_space(4))) Group;
+template <int BN, int WM, int EPI, bool BKM>
+__device__ __attribute__((noinline)) void nt_wide_tile(uint64_t group, LdsBytes* lds);
+template <int BN, int WM>
+__device__ __attribute__((noinline)) void tn_wide_tile(uint64_t group, LdsBytes* lds);
 
-// slot: of the output's range.  fp16x3: a problem with an operand that is not narrow() is left to the launch after it.
+// Where a kernel whose first argument is a Group finds it: for the functions it calls (evaluated in the kernel itself: the
+// kernel-argument pointer is null in a called function).
+__device__ __forceinline__ uint64_t group_argument() {
+  return reinterpret_cast<uint64_t>((const void*)__builtin_amdgcn_kernarg_segment_ptr());
+}
+// The same in the called function, with a wave-uniform address.
+__device__ __forceinline__ const Group& group_at(uint64_t address) {
+  const uint64_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(address)));
+  const uint64_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(address >> 32)));
+  return *(const Group*)(GroupArgument*)((hi << 32) | lo);
+}
+
 template <int BN, int WM, int EPI, bool BKM, int AR>
-__device__ __forceinline__ void nt_f16_tile(const Group& g, const TileCoord tc, unsigned char* lds, int slot) {
+__device__ __forceinline__ void nt_f16_tile(const Group& g, unsigned char* lds) {
   static_assert(EPI == EPI_BIAS || epi_fwd_act(EPI) || epi_act_grad(EPI) || EPI == EPI_STORE, "NT epilogues");
   constexpr int BM = 128, BK = 32, THREADS = WM * 128, TM = 4 / WM, TN = BN / 64, NPL = Parts<AR>::planes;
   constexpr int PLANE_A = BM * BK * 2, PLANE_B = BN * BK * 2;
-  constexpr int STAGE = NtF16<BN, WM, AR>::stage;
+  constexpr int STAGE = NPL * (PLANE_A + PLANE_B);
   constexpr int PS = 36;
 
+  const TileCoord tc = locate(g);
   const Problem& P = g.p[tc.pi];
   const int64_t lda = P.lda, ldb = P.ldb;
   const int row0 = tc.tm * BM, col0 = tc.tn * BN;
@@ -215,7 +232,10 @@ __device__ __forceinline__ void nt_f16_tile(const Group& g, const TileCoord tc, 
   int ea = 0, eb = 0;
   if constexpr (AR == ARITH_F16X3) {
     const Range ra = load_range(P.amax_a, lane), rb = load_range(P.amax_b, lane);
-    if (!ra.narrow() || !rb.narrow()) return;
+    if (!ra.narrow() || !rb.narrow()) {
+      nt_wide_tile<BN, WM, EPI, BKM>(group_argument(), (LdsBytes*)lds);
+      return;
+    }
     ea = amax_exponent(ra.top);
     eb = amax_exponent(rb.top);
   }
@@ -229,14 +249,14 @@ __device__ __forceinline__ void nt_f16_tile(const Group& g, const TileCoord tc, 
   };
 
   f32x16 acc[Parts<AR>::accs][TM][TN];
-#pragma unroll
-  for (int a = 0; a < Parts<AR>::accs; ++a)
+  auto clear = [&](int a) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[a][i][j][v] = 0.0f;
+  };
 
   const int fr = lane & 31, fc = lane >> 5;
   auto frag = [&](const unsigned char* pl, int r, int kg) {
@@ -255,15 +275,6 @@ __device__ __forceinline__ void nt_f16_tile(const Group& g, const TileCoord tc, 
     return __builtin_bit_cast(u32x4, v);
   };
 
-  if (nk > 0) {
-    mask_tail(0);
-#pragma unroll
-    for (int o = 0; o < NA + NB; ++o) {
-      split_piece(lds, o);
-      load_piece(1, o);
-    }
-    lds_barrier();
-  }
   constexpr int NT = Parts<AR>::products;
   u32x4 fa[TM][NPL], fb[TN][NPL];
   auto read = [&](const unsigned char* st, int kg) __attribute__((always_inline)) {
@@ -274,9 +285,38 @@ __device__ __forceinline__ void nt_f16_tile(const Group& g, const TileCoord tc, 
 #pragma unroll
       for (int j = 0; j < TN; ++j)
         fb[j][pp] = BKM ? frag_t(st + NPL * PLANE_A + pp * PLANE_B, wn * (BN / 2) + 32 * j, kg)
-                        : frag(st + NPL * PLANE_A + pp * PLANE_B, wn * (BN / 2) + 32 * j + fr, kg);
+                       : frag(st + NPL * PLANE_A + pp * PLANE_B, wn * (BN / 2) + 32 * j + fr, kg);
     }
   };
+#pragma unroll
+  for (int a = 0; a < Parts<AR>::accs; ++a) clear(a);
+  if constexpr (AR == ARITH_BF16X6) {  // one slab at a time in one stage
+    for (int kt = 0; kt < nk; ++kt) {
+      mask_tail(kt);
+#pragma unroll
+      for (int o = 0; o < NA + NB; ++o) {
+        split_piece(lds, o);
+        load_piece(kt + 1, o);
+      }
+      lds_barrier();
+#pragma unroll
+      for (int kg = 0; kg < 2; ++kg) {
+        read(lds, kg);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) products<AR, TM, TN, true>(acc, fa, fb, t);
+      }
+      lds_barrier();
+    }
+  } else {
+  if (nk > 0) {
+    mask_tail(0);
+#pragma unroll
+    for (int o = 0; o < NA + NB; ++o) {
+      split_piece(lds, o);
+      load_piece(1, o);
+    }
+    lds_barrier();
+  }
   for (int kt = 0; kt + 1 < nk; ++kt) {
     const unsigned char* st = lds + (kt & 1) * STAGE;
     unsigned char* nst = lds + ((kt & 1) ^ 1) * STAGE;
@@ -307,49 +347,29 @@ __device__ __forceinline__ void nt_f16_tile(const Group& g, const TileCoord tc, 
     lds_barrier();
   }
   join_acc<AR, TM, TN>(acc);
+  }
   float* const patch = reinterpret_cast<float*>(lds) + wave * 32 * PS;  // every wave is past the last barrier
   const int rw = row0 + wm * (128 / WM), cw = col0 + wn * (BN / 2);
   if constexpr (AR != ARITH_BF16) {
     const float m = nt_pipe_epilogue_t<TM, TN, EPI, epi_generic(EPI), true>(P, acc[0], rw, cw, patch, lane,
                                                                                pow2(-ea), pow2(-eb));
-    if (P.amax_c != nullptr) amax_publish(P.amax_c, m, AR == ARITH_BF16X6, lane, (THREADS / 64) * slot + wave);
+    if (P.amax_c != nullptr) amax_publish(P.amax_c, m, AR == ARITH_BF16X6, lane, (THREADS / 64) * blockIdx.x + wave);
   } else {
     nt_pipe_epilogue<TM, TN, EPI>(P, acc[0], rw, cw, patch, lane);
   }
 }
 
+template <int BN, int WM, int EPI, bool BKM>
+__device__ __attribute__((noinline)) void nt_wide_tile(uint64_t group, LdsBytes* lds) {
+  nt_f16_tile<BN, WM, EPI, BKM, ARITH_BF16X6>(group_at(group), (unsigned char*)lds);
+}
+
 template <int BN, int WM, int OCC, int EPI, bool BKM, int AR>
 __global__ __launch_bounds__(WM * 128) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemm_nt_f16_kernel(
     const Group g) {
-  __shared__ __align__(16) unsigned char lds[NtF16<BN, WM, AR>::lds];
-  nt_f16_tile<BN, WM, EPI, BKM, AR>(g, locate(g), lds, blockIdx.x);
-}
-
-// The problems (bit i: problem i) with an operand that fp16x3 does not take.
-__device__ __forceinline__ uint32_t wide_problems(const Group& g, int lane) {
-  uint32_t wide = 0;
-  for (int i = 0; i < g.count; ++i) {
-    const Range ra = load_range(g.p[i].amax_a, lane), rb = load_range(g.p[i].amax_b, lane);
-    if (!ra.narrow() || !rb.narrow()) wide |= 1u << i;
-  }
-  return wide;
-}
-
-// The launch after an fp16x3 one: its wide problems, on the same tiles in bf16x6, a block per compute unit going through
-// them; nothing where there are none (the usual case: a launch of 3 us).  Three planes take 96 KB of LDS: one block per
-// compute unit, eight waves.
-template <int BN, int EPI, bool BKM>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_nt_wide_kernel(const Group g,
-                                                                                                      int tiles) {
-  __shared__ __align__(16) unsigned char lds[NtF16<BN, 4, ARITH_BF16X6>::lds];
-  const uint32_t wide = wide_problems(g, threadIdx.x & 63);
-  if (wide == 0) return;
-  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
-    const TileCoord tc = locate_at(g, t, tiles);
-    if (((wide >> tc.pi) & 1) == 0) continue;
-    nt_f16_tile<BN, 4, EPI, BKM, ARITH_BF16X6>(g, tc, lds, t);
-    __syncthreads();  // (the next tile's stages lie where this one's patches are)
-  }
+  constexpr int STAGES = 2 * Parts<AR>::planes * (128 + BN) * 32 * 2, PATCHES = WM * 2 * 32 * 36 * 4;
+  __shared__ __align__(16) unsigned char lds[STAGES > PATCHES ? STAGES : PATCHES];
+  nt_f16_tile<BN, WM, EPI, BKM, AR>(g, lds);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -359,7 +379,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // slab's own start zeroed (and a matrix of fewer than 32 rows re-reads its last row, zeroed).
 // ------------------------------------------------------------------------------------------------------------------
 template <int BN, int WM, int AR>
-__device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, unsigned char* lds) {
+__device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, unsigned char* lds, int ea = 0, int eb = 0) {
   constexpr int BM = 128, BK = 32, THREADS = WM * 128, TM = 4 / WM, TN = BN / 64, NPL = Parts<AR>::planes;
   constexpr int PLANE_A = BK * BM * 2, PLANE_B = BK * BN * 2, STAGE = NPL * (PLANE_A + PLANE_B);
   const Problem& P = g.p[tc.pi];
@@ -416,13 +436,6 @@ __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, 
   };
 #pragma unroll
   for (int o = 0; o < NA + NB; ++o) load_piece(0, o);
-  int ea = 0, eb = 0;
-  if constexpr (AR == ARITH_F16X3) {
-    const Range ra = load_range(P.amax_a, lane), rb = load_range(P.amax_b, lane);
-    if (!ra.narrow() || !rb.narrow()) return;
-    ea = amax_exponent(ra.top);
-    eb = amax_exponent(rb.top);
-  }
   const float sa = pow2(ea), sb = pow2(eb);
   const float k2048 = 2048.0f;
   double colsum_acc[4] = {0.0, 0.0, 0.0, 0.0};
@@ -438,14 +451,14 @@ __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, 
   };
 
   f32x16 acc[Parts<AR>::accs][TM][TN];
-#pragma unroll
-  for (int a = 0; a < Parts<AR>::accs; ++a)
+  auto clear = [&](int a) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[a][i][j][v] = 0.0f;
+  };
 
   const int grp = lane >> 4, gi = lane & 3, gr = (lane >> 2) & 3;
   const int rd_k = 8 * (grp >> 1) + gr, rd_c = 4 * (grp & 1) + gi;
@@ -461,16 +474,6 @@ __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, 
     return __builtin_bit_cast(u32x4, v);
   };
 
-  if (nk > 0) {
-    mask_tail(0);
-#pragma unroll
-    for (int o = 0; o < NA + NB; ++o) {
-      split_piece(lds, o);
-      if (o < NA && want_colsum) add_colsum(o < NA ? o : 0);
-      load_piece(1, o);
-    }
-    lds_barrier();
-  }
   constexpr int NT = Parts<AR>::products;
   u32x4 fa[TM][NPL], fb[TN][NPL];
   auto read = [&](const unsigned char* st, int kg) __attribute__((always_inline)) {
@@ -483,6 +486,37 @@ __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, 
         fb[j][pp] = frag(IntC<BN>{}, st + NPL * PLANE_A + pp * PLANE_B, wn * (BN / 2) + 32 * j, kg);
     }
   };
+#pragma unroll
+  for (int a = 0; a < Parts<AR>::accs; ++a) clear(a);
+  if constexpr (AR == ARITH_BF16X6) {  // (as in nt_f16_tile)
+    for (int kt = 0; kt < nk; ++kt) {
+      mask_tail(kt);
+#pragma unroll
+      for (int o = 0; o < NA + NB; ++o) {
+        split_piece(lds, o);
+        if (o < NA && want_colsum) add_colsum(o < NA ? o : 0);
+        load_piece(kt + 1, o);
+      }
+      lds_barrier();
+#pragma unroll
+      for (int kg = 0; kg < 2; ++kg) {
+        read(lds, kg);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) products<AR, TM, TN, false>(acc, fa, fb, t);
+      }
+      lds_barrier();
+    }
+  } else {
+  if (nk > 0) {
+    mask_tail(0);
+#pragma unroll
+    for (int o = 0; o < NA + NB; ++o) {
+      split_piece(lds, o);
+      if (o < NA && want_colsum) add_colsum(o < NA ? o : 0);
+      load_piece(1, o);
+    }
+    lds_barrier();
+  }
   for (int kt = 0; kt + 1 < nk; ++kt) {
     const unsigned char* st = lds + (kt & 1) * STAGE;
     unsigned char* nst = lds + ((kt & 1) ^ 1) * STAGE;
@@ -513,6 +547,7 @@ __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, 
     }
   }
   join_acc<AR, TM, TN>(acc);
+  }
   [[maybe_unused]] const float ra = pow2(-ea), rb = pow2(-eb);
 
   const int fr = lane & 31, fc = lane >> 5;
@@ -543,33 +578,34 @@ __device__ __forceinline__ void tn_f16_tile(const Group& g, const TileCoord tc, 
   }
 }
 
+template <int BN, int WM>
+__device__ __attribute__((noinline)) void tn_wide_tile(uint64_t group, LdsBytes* lds) {
+  const Group& g = group_at(group);
+  tn_f16_tile<BN, WM, ARITH_BF16X6>(g, locate(g), (unsigned char*)lds);
+}
+
 template <int WM, int OCC, int AR>
 __global__ __launch_bounds__(WM * 128) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void gemm_tn_f16_kernel(
     const Group g) {
   __shared__ __align__(16) unsigned char lds[2 * Parts<AR>::planes * 2 * 32 * 128 * 2];
   const TileCoord tc = locate(g);
-  if (g.p[tc.pi].tn64) {
-    tn_f16_tile<64, WM, AR>(g, tc, lds);
-  } else {
-    tn_f16_tile<128, WM, AR>(g, tc, lds);
-  }
-}
-
-// As gemm_nt_wide_kernel, for the weight-grad.
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tn_wide_kernel(const Group g,
-                                                                                                      int tiles) {
-  __shared__ __align__(16) unsigned char lds[2 * Parts<ARITH_BF16X6>::planes * 2 * 32 * 128 * 2];
-  const uint32_t wide = wide_problems(g, threadIdx.x & 63);
-  if (wide == 0) return;
-  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
-    const TileCoord tc = locate_at(g, t, tiles);
-    if (((wide >> tc.pi) & 1) == 0) continue;
-    if (g.p[tc.pi].tn64) {
-      tn_f16_tile<64, 4, ARITH_BF16X6>(g, tc, lds);
-    } else {
-      tn_f16_tile<128, 4, ARITH_BF16X6>(g, tc, lds);
+  const Problem& P = g.p[tc.pi];
+  int ea = 0, eb = 0;
+  if constexpr (AR == ARITH_F16X3) {
+    const int lane = threadIdx.x & 63;
+    const Range ra = load_range(P.amax_a, lane), rb = load_range(P.amax_b, lane);
+    if (!ra.narrow() || !rb.narrow()) {
+      if (P.tn64) tn_wide_tile<64, WM>(group_argument(), (LdsBytes*)lds);
+      else tn_wide_tile<128, WM>(group_argument(), (LdsBytes*)lds);
+      return;
     }
-    __syncthreads();
+    ea = amax_exponent(ra.top);
+    eb = amax_exponent(rb.top);
+  }
+  if (P.tn64) {
+    tn_f16_tile<64, WM, AR>(g, tc, lds, ea, eb);
+  } else {
+    tn_f16_tile<128, WM, AR>(g, tc, lds, ea, eb);
   }
 }
 

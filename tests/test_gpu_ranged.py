@@ -376,3 +376,29 @@ def test_an_engine_that_uses_no_ranges_allocates_none():
     for e, slots in ((made(100), False), (made(n, **lstm), False), (made(n), True), (made(n, mixed=True), True)):
         assert hasattr(e, "w_max") is slots
         assert not e.ranged or slots
+
+
+@pytest.mark.parametrize("act", ["tanh", "elu"])
+def test_activations_are_as_close_as_the_plain_kernels(act):
+    """The ranged forward's activations on exact inputs (an identity weight, 20-bit inputs that two fp16 parts hold) against
+    fp64, in units of the last place: at most 1.4, and in root mean square the plain kernels' (tanhf; the longer ELU) plus
+    2 % (ELU's shorter polynomial is 2e-8 off, a third of a rounding)."""
+    rows, k = 1 << 15, 64
+    g = torch.Generator("cuda").manual_seed(0)
+    w, b, f = torch.eye(k, device="cuda"), torch.zeros(k, device="cuda"), {"tanh": torch.tanh, "elu": torch.nn.functional.elu}[act]
+    worst, sq = [0.0, 0.0], [0.0, 0.0]
+    for lo, hi in ((1e-3, 0.01), (0.01, 0.5), (0.5, 0.6), (0.6, 0.7), (0.69, 0.71), (0.7, 1.0), (0.99, 1.01), (1.0, 2.0), (2.0, 12.0)):
+        for sign in (1.0, -1.0):
+            x = torch.rand(rows, k, generator=g, device="cuda") * (hi - lo) + lo
+            x = (x.view(torch.int32) & ~0xF).view(torch.float32) * sign
+            sx, sw = _slots(x, w)
+            want = f(x.double())
+            ulp = torch.pow(2.0, torch.frexp(want.abs())[1].double() - 24)
+            for i, rng in enumerate(([(sx, sw, None)], None)):
+                z, h = torch.empty(rows, k, device="cuda"), torch.empty(rows, k, device="cuda")
+                ops.linear_fwd([(x, w, b, z, h)], rows, act=L.ACTIVATIONS[act], ranges=rng)
+                assert torch.equal(z, x)
+                e = (h.double() - want).abs() / ulp
+                worst[i], sq[i] = max(worst[i], float(e.max())), sq[i] + float((e ** 2).mean())
+    print(act, worst, [(s / 18) ** 0.5 for s in sq])
+    assert worst[0] <= 1.4 and sq[0] ** 0.5 <= 1.02 * sq[1] ** 0.5

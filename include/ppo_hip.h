@@ -315,7 +315,6 @@ int ppo_normalizer_update(const ppo_column_block* blocks, int32_t num_blocks, in
  * most 1,024 features per layer (PPO_EUNSUPPORTED otherwise).  A block of threads carries 16 rows through all layers, so
  * it is meant for up to some thousands of rows; larger batches are faster as ppo_linear_fwd per layer.
  * ------------------------------------------------------------------------------------------------------------------ */
-#define PPO_MAX_MLP_PROBLEMS 2
 #define PPO_MAX_MLP_LAYERS 8
 #define PPO_MAX_MLP_BLOCKS 8
 typedef struct ppo_mlp_layer {
@@ -336,13 +335,13 @@ typedef struct ppo_mlp_problem {
   int32_t num_layers;
   int32_t activation; /* PPO_ACT_*, of the hidden layers */
 } ppo_mlp_problem;
-int ppo_mlp_fwd(const ppo_mlp_problem* problems, int32_t count, int64_t rows, ppo_stream_t stream);
+int ppo_mlp_fwd(const ppo_mlp_problem* problem, int64_t rows, ppo_stream_t stream);
 /* The same in one launch per two layers, for few rows: every block computes the first of the two for its 16 rows and a
  * slice of the second's outputs, which go through the workspace (its bytes are proportional to the rows; 0: none needed).
  * The same results. */
-size_t ppo_mlp_fwd_pairs_workspace_bytes(const ppo_mlp_problem* problems, int32_t count, int64_t rows);
-int ppo_mlp_fwd_pairs(const ppo_mlp_problem* problems, int32_t count, int64_t rows, void* workspace,
-                      size_t workspace_bytes, ppo_stream_t stream);
+size_t ppo_mlp_fwd_pairs_workspace_bytes(const ppo_mlp_problem* problem, int64_t rows);
+int ppo_mlp_fwd_pairs(const ppo_mlp_problem* problem, int64_t rows, void* workspace, size_t workspace_bytes,
+                      ppo_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------------------------------
  * A8-A11  Gaussian policy head + PPO losses, forward and backward, rsl_rl/algorithms/ppo.py:226-285 with

@@ -183,7 +183,7 @@ class LstmGradProblem(C.Structure):
     _fields_ = [("dw_ih_g", vp), ("dw_hh_g", vp), ("db_g", vp), ("dw_ih", vp), ("dw_hh", vp), ("db_ih", vp),
                 ("db_hh", vp), ("input_size", i32), ("hidden", i32)]
 
-MAX_MLP_PROBLEMS, MAX_MLP_LAYERS, MAX_MLP_BLOCKS = 2, 8, 8
+MAX_MLP_LAYERS, MAX_MLP_BLOCKS = 8, 8
 MLP_MAX_WIDTH = 1024  # widest layer input of ppo_mlp_fwd
 
 
@@ -244,9 +244,9 @@ _SIGNATURES = [
                                            C.c_void_p, C.c_size_t, f32p, C.POINTER(GradRange), i32, C.c_void_p,
                                            C.c_void_p]),
     ("ppo_obs_normalize", C.c_int, [f32p, i64, f32p, i64, i64, i32, f32p, f32p, C.c_float, C.c_void_p]),
-    ("ppo_mlp_fwd", C.c_int, [C.POINTER(MlpProblem), i32, i64, C.c_void_p]),
-    ("ppo_mlp_fwd_pairs_workspace_bytes", C.c_size_t, [C.POINTER(MlpProblem), i32, i64]),
-    ("ppo_mlp_fwd_pairs", C.c_int, [C.POINTER(MlpProblem), i32, i64, C.c_void_p, C.c_size_t, C.c_void_p]),
+    ("ppo_mlp_fwd", C.c_int, [C.POINTER(MlpProblem), i64, C.c_void_p]),
+    ("ppo_mlp_fwd_pairs_workspace_bytes", C.c_size_t, [C.POINTER(MlpProblem), i64]),
+    ("ppo_mlp_fwd_pairs", C.c_int, [C.POINTER(MlpProblem), i64, C.c_void_p, C.c_size_t, C.c_void_p]),
     ("ppo_normalizer_update_workspace_bytes", C.c_size_t, [i64, i32]),
     ("ppo_normalizer_update", C.c_int, [C.POINTER(ColumnBlock), i32, i64, f32p, f32p, f32p, C.c_void_p, C.c_void_p,
                                         C.c_size_t, C.c_void_p]),

@@ -19,22 +19,21 @@ namespace {
 constexpr int kMlpRows = 16, kMlpWaves = 8, kMlpThreads = 64 * kMlpWaves;
 constexpr int kMlpMaxWidth = 1024;
 
-struct MlpGroup {
-  ppo_mlp_problem p[PPO_MAX_MLP_PROBLEMS];
-  int32_t count, blocks;  // blocks per problem
-  int32_t ldx;            // floats per LDS row
+struct MlpArgs {
+  ppo_mlp_problem p;
+  int32_t blocks;  // of 16 rows
+  int32_t ldx;     // floats per LDS row
   int64_t rows;
 };
-static_assert(sizeof(MlpGroup) <= 4096, "kernel arguments");
+static_assert(sizeof(MlpArgs) <= 4096, "kernel arguments");
 
-// One launch of ppo_mlp_fwd_pairs: layers l0 and, where there is one, l0 + 1 of every problem.
+// One launch of ppo_mlp_fwd_pairs: layers l0 and, where there is one, l0 + 1.
 struct MlpPairs {
-  MlpGroup g;
-  const float* in[PPO_MAX_MLP_PROBLEMS];  // [rows, ld] (NULL: the problem's input blocks)
-  float* to[PPO_MAX_MLP_PROBLEMS];        // [rows, ld] (NULL: its output)
-  int64_t ld[PPO_MAX_MLP_PROBLEMS];
-  int32_t slices[PPO_MAX_MLP_PROBLEMS];  // blocks per 16 rows, kSliceTiles tiles of the second layer each
-  int32_t begin1;                        // the second problem's first block
+  MlpArgs g;
+  const float* in;  // [rows, ld] (NULL: the problem's input blocks)
+  float* to;        // [rows, ld]
+  int64_t ld;
+  int32_t slices;  // blocks per 16 rows, kSliceTiles tiles of the second layer each
   int32_t l0;
 };
 static_assert(sizeof(MlpPairs) <= 4096, "kernel arguments");
@@ -181,11 +180,10 @@ __device__ __forceinline__ void mlp_input(const ppo_mlp_problem& P, float* x, in
   for (int c = col + c0; c < (col + 15) / 16 * 16; c += 32) x[r * ldx + c] = 0.0f;
 }
 
-__global__ __launch_bounds__(kMlpThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void mlp_fwd_kernel(const MlpGroup g) {
+__global__ __launch_bounds__(kMlpThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void mlp_fwd_kernel(const MlpArgs g) {
   extern __shared__ __align__(16) float lds[];
-  const int pi = static_cast<int>(blockIdx.x) >= g.blocks ? 1 : 0;
-  const ppo_mlp_problem& P = g.p[pi];
-  const int64_t row0 = static_cast<int64_t>(static_cast<int>(blockIdx.x) - pi * g.blocks) * kMlpRows;
+  const ppo_mlp_problem& P = g.p;
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kMlpRows;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int ldx = g.ldx;
   float* x = lds;
@@ -211,24 +209,21 @@ __global__ __launch_bounds__(kMlpThreads) __attribute__((amdgpu_waves_per_eu(4, 
 // Layers l0 (all of it, in LDS) and l0 + 1 (the block's slice of tiles, to global memory), or a slice of l0 alone.
 __global__ __launch_bounds__(kMlpThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void mlp_pairs_kernel(const MlpPairs a) {
   extern __shared__ __align__(16) float lds[];
-  const int pi = static_cast<int>(blockIdx.x) >= a.begin1 ? 1 : 0;
-  const ppo_mlp_problem& P = a.g.p[pi];
-  const int b = static_cast<int>(blockIdx.x) - (pi ? a.begin1 : 0);
-  const int slices = a.slices[pi], rb = b / slices, slice = b - rb * slices;
+  const ppo_mlp_problem& P = a.g.p;
+  const int b = static_cast<int>(blockIdx.x), rb = b / a.slices, slice = b - rb * a.slices;
   const int64_t row0 = static_cast<int64_t>(rb) * kMlpRows, rows = a.g.rows;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int ldx = a.g.ldx;
   float* x = lds;
   float* y = lds + kMlpRows * ldx;
-  if (a.l0 >= P.num_layers) return;  // (the other problem has more layers)
-  if (a.in[pi] == nullptr) {
+  if (a.in == nullptr) {
     mlp_input(P, x, ldx, row0, rows, tid);
   } else {  // a previous launch's rows, whole 16-byte pieces
     const int K = P.layers[a.l0].in_features, pieces = (K + 15) / 16 * 4;
-    const int64_t ld = a.ld[pi];
+    const int64_t ld = a.ld;
     for (int i = tid; i < kMlpRows * pieces; i += kMlpThreads) {
       const int r = i / pieces, c = 4 * (i - r * pieces);
-      const f32x4 v = *reinterpret_cast<const f32x4*>(a.in[pi] + min(row0 + r, rows - 1) * ld + min(c, static_cast<int>(ld) - 4));
+      const f32x4 v = *reinterpret_cast<const f32x4*>(a.in + min(row0 + r, rows - 1) * ld + min(c, static_cast<int>(ld) - 4));
       f32x4 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = c + e < K ? v[e] : 0.0f;
@@ -246,44 +241,37 @@ __global__ __launch_bounds__(kMlpThreads) __attribute__((amdgpu_waves_per_eu(4, 
   const bool last = l == P.num_layers - 1;
   const int t0 = slice * kSliceTiles, t1 = min(t0 + kSliceTiles, mlp_tiles(P.layers[l]));
   mlp_run_layer<true>(P.layers[l], last ? PPO_ACT_NONE : P.activation, x, ldx,
-                      {nullptr, last ? P.out : a.to[pi], last ? P.ldo : a.ld[pi], row0, rows}, t0, t1, wave, lane);
+                      {nullptr, last ? P.out : a.to, last ? P.ldo : a.ld, row0, rows}, t0, t1, wave, lane);
 }
 
 int64_t round16(int64_t n) { return (n + 15) / 16 * 16; }
 
-// The checked problems as kernel arguments.
-int mlp_group(const ppo_mlp_problem* problems, int32_t count, int64_t rows, const char* who, MlpGroup& g) {
-  int64_t widest = 0;
-  PPO_REQUIRE(problems != nullptr && count >= 1 && count <= PPO_MAX_MLP_PROBLEMS, "%s: count=%d outside [1, %d]", who,
-              count, PPO_MAX_MLP_PROBLEMS);
+// The checked problem as kernel arguments.
+int mlp_args(const ppo_mlp_problem* problem, int64_t rows, const char* who, MlpArgs& g) {
+  int64_t widest = 0, width = 0;
+  PPO_REQUIRE(problem != nullptr, "%s: no problem", who);
   PPO_REQUIRE(rows > 0 && rows <= INT32_MAX / 4, "%s: rows=%lld", who, (long long)rows);
-  for (int i = 0; i < count; ++i) {
-    const ppo_mlp_problem& q = problems[i];
-    PPO_REQUIRE(q.num_blocks >= 1 && q.num_blocks <= PPO_MAX_MLP_BLOCKS && q.num_layers >= 1 &&
-                    q.num_layers <= PPO_MAX_MLP_LAYERS,
-                "%s: problem %d: %d input blocks (at most %d), %d layers (at most %d)", who, i, q.num_blocks,
-                PPO_MAX_MLP_BLOCKS, q.num_layers, PPO_MAX_MLP_LAYERS);
-    PPO_REQUIRE(q.activation >= PPO_ACT_NONE && q.activation < PPO_ACT_COUNT, "%s: activation=%d", who, q.activation);
-    PPO_REQUIRE((q.norm_mean == nullptr) == (q.norm_std == nullptr), "%s: problem %d: one of mean / std", who, i);
-    int64_t width = 0;
-    for (int s = 0; s < q.num_blocks; ++s) {
-      PPO_REQUIRE(q.x[s].src && q.x[s].width > 0 && q.x[s].stride >= q.x[s].width, "%s: problem %d: input block %d",
-                  who, i, s);
-      width += q.x[s].width;
-    }
-    for (int l = 0; l < q.num_layers; ++l) {
-      const ppo_mlp_layer& L = q.layers[l];
-      PPO_REQUIRE(L.w && L.b && L.in_features == width && L.out_features > 0,
-                  "%s: problem %d layer %d: %d -> %d features after %lld", who, i, l, L.in_features, L.out_features,
-                  (long long)width);
-      if (width > kMlpMaxWidth) return fail(PPO_EUNSUPPORTED, "%s: layers of at most %d features", who, kMlpMaxWidth);
-      widest = std::max(widest, width);
-      width = L.out_features;
-    }
-    PPO_REQUIRE(q.out && q.ldo >= width, "%s: problem %d output", who, i);
-    g.p[i] = q;
+  const ppo_mlp_problem& q = *problem;
+  PPO_REQUIRE(q.num_blocks >= 1 && q.num_blocks <= PPO_MAX_MLP_BLOCKS && q.num_layers >= 1 &&
+                  q.num_layers <= PPO_MAX_MLP_LAYERS,
+              "%s: %d input blocks (at most %d), %d layers (at most %d)", who, q.num_blocks, PPO_MAX_MLP_BLOCKS,
+              q.num_layers, PPO_MAX_MLP_LAYERS);
+  PPO_REQUIRE(q.activation >= PPO_ACT_NONE && q.activation < PPO_ACT_COUNT, "%s: activation=%d", who, q.activation);
+  PPO_REQUIRE((q.norm_mean == nullptr) == (q.norm_std == nullptr), "%s: one of mean / std", who);
+  for (int s = 0; s < q.num_blocks; ++s) {
+    PPO_REQUIRE(q.x[s].src && q.x[s].width > 0 && q.x[s].stride >= q.x[s].width, "%s: input block %d", who, s);
+    width += q.x[s].width;
   }
-  g.count = count;
+  for (int l = 0; l < q.num_layers; ++l) {
+    const ppo_mlp_layer& L = q.layers[l];
+    PPO_REQUIRE(L.w && L.b && L.in_features == width && L.out_features > 0,
+                "%s: layer %d: %d -> %d features after %lld", who, l, L.in_features, L.out_features, (long long)width);
+    if (width > kMlpMaxWidth) return fail(PPO_EUNSUPPORTED, "%s: layers of at most %d features", who, kMlpMaxWidth);
+    widest = std::max(widest, width);
+    width = L.out_features;
+  }
+  PPO_REQUIRE(q.out && q.ldo >= width, "%s: output", who);
+  g.p = q;
   g.rows = rows;
   g.blocks = static_cast<int>(ceil_div(rows, static_cast<int64_t>(kMlpRows)));
   // rows of whole 64 floats plus 4: a 16-byte read of the same columns of 16 rows falls on all 64 banks
@@ -292,7 +280,7 @@ int mlp_group(const ppo_mlp_problem* problems, int32_t count, int64_t rows, cons
 }
 
 template <typename K, typename A>
-int launch_mlp(K kernel, int64_t blocks, const MlpGroup& g, const A& args, hipStream_t s, const char* name) {
+int launch_mlp(K kernel, int64_t blocks, const MlpArgs& g, const A& args, hipStream_t s, const char* name) {
   const size_t lds = 2 * static_cast<size_t>(kMlpRows) * g.ldx * sizeof(float);
   if (lds > 64 * 1024)
     PPO_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -302,7 +290,7 @@ int launch_mlp(K kernel, int64_t blocks, const MlpGroup& g, const A& args, hipSt
   return check_launch(name);
 }
 
-// Floats per row of one of a problem's two intermediate buffers: its widest layer of odd index but the last (0: none).
+// Floats per row of one of the two intermediate buffers: the widest layer of odd index but the last (0: none).
 int64_t pairs_width(const ppo_mlp_problem& q) {
   int64_t w = 0;
   for (int l = 1; l + 1 < q.num_layers && l < PPO_MAX_MLP_LAYERS; l += 2)
@@ -315,52 +303,35 @@ int64_t pairs_width(const ppo_mlp_problem& q) {
 
 using namespace ppo;
 
-extern "C" int ppo_mlp_fwd(const ppo_mlp_problem* problems, int32_t count, int64_t rows, ppo_stream_t stream) {
-  MlpGroup g{};
-  if (int rc = mlp_group(problems, count, rows, "ppo_mlp_fwd", g)) return rc;
-  return launch_mlp(mlp_fwd_kernel, static_cast<int64_t>(count) * g.blocks, g, g, static_cast<hipStream_t>(stream),
-                    "mlp_fwd_kernel");
+extern "C" int ppo_mlp_fwd(const ppo_mlp_problem* problem, int64_t rows, ppo_stream_t stream) {
+  MlpArgs g{};
+  if (int rc = mlp_args(problem, rows, "ppo_mlp_fwd", g)) return rc;
+  return launch_mlp(mlp_fwd_kernel, g.blocks, g, g, static_cast<hipStream_t>(stream), "mlp_fwd_kernel");
 }
 
-extern "C" size_t ppo_mlp_fwd_pairs_workspace_bytes(const ppo_mlp_problem* problems, int32_t count, int64_t rows) {
-  if (problems == nullptr || count < 1 || count > PPO_MAX_MLP_PROBLEMS || rows <= 0) return 0;
-  int64_t floats = 0;
-  for (int i = 0; i < count; ++i) floats += 2 * pairs_width(problems[i]);
-  return static_cast<size_t>(floats) * static_cast<size_t>(rows) * sizeof(float);
+extern "C" size_t ppo_mlp_fwd_pairs_workspace_bytes(const ppo_mlp_problem* problem, int64_t rows) {
+  if (problem == nullptr || rows <= 0) return 0;
+  return 2 * static_cast<size_t>(pairs_width(*problem)) * static_cast<size_t>(rows) * sizeof(float);
 }
 
-extern "C" int ppo_mlp_fwd_pairs(const ppo_mlp_problem* problems, int32_t count, int64_t rows, void* workspace,
-                                 size_t workspace_bytes, ppo_stream_t stream) {
+extern "C" int ppo_mlp_fwd_pairs(const ppo_mlp_problem* problem, int64_t rows, void* workspace, size_t workspace_bytes,
+                                 ppo_stream_t stream) {
   MlpPairs a{};
-  if (int rc = mlp_group(problems, count, rows, "ppo_mlp_fwd_pairs", a.g)) return rc;
-  const size_t need = ppo_mlp_fwd_pairs_workspace_bytes(problems, count, rows);
+  if (int rc = mlp_args(problem, rows, "ppo_mlp_fwd_pairs", a.g)) return rc;
+  const ppo_mlp_problem& q = *problem;
+  const size_t need = ppo_mlp_fwd_pairs_workspace_bytes(problem, rows);
   PPO_REQUIRE(need == 0 || (workspace != nullptr && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0),
               "ppo_mlp_fwd_pairs: workspace of %zu bytes (%zu, 16-byte aligned, needed)", workspace_bytes, need);
-  float* buf[PPO_MAX_MLP_PROBLEMS][2] = {};
-  int layers = 0;
-  float* ws = static_cast<float*>(workspace);
-  for (int i = 0; i < count; ++i) {
-    a.ld[i] = pairs_width(problems[i]);
-    for (int k = 0; k < 2; ++k) {
-      buf[i][k] = ws;
-      if (ws != nullptr) ws += rows * a.ld[i];
-    }
-    layers = std::max(layers, problems[i].num_layers);
-  }
-  for (int l0 = 0, p = 0; l0 < layers; l0 += 2, ++p) {
-    int64_t blocks = 0;
-    for (int i = 0; i < count; ++i) {
-      const ppo_mlp_problem& q = problems[i];
-      const int l = std::min(l0 + 1, q.num_layers - 1);  // the sliced layer
-      a.in[i] = p == 0 ? nullptr : buf[i][(p - 1) & 1];
-      a.to[i] = buf[i][p & 1];
-      a.slices[i] = static_cast<int>(ceil_div(ceil_div(q.layers[l].out_features, 16), kSliceTiles));
-      if (i == 1) a.begin1 = static_cast<int>(blocks);
-      if (l0 < q.num_layers) blocks += static_cast<int64_t>(a.g.blocks) * a.slices[i];
-      PPO_REQUIRE(blocks <= INT32_MAX, "ppo_mlp_fwd_pairs: too many rows");
-    }
-    if (count == 1) a.begin1 = INT32_MAX;
+  a.ld = pairs_width(q);
+  float* const ws = static_cast<float*>(workspace);
+  float* const buf[2] = {ws, ws == nullptr ? nullptr : ws + rows * a.ld};
+  for (int l0 = 0, p = 0; l0 < q.num_layers; l0 += 2, ++p) {
+    const int l = std::min(l0 + 1, q.num_layers - 1);  // the sliced layer
+    a.in = p == 0 ? nullptr : buf[(p - 1) & 1];
+    a.to = buf[p & 1];
+    a.slices = static_cast<int>(ceil_div(ceil_div(q.layers[l].out_features, 16), kSliceTiles));
     a.l0 = l0;
+    const int64_t blocks = static_cast<int64_t>(a.g.blocks) * a.slices;
     if (int rc = launch_mlp(mlp_pairs_kernel, blocks, a.g, a, static_cast<hipStream_t>(stream), "mlp_pairs_kernel")) return rc;
   }
   return PPO_OK;

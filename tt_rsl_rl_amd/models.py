@@ -415,7 +415,7 @@ class MLPModel(nn.Module):
             if norm is not None:
                 rec.norm_mean, rec.norm_std, rec.norm_eps = norm._mean.data_ptr(), norm._std.data_ptr(), norm.eps
             if second >= PAIR_WEIGHTS:
-                per_row = L.load().ppo_mlp_fwd_pairs_workspace_bytes(ops.C_ref(rec), 1, 1)
+                per_row = L.load().ppo_mlp_fwd_pairs_workspace_bytes(ops.C_ref(rec), 1)
             route = _Route.of([shapes[0][1], *[w[0] for w in shapes[0:2 * len(layers):2]]])
         self._fused = _FusedRecord((key, rec, per_row, route))
         return self._fused, tensors
@@ -451,9 +451,9 @@ class MLPModel(nn.Module):
         if by == "pairs":
             nbytes = rows * per_row
             ws = torch.empty(nbytes, dtype=torch.uint8, device=out.device)
-            L.call("ppo_mlp_fwd_pairs", ops.C_ref(rec), 1, rows, ws.data_ptr(), nbytes, stream)
+            L.call("ppo_mlp_fwd_pairs", ops.C_ref(rec), rows, ws.data_ptr(), nbytes, stream)
         else:
-            L.call("ppo_mlp_fwd", ops.C_ref(rec), 1, rows, stream)
+            L.call("ppo_mlp_fwd", ops.C_ref(rec), rows, stream)
         return out
 
     def mlp_forward(self, latent: torch.Tensor) -> torch.Tensor:

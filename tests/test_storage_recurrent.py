@@ -65,3 +65,26 @@ def test_recurrent_generator_partition_errors():
     mine, _ = _fill()
     with pytest.raises(ValueError):
         next(mine.recurrent_mini_batch_generator(8))
+
+
+def test_hidden_states_are_saved_through_upstreams_method():
+    """A subclass's _save_hidden_states takes the states alone, as upstream's does, and the method works by itself."""
+    n, h = 6, 8
+
+    class Own(RolloutStorage):
+        seen = 0
+
+        def _save_hidden_states(self, hidden_states):
+            self.seen += 1
+            super()._save_hidden_states(hidden_states)
+
+    st = Own("rl", n, 2, {"policy": torch.zeros(n, 3)}, [2], device="cpu")
+    states = tuple(torch.randn(1, n, h) for _ in range(2)), torch.randn(1, n, h)
+    tr = RolloutStorage.Transition()
+    tr.observations, tr.actions, tr.values = {"policy": torch.randn(n, 3)}, torch.randn(n, 2), torch.randn(n, 1)
+    tr.rewards, tr.dones, tr.actions_log_prob = torch.randn(n), torch.zeros(n), torch.randn(n)
+    tr.distribution_params, tr.hidden_states = (torch.randn(n, 2), torch.ones(n, 2)), states
+    st.add_transition(tr)
+    assert st.seen == 1 and torch.equal(st.saved_hidden_state_a[1][0], states[0][1])
+    st._save_hidden_states(states)
+    assert torch.equal(st.saved_hidden_state_c[0][1], states[1])

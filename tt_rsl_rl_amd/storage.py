@@ -93,6 +93,7 @@ class RolloutStorage:
         self.advantages = torch.zeros(T, N, 1, device=self.device)
         self.saved_hidden_state_a = None
         self.saved_hidden_state_c = None
+        self._writes: ops.RowStores | None = None  # the transition's writes while add_transition gathers them
         self.step = 0
 
     def add_transition(self, transition: "RolloutStorage.Transition", bootstrap: "Bootstrap | None" = None) -> None:
@@ -103,21 +104,24 @@ class RolloutStorage:
         s = self.step
         if self.distribution_params is None:
             self._interleave(transition.distribution_params)
-        w = ops.RowStores(self.device)
-        for k in self.observations:
-            w.copy(self.observations[k][s], transition.observations[k])
-        w.copy(self.actions[s], transition.actions)
-        if bootstrap is None:
-            w.copy(self.rewards[s], transition.rewards.view(-1, 1))
-        else:
-            w.bootstrap(self.rewards[s], transition.rewards, *bootstrap)
-        w.copy(self.dones[s], transition.dones.view(-1, 1))
-        w.copy(self.values[s], transition.values)
-        w.copy(self.actions_log_prob[s], transition.actions_log_prob.view(-1, 1))
-        for i, p in enumerate(transition.distribution_params):
-            w.copy(self.distribution_params[i][s], p)
-        self._save_hidden_states(transition.hidden_states, w)
-        w.flush()
+        w = self._writes = ops.RowStores(self.device)
+        try:
+            for k in self.observations:
+                w.copy(self.observations[k][s], transition.observations[k])
+            w.copy(self.actions[s], transition.actions)
+            if bootstrap is None:
+                w.copy(self.rewards[s], transition.rewards.view(-1, 1))
+            else:
+                w.bootstrap(self.rewards[s], transition.rewards, *bootstrap)
+            w.copy(self.dones[s], transition.dones.view(-1, 1))
+            w.copy(self.values[s], transition.values)
+            w.copy(self.actions_log_prob[s], transition.actions_log_prob.view(-1, 1))
+            for i, p in enumerate(transition.distribution_params):
+                w.copy(self.distribution_params[i][s], p)
+            self._save_hidden_states(transition.hidden_states)
+            w.flush()
+        finally:
+            self._writes = None
         self.step += 1
 
     def _interleave(self, params) -> None:
@@ -138,7 +142,7 @@ class RolloutStorage:
         else:
             self.distribution_params = tuple(torch.zeros(T, *p.shape, device=self.device) for p in params)
 
-    def _save_hidden_states(self, hidden_states, writes: ops.RowStores) -> None:
+    def _save_hidden_states(self, hidden_states) -> None:
         """rollout_storage.py:333-359: the recurrent models' state before each step's forward, as saved_hidden_state_a /
         _c = [h, c] each [T, num_layers, N, H] (zero where a model had no state yet)."""
         if hidden_states is None or hidden_states == (None, None):
@@ -152,7 +156,10 @@ class RolloutStorage:
             if getattr(self, name) is None:
                 setattr(self, name, [torch.zeros(T, *h.shape, device=self.device) for h in hs])
             for buf, h in zip(getattr(self, name), hs):
-                writes.copy(buf[self.step], h)
+                if self._writes is None:  # (called by itself)
+                    buf[self.step].copy_(h)
+                else:
+                    self._writes.copy(buf[self.step], h)
 
     def clear(self) -> None:
         self.step = 0

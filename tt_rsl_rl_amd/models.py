@@ -388,7 +388,7 @@ class MLPModel(nn.Module):
         """The cached (key, record, workspace bytes per row by pairs, route) of this model, the record None where
         ppo_mlp_fwd does not take the layers, and the tensors the record points into, which the caller holds until its
         launch (a parametrised weight is a new tensor on each access).  Kept from call to call, rebuilt when anything it was
-        made from changed: a tensor's address, shape, strides or type, the activation, the normaliser's eps."""
+        made from changed: a tensor's address, shape, layout or type, the activation, the normaliser's eps."""
         layers = [m for m in self.mlp if isinstance(m, nn.Linear)]
         tensors = [t for l in layers for t in (l.weight, l.bias)]
         if norm is not None:
@@ -396,7 +396,7 @@ class MLPModel(nn.Module):
         if any(t is None for t in tensors):
             return (None, None, 0, None), tensors
         key = (self.act_code, None if norm is None else norm.eps,
-               *[(t.data_ptr(), t.shape, t.stride(), t.dtype) for t in tensors])
+               *[(t.data_ptr(), t.shape, t.is_contiguous(), t.dtype) for t in tensors])
         if self._fused is not None and self._fused[0] == key:
             return self._fused, tensors
         rec, per_row, route = None, 0, None

@@ -306,6 +306,11 @@ _STOCHASTIC = frozenset(("forward", "get_output_log_prob", "update", "sample", "
                          "deterministic_output"))
 
 
+# methods that a call of a model goes through
+_LATENT = frozenset(("get_latent", "latent_into", "mlp_forward"))
+_FORWARD = _LATENT | {"__call__", "forward"}
+
+
 class _FusedRecord(tuple):
     """(what it was built from, the ppo_mlp_fwd record, workspace bytes per row, the _Route).  The record holds pointers:
     a copied or pickled model starts without one."""
@@ -365,6 +370,19 @@ class MLPModel(nn.Module):
     def linears(self) -> list[nn.Linear]:
         return [m for m in self.mlp if isinstance(m, nn.Linear)]
 
+    def _weights(self) -> list[tuple]:
+        """(weight, bias) of the linear layers, each as a call of its layer takes it (a parametrised one, of another class,
+        computes it)."""
+        out = []
+        for m in self.mlp._modules.values():
+            if type(m) is nn.Linear:  # (past nn.Module's attribute lookup: 5 us of a forward)
+                p = m._parameters
+                w, b = p.get("weight"), p.get("bias")
+                out.append((m.weight if w is None else w, m.bias if b is None else b))
+            elif isinstance(m, nn.Linear):
+                out.append((m.weight, m.bias))
+        return out
+
     # -- forward on the GPU ------------------------------------------------------------------------------------------
     def latent_into(self, obs: Mapping, out: torch.Tensor) -> None:
         """Concatenate this model's observation groups into ``out`` [rows, obs_dim], normalised if enabled."""
@@ -389,8 +407,8 @@ class MLPModel(nn.Module):
         ppo_mlp_fwd does not take the layers, and the tensors the record points into, which the caller holds until its
         launch (a parametrised weight is a new tensor on each access).  Kept from call to call, rebuilt when anything it was
         made from changed: a tensor's address, shape, layout or type, the activation, the normaliser's eps."""
-        layers = [m for m in self.mlp if isinstance(m, nn.Linear)]
-        tensors = [t for l in layers for t in (l.weight, l.bias)]
+        layers = self._weights()
+        tensors = [t for wb in layers for t in wb]
         if norm is not None:
             tensors += [norm._mean, norm._std]
         if any(t is None for t in tensors):
@@ -466,16 +484,15 @@ class MLPModel(nn.Module):
 
     def _mlp_layers(self, latent: torch.Tensor) -> torch.Tensor:
         rows = latent.shape[0]
-        lin = self.linears
-        widths = [l.out_features for l in lin[:-1]]
-        bufs = self._fwd.get(rows, widths, latent.device)
+        lin = self._weights()
+        bufs = self._fwd.get(rows, [w.shape[0] for w, _ in lin[:-1]], latent.device)
         x = latent
-        for i, l in enumerate(lin[:-1]):
-            h = bufs[i]  # hidden layers: only act(z) is needed
-            ops.linear_fwd([(x, l.weight, l.bias, None, h)], rows, act=self.act_code)
+        for (w, b), h in zip(lin, bufs):  # hidden layers: only act(z) is needed
+            ops.linear_fwd([(x, w, b, None, h)], rows, act=self.act_code)
             x = h
-        out = torch.empty(rows, lin[-1].out_features, device=latent.device)
-        ops.linear_fwd([(x, lin[-1].weight, lin[-1].bias, out, None)], rows, act=L.PPO_ACT_NONE)
+        w, b = lin[-1]
+        out = torch.empty(rows, w.shape[0], device=latent.device)
+        ops.linear_fwd([(x, w, b, out, None)], rows, act=L.PPO_ACT_NONE)
         return out
 
     def get_latent(self, obs: Mapping, masks=None, hidden_state=None) -> torch.Tensor:
@@ -488,7 +505,7 @@ class MLPModel(nn.Module):
         if masks is not None:
             raise NotImplementedError("padded (recurrent) batches are not supported by the MLP HIP path")
         out = None
-        if self._own(MLPModel, "get_latent", "latent_into", "mlp_forward"):
+        if self._own(MLPModel, _LATENT):
             cols = [obs[g] for g in self.obs_groups]
             if all(x.is_cuda and x.dim() == 2 for x in cols):
                 out = self._fused_forward(cols, self.obs_normalizer if self.obs_normalization else None)
@@ -501,9 +518,10 @@ class MLPModel(nn.Module):
             return self.distribution.deterministic_output(out)
         return out
 
-    def _own(self, cls: type, *names: str) -> bool:
+    def _own(self, cls: type, names: frozenset) -> bool:
         """These methods are `cls`'s: neither a subclass nor the instance has one of its own."""
-        return all(getattr(type(self), n) is getattr(cls, n) and n not in self.__dict__ for n in names)
+        mine = type(self)
+        return (mine is cls or all(getattr(mine, n) is getattr(cls, n) for n in names)) and names.isdisjoint(self.__dict__)
 
     def _called_directly(self) -> bool:
         """Nothing stands between a call of this model and its forward: no hook, no compiled call."""
@@ -522,7 +540,7 @@ class MLPModel(nn.Module):
         gives, but for the rounding)."""
         cls = RNNModel if isinstance(self, RNNModel) else MLPModel
         return self._called_directly() and \
-            self._own(cls, "__call__", "forward", "get_latent", "latent_into", "mlp_forward") and \
+            self._own(cls, _FORWARD) and \
             (self.distribution is None or (type(self.distribution) is GaussianDistribution and
                                            _STOCHASTIC.isdisjoint(self.distribution.__dict__)))
 

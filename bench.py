@@ -35,13 +35,15 @@ PEAK_FP32_MFMA_TFLOPS = 157.3
 # ceiling, in algorithmic fp32 FLOP/s, is the dense bf16 MFMA peak (2.5 PFLOP/s) over six.
 PEAK_BF16_MFMA_TFLOPS = 2500.0
 PEAK_BX6_TFLOPS = PEAK_BF16_MFMA_TFLOPS / 6
+# fp16x3 (mini-batches of engine.RANGED_ROWS rows and more): three fp16 MFMA products, at the bf16 ones' rate
+PEAK_F16X3_TFLOPS = PEAK_BF16_MFMA_TFLOPS / 3
 PEAK_HBM_GBS = 8000.0
 
 
 def dw_arith(engine, R: int) -> str:
-    """Arithmetic of the weight-grad launch: the bf16x6 kernel runs when every problem's operands (dz and the layer
-    input) have 16-byte aligned rows, else the fp32-MFMA kernel (the library's own rule, restated on the operands the
-    engine passes)."""
+    """Arithmetic of the weight-grad launch: the bf16x6 kernel (fp16x3 where the engine gives the operands' ranges) runs
+    when every problem's operands (dz and the layer input) have 16-byte aligned rows, else the fp32-MFMA kernel (the
+    library's own rule, restated on the operands the engine passes)."""
     tab = engine.table[:R]
     lay = engine.layout
     alg = engine.alg
@@ -55,7 +57,7 @@ def dw_arith(engine, R: int) -> str:
     else:
         ops = [(dz, x) for dz, x, *_ in engine.head_dw(xa, xc, R)]
     aligned = all(t.data_ptr() % 16 == 0 and t.stride(0) % 4 == 0 for pair in ops for t in pair)
-    return "bf16x6" if aligned else "fp32"
+    return "fp32" if not aligned else "fp16x3" if engine.ranged else "bf16x6"
 
 
 def _sample_obs(workload, n, device, gen):
@@ -474,12 +476,15 @@ def main() -> int:
         ach = flops[dom] / (t * 1e-3) / 1e12
         arith = dw_arith(engine, R) if dom in ("dw", "lstm_dw") else "fp32"
         if arith == "bf16x6" and args.mixed_precision:
-            arith = "bf16"  # (the same kernels at one bf16 product per k-group)
-        peak = {"bf16x6": PEAK_BX6_TFLOPS, "bf16": PEAK_BF16_MFMA_TFLOPS}.get(arith, PEAK_FP32_MFMA_TFLOPS)
+            arith = "bf16"  # (one bf16 product per k-group)
+        peak = {"bf16x6": PEAK_BX6_TFLOPS, "fp16x3": PEAK_F16X3_TFLOPS,
+                "bf16": PEAK_BF16_MFMA_TFLOPS}.get(arith, PEAK_FP32_MFMA_TFLOPS)
         roofline = {"bound": "mfma", "achieved": round(ach, 2), "peak": round(peak, 2), "unit": "TFLOP/s",
                     "frac": round(ach / peak, 4), "traffic": load_traffic(args.workload, dom), "kernel": dom,
                     "arith": arith, "peak_basis": {"bf16x6": "bf16 dense MFMA 2.5 PFLOP/s / 6 products per fp32 "
-                                                             "product", "bf16": "bf16 dense MFMA 2.5 PFLOP/s"}.get(
+                                                             "product", "fp16x3": "fp16 dense MFMA 2.5 PFLOP/s / 3 "
+                                                             "products per fp32 product",
+                                                   "bf16": "bf16 dense MFMA 2.5 PFLOP/s"}.get(
                                                        arith, "fp32 dense MFMA"),
                     "frac_of_fp32_mfma_peak": round(ach / PEAK_FP32_MFMA_TFLOPS, 4),
                     "flops_per_launch": flops[dom], "mean_launch_ms": round(t, 5), "launches_timed": n}
@@ -509,6 +514,9 @@ def main() -> int:
         "gemm_arith": ("use_mixed_precision: the layers' GEMMs with bf16 operands (rounded to nearest even), one bf16 "
                        "MFMA product, fp32 accumulation and results; loss, head and optimiser in fp32"
                        if args.mixed_precision else
+                       "fp32 operands and results; GEMMs with 16-byte aligned operand rows and k of at least 64 as fp16x3 "
+                       "(two scaled fp16 parts per operand, three fp16 MFMA products, fp32 accumulation; bf16x6 where an "
+                       "operand's parts lie too far apart), the rest as bf16x6 or on fp32 MFMA" if engine.ranged else
                        "fp32 operands and results; GEMMs with 16-byte aligned operand rows as bf16x6 (three bf16 "
                        "parts per operand, six bf16 MFMA products, fp32 accumulation), the rest on fp32 MFMA"),
         "config": {"workload": f"{args.workload}: {lstm}{len(W.linear_shapes(workload)[0])}-layer actor/critic MLPs "

@@ -37,7 +37,7 @@ DESC = {
                "x 4 env-slice mini-batches of 1024 envs)",
 }
 # the kernels each candidate dominant phase launches once per mini-batch (name prefix; the largest grid of that name)
-PHASES_MLP = {"dw": ["gemm_tn_bx6_kernel", "dw_reduce_kernel"]}
+PHASES_MLP = {"dw": [("gemm_tn_bx6_kernel", "gemm_tn_f16_kernel"), "dw_reduce_kernel"]}  # (fp16x3 for large mini-batches)
 PHASES_LSTM = {"lstm_fwd": ["lstm_pack_kernel", "gemm_nt_bx6_kernel", "lstm_seq_fwd_kernel"],
                "lstm_bwd": ["lstm_seq_bwd_kernel"],
                "lstm_dw": ["gemm_tn_bx6_kernel", "dw_reduce_kernel", "lstm_unpack_kernel"]}

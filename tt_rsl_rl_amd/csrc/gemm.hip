@@ -1,7 +1,8 @@
 // A6 linear layers (rsl_rl/modules/mlp.py:27-95; autograd of nn.Linear / nn.ELU) as fp32-accurate MFMA GEMMs for
 // gfx950.  Launches whose operands all have 16-byte rows run the bf16x6 kernels of gemm_core.hpp (each fp32 operand
-// split into three bf16 parts, six bf16 MFMA products per fp32 product, fp32 accumulation); the others run the fp32
-// MFMA kernels described here.
+// split into three bf16 parts, six bf16 MFMA products per fp32 product, fp32 accumulation), or where the operands' ranges
+// are given the fp16x3 kernels of gemm_f16.hpp (two scaled fp16 parts, three products), which also hold the one-product
+// bf16-operand mode; the others run the fp32 MFMA kernels described here.
 //
 // Two fp32 kernel families, both 256 threads = 4 wavefronts in a 2 x 2 arrangement over a BM x BN output tile, each
 // wave owning (BM/2) x (BN/2) of 32 x 32 v_mfma_f32_32x32x2f32 accumulators, both fed by gfx950's direct
@@ -183,9 +184,9 @@ __global__ __launch_bounds__(256) void transpose_kernel(const TransposeGroup g) 
   }
 }
 
-// Below this k the two-part split's own error (7e-8 of a product, root mean square) is more than what bf16x6's six
-// roundings per k-group add up to: relative errors against fp64 of 7.3e-8 / 3.8e-8 (fp16x3 / bf16x6) at k = 16, 7.2e-8 /
-// 7.0e-8 at 48, 8.0e-8 / 1.0e-7 at 96, 1.2e-7 / 2.4e-7 at 512.
+// fp16x3 only where its error is below bf16x6's: the two-part split's own (7e-8 of a product, root mean square) against the
+// six roundings per k-group.  Relative errors against fp64 of 7.3e-8 / 3.8e-8 (fp16x3 / bf16x6) at k = 16, 7.2e-8 / 7.0e-8 at
+// 48, 8.0e-8 / 1.0e-7 at 96, 1.2e-7 / 2.4e-7 at 512: equal at about 48, the next whole slab pair above is the line.
 constexpr int kF16MinK = 64;
 
 // Weight-grad: 128 x 128 tiles; split-K over the rows, in chunks that are multiples of the deepest (64-row) slab.
@@ -235,8 +236,8 @@ struct DwPlan {
 // the bf16x6 kernel, which its products bound, it gets half the splits of the others (every block of the launch then has
 // about the same work).  In the fp16x3 kernel, half as many products, a slab takes a narrow tile as long as a full one
 // (loads, barrier), and with half the splits its blocks ran on alone: compute units busy 68 % of 2,017 us (flat48 with
-// 393,216 rows per mini-batch; the update 112.7 ms).  As many splits as the others: the update 104.4 ms (three quarters
-// of them: 105.6 ms, 1,517 us).
+// 393,216 rows per mini-batch; the update 112.7 ms).  As many splits as the others: 1,650 us, the update 104.4 ms; three
+// quarters of them did not measure apart (105.6 ms, within the runs' spread).
 bool dw_narrow(const ppo_linear_bwd_dw_problem& q) { return q.in_features <= kDwBN / 2; }
 
 // `weight` and `share`: a narrow tile's work and its problem's split count, in quarters of a full one's.

@@ -9,8 +9,9 @@
 // into the MFMA operand registers, 64 k ahead, and nothing is written but the output: one launch of 33 us for 16 to
 // 2,048 rows, 34 for 4,096 (the layers one by one 64 us).  16 rows give 4,096 rows 256 blocks, one per
 // compute unit.  v_mfma_f32_16x16x4f32 with the weights as the first operand leaves each lane 4 consecutive outputs of one
-// row: one 16-byte LDS store each.  Past some thousands of rows the layers' own GEMMs (weights read once per 128 rows, bf16
-// matrix cores) are faster: the caller's choice.
+// row: one 16-byte LDS store each.  Past some thousands of rows, and for networks of more weights than those launches' time
+// (every block reads all of them; _Route in models.py), the layers' own GEMMs (weights read once per 128 rows, bf16 matrix
+// cores) are faster: the caller's choice.
 #include "gemm_core.hpp"
 
 namespace ppo {

@@ -36,11 +36,12 @@ K_SLACK = 16
 
 
 # Mini-batches of at least this many rows run their GEMMs as fp16x3 (two fp16 parts per operand, csrc/gemm_f16.hpp), the
-# others as bf16x6.  fp16x3 is the faster and the closer to fp64 at every size (24,576 rows, humanoid: 8.9 against 10.0
-# ms per update; weight-grads of 393,216 rows: 4e-7 relative error against 2e-6).  What the line keeps is the trajectory
-# of smaller updates: any other rounding puts a row now and then on the other side of a clip boundary, which moves that
-# step's gradient by about 1 / sqrt(rows), and twenty steps carry it on (humanoid, 16 seeds, two updates: first moments
-# up to 4.5e-2 apart on 8 of them; 393,216 rows: 8e-4 at most on 4).  1 / sqrt(40,000) is 5e-3.
+# others as bf16x6.  The line is one of compatibility, not of speed: fp16x3 is the faster and the closer to fp64 below it as
+# well (24,576 rows, humanoid: 8.9 against 10.0 ms per update; weight-grads of 393,216 rows: 4e-7 relative error against
+# 2e-6), but any other rounding puts a row now and then on the other side of a clip boundary, which moves that step's
+# gradient by about 1 / sqrt(rows), and twenty steps carry it on (humanoid, 16 seeds, two updates: first moments up to
+# 4.5e-2 apart on 8 of them; 393,216 rows: 8e-4 at most on 4).  40,000 is where 1 / sqrt(rows) is the 5e-3 that
+# perf/cases.py allows an update of several steps; smaller updates keep the trajectory they had.
 RANGED_ROWS = 40_000
 
 

@@ -280,8 +280,9 @@ class PPO:
     def compute_returns(self, obs: Mapping) -> None:
         """ppo.py:166-191: bootstrap value, GAE scan and global advantage normalisation on the GPU."""
         critic_hidden_state = self.critic.get_hidden_state()
-        # layer by layer at every size: the bootstrap value enters every advantage, and its rounding (another one in the
-        # one-launch forward that act() uses) is carried through all of the update's steps (see RANGED_ROWS in engine.py)
+        # layer by layer at every size, the rounding it has always had: the bootstrap value enters every advantage, and
+        # another rounding (the one-launch forward's, which act() uses) is carried through all of the update's steps (see
+        # RANGED_ROWS in engine.py)
         # where something stands between (a hook, a compiled call, a method of the user's own), the call itself
         plain = isinstance(self.critic, MLPModel) and self.critic.forwards_plainly()
         last_values = (self.critic.forward_layers(obs) if plain else self.critic(obs)).detach().contiguous()

@@ -285,7 +285,7 @@ _SIGNATURES = [
 ]
 
 EXPORTED_SYMBOLS = [name for name, _, _ in _SIGNATURES]
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 _lib: C.CDLL | None = None
 

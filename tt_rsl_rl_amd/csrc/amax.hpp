@@ -40,8 +40,12 @@ __device__ __forceinline__ uint32_t part_code(uint32_t u) { return u == 0 ? 0u :
 // the others (a sentinel in one row, a column of another unit) would cost the others their digits: to 2^-22 of a part 2^28
 // below the largest, whence kMaxSpread.  The parts of the inputs and the weights are single rows and columns, those of
 // activations and gradients the tiles of the waves that write them (16 to 64 rows): an outlier there comes of one in the
-// inputs or the weights, which amax_publish hands on, or of single rows of the loss.  Operands beyond it, with an infinity, or so large (2^61) that the two scales taken
-// out one after the other could overflow in between, are multiplied in three bf16 parts, which have fp32's exponents.
+// inputs or the weights, which amax_publish hands on, or of single rows of the loss.  Not seen are rows and columns of
+// gradients that are small in every tile, such as those of a unit that ELU saturates in every row (at z = -25 they are
+// 2^-36 of the others' and kept to 2^-14 of themselves): their sums matter to that unit alone, whose steps they leave as
+// they are (Adam divides by no less than its eps of 1e-8, which gradients clipped to a norm of 1 are far below there).
+// Operands beyond the spread, with an infinity, or so large (2^61) that the two scales taken out one after the other could
+// overflow in between, are multiplied in three bf16 parts, which have fp32's exponents.
 constexpr int kMaxSpread = 28, kMaxExponent = 127 + 60;
 struct Range {
   uint32_t top, low;

@@ -252,8 +252,8 @@ __device__ __forceinline__ float elu_fast(float x) {
 }
 
 // tanh: on |x| < 1 x + x^3 q(x^2) with q of degree 6 fitted as above (4.6e-9), beyond 1 - 2 / (2^(2 |x| log2 e) + 1) on
-// the hardware exp2 and reciprocal, whose
-// value is at most 0.24 off 1 there.  Measured against fp64: at most 1.31 ulp, 0.31 root mean square (tanhf 1.36 and 0.35).
+// the hardware exp2 and reciprocal, whose quotient is at most 0.24 there.  Measured against fp64: at most 1.31 ulp, 0.31
+// root mean square (tanhf 1.36 and 0.35).
 __device__ __forceinline__ float tanh_fast(float x) {
   const float x2 = x * x, ax = fabsf(x);
   float q = -0.00035845203092321754f;

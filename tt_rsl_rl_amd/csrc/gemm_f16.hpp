@@ -4,9 +4,10 @@
 // fp16x3.  Every operand element x is scaled by a power of two s (one per tensor: its largest |x| lands in
 // [2^14, 2^15)) and split into two fp16 parts, hi = fp16(s x) and lo = fp16(2^11 (s x - hi)), both rounded to nearest:
 // s x = hi + 2^-11 lo with a residual of at most 2^-23 |s x| (2^-24 on average), and of at most 2^-36 where lo is
-// subnormal, i.e. 2^-50 of the tensor's largest value (what that means for a tensor of wide range: amax.hpp).  A product is taken as hi.hi + 2^-11 (hi.lo + lo.hi): three
-// MFMAs, the hi.hi sums in one accumulator and the cross terms in another (added at the end, in fp32); the left-out
-// lo.lo is at most 2^-22 of the product and 2^-24 on average.  This is the published scheme of Ootomo and Yokota
+// subnormal, i.e. 2^-50 of the tensor's largest value (what that means for a tensor of wide range: amax.hpp).  A product
+// is taken as hi.hi + 2^-11 (hi.lo + lo.hi): three MFMAs, the hi.hi sums in one accumulator and the cross terms in another
+// (added at the end, in fp32); the left-out lo.lo is at most 2^-22 of the product and 2^-24 on average.  This is the
+// published scheme of Ootomo and Yokota
 // ("Recovering single precision accuracy from Tensor Cores while surpassing the FP32 theoretical peak performance",
 // IJHPCA 2022) with the scaling made explicit.  Against bf16x6 (gemm_core.hpp) it issues half the MFMAs, moves two
 // 16-bit planes through LDS instead of three and splits in 6 VALU instructions per pair of elements instead of 11; its

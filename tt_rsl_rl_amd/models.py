@@ -252,8 +252,8 @@ class _ForwardBuffers:
 
 
 # Up to this many rows a model's forward is one launch (ppo_mlp_fwd) where its weights are few enough (_Route), above it one
-# GEMM launch per layer: 256 blocks of 16 rows, one per compute unit.  48 -> [512, 256, 128] -> 12, one launch / layer by layer: 16 rows 33 / 64 us, 4,096 rows
-# 34 / 63, 8,192 rows 59 / 62, 16,384 rows 112 / 74.
+# GEMM launch per layer: 256 blocks of 16 rows, one per compute unit.  48 -> [512, 256, 128] -> 12, one launch / layer by
+# layer: 16 rows 33 / 64 us, 4,096 rows 34 / 63, 8,192 rows 59 / 62, 16,384 rows 112 / 74.
 FUSED_ROWS = 4096
 # Up to this many rows that forward is a launch per two layers, the second one's outputs spread over several blocks
 # (ppo_mlp_fwd_pairs), where those second layers (but the last) hold at least PAIR_WEIGHTS weights: fewer do not pay for

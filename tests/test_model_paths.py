@@ -217,16 +217,3 @@ def test_a_wide_network_of_few_rows_runs_layer_by_layer():
     obs = {"g": torch.randn(100, 20, device="cuda")}
     with torch.no_grad():
         assert torch.equal(m(obs), m.forward_layers(obs))
-
-
-@pytest.mark.gpu
-def test_an_observation_group_without_columns():
-    """A group of no columns beside others adds nothing to the input, on few rows (the one-launch forward) as on many."""
-    torch.manual_seed(0)
-    groups = {"g": torch.zeros(2, 20), "none": torch.zeros(2, 0)}
-    m = MLPModel(groups, {"critic": ["g", "none"]}, "critic", 4, hidden_dims=[32, 16], activation="elu").to("cuda")
-    x = torch.randn(5000, 20, device="cuda")
-    with torch.no_grad():
-        want = m({"g": x, "none": x[:, :0]})
-        got = m({"g": x[:50], "none": x[:50, :0]})
-    assert float((got - want[:50]).norm() / want[:50].norm()) < 1e-5

@@ -453,7 +453,7 @@ class MLPModel(nn.Module):
         rec = L.MlpProblem.from_buffer_copy(rec)  # (this call's own: its buffers go into it)
         width = 0
         for i, x in enumerate(columns):
-            if x.dtype != torch.float32 or x.shape[0] != rows or not x.is_cuda or x.shape[1] == 0:
+            if x.dtype != torch.float32 or x.shape[0] != rows or not x.is_cuda:
                 return None
             if x.stride(1) != 1 or (rows > 1 and x.stride(0) < x.shape[1]):
                 x = columns[i] = x.contiguous()

@@ -294,10 +294,11 @@ class _Route(NamedTuple):
 
     def choose(self, rows: int, pairs_fit: bool) -> str:
         """"one", "pairs" or "layers".  More blocks by pairs than the 256 compute units take run one after another."""
-        waves = -(-(-(-rows // 16) * self.slices) // 256)
-        by_pairs = self.pairs * max(1.0, 0.75 * waves)
-        if pairs_fit and rows <= PAIR_ROWS and (waves == 1 or by_pairs < self.one):
-            return "pairs" if by_pairs <= self.layers else "layers"
+        if pairs_fit and rows <= PAIR_ROWS:
+            waves = -(-(-(-rows // 16) * self.slices) // 256)
+            by_pairs = self.pairs * max(1.0, 0.75 * waves)
+            if waves == 1 or by_pairs < self.one:
+                return "pairs" if by_pairs <= self.layers else "layers"
         return "one" if self.one <= self.layers else "layers"
 
 
@@ -410,7 +411,8 @@ class MLPModel(nn.Module):
         layers = self._weights()
         tensors = [t for wb in layers for t in wb]
         if norm is not None:
-            tensors += [norm._mean, norm._std]
+            stats = norm._buffers  # (as _weights)
+            tensors += [stats["_mean"], stats["_std"]] if type(norm) is EmpiricalNormalization else [norm._mean, norm._std]
         if any(t is None for t in tensors):
             return (None, None, 0, None), tensors
         key = (self.act_code, None if norm is None else norm.eps,
@@ -453,13 +455,16 @@ class MLPModel(nn.Module):
         rec = L.MlpProblem.from_buffer_copy(rec)  # (this call's own: its buffers go into it)
         width = 0
         for i, x in enumerate(columns):
-            if x.dtype != torch.float32 or x.shape[0] != rows or not x.is_cuda:
+            n, w = x.shape
+            if x.dtype != torch.float32 or n != rows or not x.is_cuda:
                 return None
-            if x.stride(1) != 1 or (rows > 1 and x.stride(0) < x.shape[1]):
+            step, inner = x.stride()
+            if inner != 1 or (rows > 1 and step < w):
                 x = columns[i] = x.contiguous()
+                step = x.stride(0)
             b = rec.x[i]
-            b.src, b.stride, b.width = x.data_ptr(), max(x.stride(0), x.shape[1]), x.shape[1]
-            width += x.shape[1]
+            b.src, b.stride, b.width = x.data_ptr(), max(step, w), w
+            width += w
         if width != rec.layers[0].in_features:
             return None
         rec.num_blocks = len(columns)
@@ -475,7 +480,7 @@ class MLPModel(nn.Module):
         return out
 
     def mlp_forward(self, latent: torch.Tensor) -> torch.Tensor:
-        out = self._fused_forward([latent], None)
+        out = self._fused_forward([latent], None) if latent.dim() == 2 else None
         return self._mlp_layers(latent) if out is None else out
 
     def forward_layers(self, obs: Mapping) -> torch.Tensor:

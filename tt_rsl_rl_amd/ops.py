@@ -123,22 +123,27 @@ class RowStores:
         self.held: list[tuple] = []
 
     def copy(self, dst: torch.Tensor, src: torch.Tensor) -> None:
-        kind = L.STORE_F32 if dst.dtype == torch.float32 else L.STORE_U8 if dst.dtype == torch.uint8 else None
-        t = STORE_FLAGS.get(src.dtype, -1) if kind == L.STORE_U8 else L.STORE_T_F32
-        if (kind is None or t < 0 or (kind == L.STORE_F32 and src.dtype != torch.float32) or
-                type(src) is not torch.Tensor or type(dst) is not torch.Tensor or src.shape != dst.shape or
+        of, to, n = src.dtype, dst.dtype, dst.numel()
+        if to == torch.float32:
+            kind, t = L.STORE_F32, L.STORE_T_F32 if of == to else -1
+        else:
+            kind, t = L.STORE_U8, STORE_FLAGS.get(of, -1) if to == torch.uint8 else -1
+        if (t < 0 or type(src) is not torch.Tensor or type(dst) is not torch.Tensor or src.shape != dst.shape or
                 src.device != self.device or dst.device != self.device or src.requires_grad or dst.requires_grad or
-                dst.numel() >= 1 << 31):
+                not 0 < n < 1 << 31):
             dst.copy_(src)
             return
-        d, s = _rows_of(dst), _rows_of(src)
-        if d is None or s is None:
-            dst.copy_(src)
-            return
-        if d[0] != s[0]:  # one side without gaps: the other's rows
-            rows, width = max(d[:2], s[:2])
-            d = (rows, width, width) if d[0] == 1 else d
-            s = (rows, width, width) if s[0] == 1 else s
+        if dst.is_contiguous() and src.is_contiguous():
+            d = s = (1, n, n)
+        else:
+            d, s = _rows_of(dst), _rows_of(src)
+            if d is None or s is None:
+                dst.copy_(src)
+                return
+            if d[0] != s[0]:  # one side without gaps: the other's rows
+                rows, width = max(d[:2], s[:2])
+                d = (rows, width, width) if d[0] == 1 else d
+                s = (rows, width, width) if s[0] == 1 else s
         self._add(L.STORE_ITEM.pack(src.data_ptr(), s[2], dst.data_ptr(), d[2], d[0], d[1], kind, 0, 0, 0.0, t), dst, src)
 
     def bootstrap(self, dst: torch.Tensor, rewards: torch.Tensor, gamma: float, values: torch.Tensor,
